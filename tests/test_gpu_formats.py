@@ -93,3 +93,36 @@ def test_q3_repack_checkpoint_layout_bit_exact(rows, cols):
     np.testing.assert_array_equal(got, want)
     words = torch.from_numpy(src.view("<i4").copy()).to(DEV)
     np.testing.assert_array_equal(dsk_moe.q3_repack(words).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("rows,cols,shift", [(1, 128, 0), (3, 384, 1), (17, 2304, 3), (9, 4096, 2)])
+def test_q3_quantize_edges_bit_exact(rows, cols, shift):
+    """A part of a wave, a row that ends inside a wave, weights at 4-byte alignment;
+    groups of equal values, of zeros of both signs and with a NaN or an infinity."""
+    g = torch.Generator().manual_seed(rows)
+    w = torch.randn((rows * cols + shift,), generator=g) * 0.02
+    v = w[shift:].view(rows, cols)
+    v[0, :64] = 0.25
+    v[-1, 64:96], v[-1, 96:128] = 0.0, -0.0
+    if rows > 1:
+        v[1, 5], v[2, 70] = float("nan"), float("inf")
+    d = w.to(DEV)[shift:].view(rows, cols)
+    with np.errstate(all="ignore"):
+        got = [t.cpu().numpy() for t in dsk_moe.q3_quantize(d)]
+        clean = np.isfinite(v.numpy()).reshape(rows, -1, 64).all(-1)       # 64-groups the oracle defines
+        want = F.q3_quantize(np.where(np.isfinite(v.numpy()), v.numpy(), 0.0).astype(np.float32))
+    q_got, q_want = F.q3_unpack(got[0], cols), F.q3_unpack(want[0], cols)
+    codes = np.repeat(clean, 64, axis=1)
+    np.testing.assert_array_equal(q_got[codes], q_want[codes])
+    np.testing.assert_array_equal(got[1].view(np.uint16)[clean], want[1].view(np.uint16)[clean])
+    np.testing.assert_array_equal(got[2][clean], want[2][clean])           # a zero's sign does not count
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 32), (3, 96), (65, 2304), (129, 4096)])
+def test_fp4_dequant_f32_edges_exact(rows, cols):
+    """Fewer words than a block takes, and a last block that is partly filled."""
+    rng = np.random.default_rng(rows)
+    packed = rng.integers(0, 256, size=(rows, cols // 2), dtype=np.uint8)
+    scales = rng.integers(100, 150, size=(rows, cols // 32), dtype=np.uint8)
+    got = dsk_moe.fp4_dequant(torch.from_numpy(packed).to(DEV), torch.from_numpy(scales).to(DEV)).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), F.fp4_dequant(packed, scales).view(np.uint32))
