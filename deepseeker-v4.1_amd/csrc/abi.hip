@@ -87,9 +87,13 @@ Workspace workspace_layout(const dsk_moe_desc& d) {
   L.shared_x = take(mx && Is > 0 ? T * H * 2 : 0);
   // the grouped FP4 gate/up's x planes: every batch the grouped path may take (below the
   // prefill GEMM), bf16 x
-  if (prefill_mx(d)) {
+  if (prefill_mx_own_space(d)) {
     L.xp = take(T * (2 * H + H / 32));
     L.hp = take(N * (2 * I + I / 32));
+  } else if (prefill_mx(d)) {
+    // x's planes where the down later writes its rows, h's where the bf16 h would be
+    L.xp = L.y;
+    L.hp = L.h_hi;
   } else {
     // q3: x scaled for the factored gate/up [T][H] bf16, then its 64-group sums [T][H/64][2] f32
     const bool bf16x = d.x_dtype == DSK_DTYPE_BF16 && !prefill_gemm(d);
@@ -98,7 +102,16 @@ Workspace workspace_layout(const dsk_moe_desc& d) {
                                                : 0);
     L.hp = take(!prefill_gemm(d) && grouped_h_planes(d) ? N * 3 * (I + I / 32) : 0);
   }
-  L.pf_tiles = take(prefill_gemm(d) ? (3 + 2 * static_cast<size_t>(prefill_max_tiles(d))) * 4 : 0);
+  const size_t tile_bytes = prefill_gemm(d) ? (3 + 2 * static_cast<size_t>(prefill_max_tiles(d))) * 4 : 0;
+  if (prefill_mx(d) && !prefill_mx_own_space(d)) {
+    // the end of y, whose rows are bf16 here (its lower half); tiles of 256 rows set the size
+    L.pf_tiles = L.ys - align_up(tile_bytes);
+    dsk_moe_desc w = d;
+    w.quant = DSK_QUANT_Q3;   // counts 256-row tiles
+    take((3 + 2 * static_cast<size_t>(prefill_max_tiles(w))) * 4);
+  } else {
+    L.pf_tiles = take(tile_bytes);
+  }
   L.disp_hist = take(dispatch_hist_ints(static_cast<int>(N), static_cast<int>(E)) * 4);
   L.total = o;
   return L;

@@ -184,11 +184,20 @@ inline bool prefill_gemm(const dsk_moe_desc& d) {
          d.inter % 128 == 0 && d.inter_shared % 128 == 0;
 }
 int prefill_max_tiles(const dsk_moe_desc& d);
-// FP4 prefill GEMMs on the scaled FP4 x FP8 MFMAs (x and h as two FP8 planes;
-// K of both products a multiple of 512, the LDS DMA loop's).
+// FP4 prefill GEMMs on the scaled FP4 x FP8 MFMAs (x and h as two FP8 planes).
+// The LDS DMA loop takes any K that is a multiple of 128 from 512 (code pairs of
+// two stages, scale pieces of eight); x's planes are written a wave at a time,
+// so H stays a multiple of 512.  At H 5120, I 2304 and 2000 tokens on 384
+// experts the register-staged bf16 tiles that ran before took 1244 us for the
+// down (now 752 with the shared expert) and, the layer being bf16 altogether, 2514 us for the
+// gate/up (now 1562).
 inline bool prefill_mx(const dsk_moe_desc& d) {
-  return prefill_gemm(d) && d.quant == DSK_QUANT_FP4 && d.hidden % 512 == 0 && d.inter % 512 == 0;
+  return prefill_gemm(d) && d.quant == DSK_QUANT_FP4 && d.hidden % 512 == 0 && d.inter >= 512;
 }
+// Its planes and tile list have workspace of their own where I is a multiple of
+// 512; other I place them in regions that are free at the time, so that their
+// workspace is as large as it was without the planes (workspace_layout).
+inline bool prefill_mx_own_space(const dsk_moe_desc& d) { return prefill_mx(d) && d.inter % 512 == 0; }
 // The prefill GEMM's routed rows for the combine are rounded to bf16 when the
 // experts are FP4 (relative 2^-9 per row, inside the layer tolerance); q3
 // layers, whose dequantised weights are already rounded to bf16, and rows

@@ -30,8 +30,8 @@
 // x is bf16 (exact); h is rounded once to bf16 (relative 2^-9 per element),
 // where the decode and general kernels carry it as a bf16 hi/lo pair.
 //
-// FP4 experts with H and I multiples of 512 (and 16-byte aligned arrays) run
-// both products on the scaled FP4 x FP8 MFMA instead (the MX loop below):
+// FP4 experts with H a multiple of 512 and I one of 128 from 512 (and 16-byte
+// aligned arrays) run both products on the scaled FP4 x FP8 MFMA instead (the MX loop below):
 // x and h as two FP8 planes each, which hold their bf16 values exactly (see
 // the MX loop's note); on random data the part runs these at ~1.36x the
 // bf16 products' rate for the same work.  k_pf_planes writes x's planes
@@ -575,15 +575,20 @@ struct DmaMx {
 #pragma unroll
     for (int j = 0; j < 4; ++j) dma16(gc[j] + g * kPfK, c + (4 * wave + j) * 1024);
   }
-  __device__ __forceinline__ int scales(char* lds, int G, int wave) const {
-    dma16(gs + G * 16, lds + kS + (G & 1) * kSBuf + wave * 1024);
+  // first scale byte of group G's 16: eight stages from 8 G, or the row's last
+  // eight when fewer are left (the pieces of a row with K % 512 != 0 then start
+  // at 4-byte alignment, which the loads take)
+  __device__ __forceinline__ static int sbase(int G, int nst) { return min(16 * G, 2 * nst - 16); }
+  __device__ __forceinline__ int scales(char* lds, int G, int nst, int wave) const {
+    const int o = sbase(G, nst);
+    dma16(gs + o, lds + kS + (G & 1) * kSBuf + wave * 1024);
     if (wave >= 2) return 1;
-    dma16(ge + G * 16, lds + kE + (G & 1) * kEBuf + wave * 1024);
+    dma16(ge + o, lds + kE + (G & 1) * kEBuf + wave * 1024);
     return 2;
   }
   // loads before stage 0 (all waited for)
   __device__ __forceinline__ void prologue(char* lds, int nst, int wave) const {
-    scales(lds, 0, wave);
+    scales(lds, 0, nst, wave);
     codes(lds, 0, wave);
     tokens(lds, 0, wave);
   }
@@ -596,7 +601,7 @@ struct DmaMx {
       codes(lds, (st >> 1) + 1, wave);
       n += 4;
     }
-    if ((st & 7) == 0 && st + 8 < nst) n += scales(lds, (st >> 3) + 1, wave);
+    if ((st & 7) == 0 && st + 8 < nst) n += scales(lds, (st >> 3) + 1, nst, wave);
     return n;
   }
 };
@@ -622,14 +627,15 @@ __device__ __forceinline__ void pf_loop_mx(const DmaMx& src, int nst, int n_ct, 
   auto read = [&](MxOps& o, int st) {
     const char* c = lds + DmaMx::kC + DmaMx::cbuf(st) * DmaMx::kCBuf + (128 * wm + l) * 64 +
                     ((((st & 1) * 2 + g) ^ ((l >> 2) & 3)) * 16);
-    const char* sp = lds + DmaMx::kS + ((st >> 3) & 1) * DmaMx::kSBuf + (128 * wm + l) * 16 + (st & 7) * 2 + g;
+    const int so = 2 * st - DmaMx::sbase(st >> 3, nst);
+    const char* sp = lds + DmaMx::kS + ((st >> 3) & 1) * DmaMx::kSBuf + (128 * wm + l) * 16 + so + g;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       o.a[i] = *reinterpret_cast<const u32x4*>(c + i * 32 * 64);
       o.sa[i] = *reinterpret_cast<const uint8_t*>(sp + i * 32 * 16);
     }
     const char* B = lds + DmaMx::kB + DmaMx::tbuf(st) * DmaMx::kBBuf + brow;
-    const char* E = lds + DmaMx::kE + ((st >> 3) & 1) * DmaMx::kEBuf + erow + (st & 7) * 2;
+    const char* E = lds + DmaMx::kE + ((st >> 3) & 1) * DmaMx::kEBuf + erow + so;
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) {
 #pragma unroll

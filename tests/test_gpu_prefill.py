@@ -53,6 +53,17 @@ def test_prefill_layer(label, spec, T, zipf):
         assert int(r["counts"].max()) > 256          # an expert spans several token tiles
 
 
+@pytest.mark.parametrize("label,spec,T,zipf", [
+    ("I 640: a tail of two stages", L.LayerSpec(H=512, E=16, k=4, I=640, I_shared=128), 300, None),
+    ("I 768: a tail of four stages", L.LayerSpec(H=1024, E=32, k=2, I=768, I_shared=256), 700, 1.1),
+    ("I 1152, k 1", L.LayerSpec(H=1536, E=8, k=1, I=1152, I_shared=1152), 400, None),
+])
+def test_prefill_mx_intermediate_not_a_multiple_of_512(label, spec, T, zipf):
+    """The scaled-MFMA tiles with an intermediate whose last scale piece is shared by two
+    groups of stages, and its planes in regions of the workspace that are free then."""
+    _check(spec, synth.make_layer(spec, 24, T, zipf_s=zipf), T, label)
+
+
 def test_prefill_no_shared_and_callable():
     spec = L.LayerSpec(H=1024, E=64, k=8, I=512, I_shared=512)
     T = 260
