@@ -509,25 +509,26 @@ __device__ __forceinline__ f32x16 mx32(const u32x4& a, uint32_t sa, const u32x4&
                                                          static_cast<int>(sb));
 }
 
-// One stage's operands of a wave: 4 weight fragments with their scale bytes,
+// One stage's operands of a wave: AF weight fragments with their scale bytes,
 // 2 token fragments per plane with their scale bytes (plane 0's).
+template <int AF>
 struct MxOps {
-  u32x4 a[4];
-  uint32_t sa[4];
+  u32x4 a[AF];
+  uint32_t sa[AF];
   u32x4 b[2][2][2];   // [token fragment][plane][low / high 16 bytes]
   uint32_t sb[2];
 };
 
-// 8 products of one plane: acc[i][c] += A(i) x B(c, plane); unless kFull,
+// 2 AF products of one plane: acc[i][c] += A(i) x B(c, plane); unless kFull,
 // token fragments c >= n_ct (wave-uniform) are skipped.
-template <bool kFull>
-__device__ __forceinline__ void mx_mma(const MxOps& o, int pl, int n_ct, f32x16 (&acc)[4][2]) {
+template <bool kFull, int AF>
+__device__ __forceinline__ void mx_mma(const MxOps<AF>& o, int pl, int n_ct, f32x16 (&acc)[AF][2]) {
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     if (kFull || c < n_ct) {
       const uint32_t sb = o.sb[c] - 4u * static_cast<uint32_t>(pl);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i][c] = mx32(o.a[i], o.sa[i], o.b[c][pl][0], o.b[c][pl][1], sb, acc[i][c]);
+      for (int i = 0; i < AF; ++i) acc[i][c] = mx32(o.a[i], o.sa[i], o.b[c][pl][0], o.b[c][pl][1], sb, acc[i][c]);
     }
   }
 }
@@ -545,21 +546,31 @@ __device__ __forceinline__ void mx_mma(const MxOps& o, int pl, int n_ct, f32x16 
 // buffer G & 1).  Stage st + 1's tokens are loaded when stage st starts and
 // waited for at its end; code pair g + 1 when stage 2g starts (two stages
 // ahead); the scales of group G + 1 when stage 8G starts.
+//
+// A tile of at most 64 dispatch rows (the end of a slot's rows, or a slot of
+// few) runs as 64 columns: the four waves split the weight rows (64 each)
+// instead of leaving the two waves of columns 64..127 idle, and half the
+// token rows are loaded.  At H 5120 and 2000 tokens (31 rows a
+// slot): gate/up 1419 -> 1328 us, down 679 -> 632.
 constexpr int kMxThreads = 256;
 constexpr int kPfToksMx = 128;   // dispatch rows of an MX tile
 
+template <int TOK>
 struct DmaMx {
-  static constexpr int kB = 0, kBBuf = 16384;
+  static constexpr int kBL = TOK / 32;           // token loads per lane and stage
+  static constexpr int kWm = TOK == 128 ? 2 : 4; // waves over the weight rows
+  static constexpr int kAF = 8 / kWm;            // a wave's 32-row weight fragments
+  static constexpr int kB = 0, kBBuf = TOK * 128;
   static constexpr int kC = 2 * kBBuf, kCBuf = 16384;
   static constexpr int kS = kC + 2 * kCBuf, kSBuf = 4096;
-  static constexpr int kE = kS + 2 * kSBuf, kEBuf = 2048;
+  static constexpr int kE = kS + 2 * kSBuf, kEBuf = TOK * 16;
   static constexpr int kEnd = kE + 2 * kEBuf;
-  const uint8_t* gb[4];   // this lane's token chunk of stage 0, loads j = 0..3
+  const uint8_t* gb[kBL]; // this lane's token chunk of stage 0
   const uint8_t* gc[4];   // its code chunk of stage pair 0
   const uint8_t* gs;      // the scales of weight row 64 w + lane, stages 0..7
-  const uint8_t* ge;      // waves 0, 1: the exponents of token row 64 w + lane, stages 0..7
-  // load j of wave w, lane i writes LDS position (4 w + j) 64 + i (16 bytes each)
-  __device__ __forceinline__ static int brow(int w, int j, int i) { return ((4 * w + j) * 64 + i) >> 3; }
+  const uint8_t* ge;      // waves below TOK / 64: the exponents of token row 64 w + lane, stages 0..7
+  // load j of wave w, lane i writes LDS position (n w + j) 64 + i (16 bytes each; n loads per lane)
+  __device__ __forceinline__ static int brow(int w, int j, int i) { return ((kBL * w + j) * 64 + i) >> 3; }
   __device__ __forceinline__ static int bchunk(int w, int j, int i) { return swz(brow(w, j, i), i & 7); }
   __device__ __forceinline__ static int crow(int w, int j, int i) { return ((4 * w + j) * 64 + i) >> 2; }
   __device__ __forceinline__ static int cchunk(int w, int j, int i) { return (i & 3) ^ ((crow(w, j, i) >> 2) & 3); }
@@ -568,7 +579,7 @@ struct DmaMx {
   __device__ __forceinline__ void tokens(char* lds, int st, int wave) const {
     char* b = lds + kB + (st & 1) * kBBuf;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dma16(gb[j] + st * (kPfK * 2), b + (4 * wave + j) * 1024);
+    for (int j = 0; j < kBL; ++j) dma16(gb[j] + st * (kPfK * 2), b + (kBL * wave + j) * 1024);
   }
   __device__ __forceinline__ void codes(char* lds, int g, int wave) const {
     char* c = lds + kC + (g & 1) * kCBuf;
@@ -582,7 +593,7 @@ struct DmaMx {
   __device__ __forceinline__ int scales(char* lds, int G, int nst, int wave) const {
     const int o = sbase(G, nst);
     dma16(gs + o, lds + kS + (G & 1) * kSBuf + wave * 1024);
-    if (wave >= 2) return 1;
+    if (wave >= TOK / 64) return 1;
     dma16(ge + o, lds + kE + (G & 1) * kEBuf + wave * 1024);
     return 2;
   }
@@ -611,11 +622,14 @@ struct DmaMx {
 // stage's plane-1 products (operands kept in registers); this stage's plane-0
 // products; wait until stage st + 1 has landed, barrier.  Wave w (0..3)
 // multiplies weight rows 128 (w & 1) + [0, 128) by tokens 64 (w >> 1) +
-// [0, 64).
-template <bool kFull>
-__device__ __forceinline__ void pf_loop_mx(const DmaMx& src, int nst, int n_ct, char* lds, f32x16 (&acc)[4][2]) {
+// [0, 64), or, of a 64-column tile, rows 64 w + [0, 64) by all of it.
+template <bool kFull, int TOK>
+__device__ __forceinline__ void pf_loop_mx(const DmaMx<TOK>& src, int nst, int n_ct, char* lds,
+                                           f32x16 (&acc)[DmaMx<TOK>::kAF][2]) {
+  using D = DmaMx<TOK>;
+  constexpr int kAF = D::kAF;
   const int lane = threadIdx.x & 63, wave = wave_id();
-  const int wm = wave & 1, wn = wave >> 1, g = lane >> 5, l = lane & 31;
+  const int wm = wave % D::kWm, wn = wave / D::kWm, g = lane >> 5, l = lane & 31;
   // token rows 64 wn + 32 c + l share the swizzle of l
   int koff[2][2];
 #pragma unroll
@@ -624,18 +638,18 @@ __device__ __forceinline__ void pf_loop_mx(const DmaMx& src, int nst, int n_ct, 
     for (int hf = 0; hf < 2; ++hf) koff[pl][hf] = swz(l, 4 * pl + 2 * hf + g) * 16;
   const int brow = (64 * wn + l) * 128;
   const int erow = (64 * wn + l) * 16 + g;
-  auto read = [&](MxOps& o, int st) {
-    const char* c = lds + DmaMx::kC + DmaMx::cbuf(st) * DmaMx::kCBuf + (128 * wm + l) * 64 +
+  auto read = [&](MxOps<kAF>& o, int st) {
+    const char* c = lds + D::kC + D::cbuf(st) * D::kCBuf + (32 * kAF * wm + l) * 64 +
                     ((((st & 1) * 2 + g) ^ ((l >> 2) & 3)) * 16);
-    const int so = 2 * st - DmaMx::sbase(st >> 3, nst);
-    const char* sp = lds + DmaMx::kS + ((st >> 3) & 1) * DmaMx::kSBuf + (128 * wm + l) * 16 + so + g;
+    const int so = 2 * st - D::sbase(st >> 3, nst);
+    const char* sp = lds + D::kS + ((st >> 3) & 1) * D::kSBuf + (32 * kAF * wm + l) * 16 + so + g;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kAF; ++i) {
       o.a[i] = *reinterpret_cast<const u32x4*>(c + i * 32 * 64);
       o.sa[i] = *reinterpret_cast<const uint8_t*>(sp + i * 32 * 16);
     }
-    const char* B = lds + DmaMx::kB + DmaMx::tbuf(st) * DmaMx::kBBuf + brow;
-    const char* E = lds + DmaMx::kE + ((st >> 3) & 1) * DmaMx::kEBuf + erow + so;
+    const char* B = lds + D::kB + D::tbuf(st) * D::kBBuf + brow;
+    const char* E = lds + D::kE + ((st >> 3) & 1) * D::kEBuf + erow + so;
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) {
 #pragma unroll
@@ -648,7 +662,7 @@ __device__ __forceinline__ void pf_loop_mx(const DmaMx& src, int nst, int n_ct, 
   };
   src.prologue(lds, nst, wave);
   wait_barrier<0>();
-  MxOps cur, prev;
+  MxOps<kAF> cur, prev;
   for (int st = 0; st < nst; ++st) {
     const int n = src.issue_at(lds, st, nst, wave);
     read(cur, st);
@@ -660,7 +674,9 @@ __device__ __forceinline__ void pf_loop_mx(const DmaMx& src, int nst, int n_ct, 
   mx_mma<kFull>(prev, 1, n_ct, acc);
 }
 
-__device__ __forceinline__ void pf_gemm_mx(const DmaMx& src, int nst, int n_ct, char* lds, f32x16 (&acc)[4][2]) {
+template <int TOK>
+__device__ __forceinline__ void pf_gemm_mx(const DmaMx<TOK>& src, int nst, int n_ct, char* lds,
+                                           f32x16 (&acc)[DmaMx<TOK>::kAF][2]) {
   if (n_ct == 2) pf_loop_mx<true>(src, nst, n_ct, lds, acc);
   else pf_loop_mx<false>(src, nst, n_ct, lds, acc);
 }
@@ -669,7 +685,8 @@ static_assert(DmaBf16::kEnd <= DmaFp4::kEnd && 2 * (Bf16Tile::kBytes + kPfBBytes
               "every loop's stages fit the FP4 DMA loop's LDS");
 
 constexpr size_t kPfLdsBytes = DmaFp4::kEnd;
-constexpr size_t kMxLdsBytes = DmaMx::kEnd;
+constexpr size_t kMxLdsBytes = DmaMx<kPfToksMx>::kEnd;
+static_assert(DmaMx<64>::kEnd <= DmaMx<kPfToksMx>::kEnd, "the narrow tile fits the wide one's LDS");
 static_assert(2 * kMxLdsBytes <= kMaxLds, "two MX workgroups share a CU's LDS");
 static_assert(kPfLdsBytes <= kMaxLds, "LDS stage buffers do not fit");
 
@@ -742,9 +759,10 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return static_cast<uint32_t>(f32_to_bf16_bits(a)) | (static_cast<uint32_t>(f32_to_bf16_bits(b)) << 16);
 }
 
-__device__ __forceinline__ void zero(f32x16 (&acc)[4][2]) {
+template <int AF>
+__device__ __forceinline__ void zero(f32x16 (&acc)[AF][2]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < AF; ++i)
 #pragma unroll
     for (int c = 0; c < 2; ++c) acc[i][c] = f32x16{};
 }
@@ -962,42 +980,42 @@ __global__ __launch_bounds__(kPfThreads, 1) void k_pf_down(PfArgs p) {
   }
 }
 
-// MX gate/up: a routed tile of 128 dispatch rows; local weight row r =
-// 0..255 of the unit is w1 (r & 64 == 0) or w3 row rt*128 + (r >> 7)*64 +
-// (r & 63), so wave rows 0..63 are gate rows and 64..127 the matching up
-// rows.  h is rounded to bf16, then written as two FP8 planes in stage rows:
-// features f0 + [0, 32) of fragment i (f0 = rt 128 + wm 64 + 32 i) are one
-// 32-group; this lane holds 16 of them, at 8 (r >> 2) + 4 g + (r & 3), lane
-// l ^ 32 (same token) the other 16.
-__global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_up(PfArgs p) {
-  extern __shared__ __align__(16) char mx_lds[];
-  int tile, rt;
-  if (!*p.mx_on || !pf_unit_in(p, 0, p.tiles[1], tile, rt)) return;
-  const int slot = p.tiles[2 + tile], first = p.tiles[2 + p.max_tiles + tile];
-  const SlotDesc* d = p.desc + slot;
+// MX gate/up: a routed tile of 128 (or 64) dispatch rows; of every 2 G local
+// weight rows of the unit (G = 64, of a 64-column tile 32) the first G are w1
+// rows and the others the w3 rows of the same features, so that a wave's first
+// fragments are gate rows and the others the matching up rows: row r is
+// feature rt*128 + (r / 2G) G + r % G.  h is rounded to bf16, then written as
+// two FP8 planes in stage rows: the 32 features of a fragment are one 32-group;
+// this lane holds 16 of them, at 8 (r >> 2) + 4 g + (r & 3), lane l ^ 32 (same
+// token) the other 16.
+template <int TOK>
+__device__ __forceinline__ void mx_up_tile(const PfArgs& p, const SlotDesc* d, int first, int cnt, int rt, char* lds) {
+  using D = DmaMx<TOK>;
+  constexpr int kG = 16 * D::kAF;   // gate rows of a wave
   const int tok_base = d->tok_base;
-  const int cnt = min(kPfToksMx, d->n_tok - first);
   const int lane = threadIdx.x & 63, wave = wave_id();
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % D::kWm, wn = wave / D::kWm;
   const int n_ct = max(0, min(2, (cnt - 64 * wn + 31) >> 5));
   const int K = p.H;
-  auto role_of = [](int r) { return (r >> 6) & 1; };
-  auto arow_of = [&](int r) { return static_cast<int64_t>(rt * 128 + (r >> 7) * 64 + (r & 63)); };
+  auto role_of = [](int r) { return (r / kG) & 1; };
+  auto arow_of = [&](int r) { return static_cast<int64_t>(rt * 128 + r / (2 * kG) * kG + r % kG); };
   auto xrow_of = [&](int r) { return static_cast<int64_t>(p.xrow[tok_base + first + min(r, cnt - 1)]); };
-  DmaMx src;
+  D src;
+#pragma unroll
+  for (int j = 0; j < D::kBL; ++j)
+    src.gb[j] = p.xq + xrow_of(D::brow(wave, j, lane)) * (2 * K) + D::bchunk(wave, j, lane) * 16;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    src.gb[j] = p.xq + xrow_of(DmaMx::brow(wave, j, lane)) * (2 * K) + DmaMx::bchunk(wave, j, lane) * 16;
-    const int r = DmaMx::crow(wave, j, lane);
+    const int r = D::crow(wave, j, lane);
     src.gc[j] = static_cast<const uint8_t*>(d->p[3 * role_of(r)]) + arow_of(r) * (K / 2) +
-                DmaMx::cchunk(wave, j, lane) * 16;
+                D::cchunk(wave, j, lane) * 16;
   }
   const int rs = 64 * wave + lane;
   src.gs = static_cast<const uint8_t*>(d->p[3 * role_of(rs) + 1]) + arow_of(rs) * (K / 32);
-  src.ge = p.xe + xrow_of(rs & 127) * (K / 32);
-  f32x16 acc[4][2];
+  src.ge = p.xe + xrow_of(rs % TOK) * (K / 32);
+  f32x16 acc[D::kAF][2];
   zero(acc);
-  pf_gemm_mx(src, K / kPfK, n_ct, mx_lds, acc);
+  pf_gemm_mx(src, K / kPfK, n_ct, lds, acc);
   const int g = lane >> 5;
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
@@ -1005,14 +1023,15 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_up(PfArgs p) {
     if (n >= cnt) continue;
     const int64_t drow = tok_base + first + n;
     const float wr = p.wrow[drow];
-    uint8_t* hrow = p.hq + drow * (2 * p.I) + (2 * rt + wm) * 128;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < D::kAF / 2; ++i) {
+      const int f0 = rt * 128 + wm * kG + 32 * i;   // the fragment's first feature
+      uint8_t* hrow = p.hq + drow * (2 * p.I) + (f0 >> 6) * 128 + (f0 & 63);
       float hv[16];
       float m = 0.0f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float v = silu_clamped(acc[i][c][r], acc[i + 2][c][r], p.limit) * wr;
+        const float v = silu_clamped(acc[i][c][r], acc[i + D::kAF / 2][c][r], p.limit) * wr;
         hv[r] = __uint_as_float(static_cast<uint32_t>(f32_to_bf16_bits(v)) << 16);
         m = fmaxf(m, fabsf(hv[r]));
       }
@@ -1024,53 +1043,61 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_up(PfArgs p) {
         uint32_t w[2];
         fp8_planes4<2>(v4, e, w);
 #pragma unroll
-        for (int pl = 0; pl < 2; ++pl)
-          *reinterpret_cast<uint32_t*>(hrow + 64 * pl + 32 * i + 8 * q + 4 * g) = w[pl];
+        for (int pl = 0; pl < 2; ++pl) *reinterpret_cast<uint32_t*>(hrow + 64 * pl + 8 * q + 4 * g) = w[pl];
       }
-      if (g == 0) p.he[drow * (p.I / 32) + 4 * rt + 2 * wm + i] = static_cast<uint8_t>(e8m0_byte(e));
+      if (g == 0) p.he[drow * (p.I / 32) + (f0 >> 5)] = static_cast<uint8_t>(e8m0_byte(e));
     }
   }
 }
 
-// MX down: w2 rows rt*256 + [0, 256) by a routed tile of 128 dispatch rows,
-// from h's planes; routed rows in float32 or bf16 (y_bf16).
-__global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_down(PfArgs p) {
+__global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_up(PfArgs p) {
   extern __shared__ __align__(16) char mx_lds[];
   int tile, rt;
   if (!*p.mx_on || !pf_unit_in(p, 0, p.tiles[1], tile, rt)) return;
   const int slot = p.tiles[2 + tile], first = p.tiles[2 + p.max_tiles + tile];
   const SlotDesc* d = p.desc + slot;
-  const int tok_base = d->tok_base;
   const int cnt = min(kPfToksMx, d->n_tok - first);
+  if (cnt <= 64) mx_up_tile<64>(p, d, first, cnt, rt, mx_lds);
+  else mx_up_tile<kPfToksMx>(p, d, first, cnt, rt, mx_lds);
+}
+
+// MX down: w2 rows rt*256 + [0, 256) by a routed tile of 128 (or 64) dispatch
+// rows, from h's planes; routed rows in float32 or bf16 (y_bf16).
+template <int TOK>
+__device__ __forceinline__ void mx_down_tile(const PfArgs& p, const SlotDesc* d, int first, int cnt, int rt,
+                                             char* lds) {
+  using D = DmaMx<TOK>;
+  const int tok_base = d->tok_base;
   const int lane = threadIdx.x & 63, wave = wave_id();
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % D::kWm, wn = wave / D::kWm;
   const int n_ct = max(0, min(2, (cnt - 64 * wn + 31) >> 5));
   const int K = p.I;
   const int64_t row0 = static_cast<int64_t>(rt) * 256;
   auto hrow_of = [&](int r) { return static_cast<int64_t>(tok_base + first + min(r, cnt - 1)); };
-  DmaMx src;
+  D src;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    src.gb[j] = p.hq + hrow_of(DmaMx::brow(wave, j, lane)) * (2 * K) + DmaMx::bchunk(wave, j, lane) * 16;
-    src.gc[j] = static_cast<const uint8_t*>(d->p[6]) + (row0 + DmaMx::crow(wave, j, lane)) * (K / 2) +
-                DmaMx::cchunk(wave, j, lane) * 16;
-  }
+  for (int j = 0; j < D::kBL; ++j)
+    src.gb[j] = p.hq + hrow_of(D::brow(wave, j, lane)) * (2 * K) + D::bchunk(wave, j, lane) * 16;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    src.gc[j] = static_cast<const uint8_t*>(d->p[6]) + (row0 + D::crow(wave, j, lane)) * (K / 2) +
+                D::cchunk(wave, j, lane) * 16;
   const int rs = 64 * wave + lane;
   src.gs = static_cast<const uint8_t*>(d->p[7]) + (row0 + rs) * (K / 32);
-  src.ge = p.he + hrow_of(rs & 127) * (K / 32);
-  f32x16 acc[4][2];
+  src.ge = p.he + hrow_of(rs % TOK) * (K / 32);
+  f32x16 acc[D::kAF][2];
   zero(acc);
-  pf_gemm_mx(src, K / kPfK, n_ct, mx_lds, acc);
+  pf_gemm_mx(src, K / kPfK, n_ct, lds, acc);
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     const int n = 64 * wn + 32 * c + (lane & 31);
     if (n >= cnt) continue;
     const int64_t drow = tok_base + first + n;
-    const int64_t col0 = drow * p.H + row0 + wm * 128 + 4 * (lane >> 5);
+    const int64_t col0 = drow * p.H + row0 + wm * (32 * D::kAF) + 4 * (lane >> 5);
     if (p.y_bf16) {
       uint16_t* out = reinterpret_cast<uint16_t*>(p.y);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < D::kAF; ++i)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           *reinterpret_cast<uint2*>(out + col0 + 32 * i + 8 * q) =
@@ -1078,13 +1105,24 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_down(PfArgs p) {
                     pack_bf16x2(acc[i][c][4 * q + 2], acc[i][c][4 * q + 3])};
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < D::kAF; ++i)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           *reinterpret_cast<f32x4*>(p.y + col0 + 32 * i + 8 * q) =
               f32x4{acc[i][c][4 * q], acc[i][c][4 * q + 1], acc[i][c][4 * q + 2], acc[i][c][4 * q + 3]};
     }
   }
+}
+
+__global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_down(PfArgs p) {
+  extern __shared__ __align__(16) char mx_lds[];
+  int tile, rt;
+  if (!*p.mx_on || !pf_unit_in(p, 0, p.tiles[1], tile, rt)) return;
+  const int slot = p.tiles[2 + tile], first = p.tiles[2 + p.max_tiles + tile];
+  const SlotDesc* d = p.desc + slot;
+  const int cnt = min(kPfToksMx, d->n_tok - first);
+  if (cnt <= 64) mx_down_tile<64>(p, d, first, cnt, rt, mx_lds);
+  else mx_down_tile<kPfToksMx>(p, d, first, cnt, rt, mx_lds);
 }
 
 // x [T][H] bf16 as two FP8 planes in stage rows (the MX gate/up's B tiles),
