@@ -100,7 +100,11 @@ Workspace workspace_layout(const dsk_moe_desc& d) {
     L.xp = take(bf16x && d.quant == DSK_QUANT_FP4 ? T * 2 * (H + H / 32)
                 : bf16x && grouped_x_q3(d)     ? T * (2 * H + H / 8)
                                                : 0);
-    L.hp = take(!prefill_gemm(d) && grouped_h_planes(d) ? N * 3 * (I + I / 32) : 0);
+    // the wide kernels' h planes: up to 512 rows of the sizes below in space of their own,
+    // else where the bf16 h pair would be (so that workspaces keep their sizes)
+    const bool own = bf16x && d.quant == DSK_QUANT_FP4 && H % 1024 == 0 && H <= 4096 &&
+                     (I == 512 || I == 1024 || I == 2048) && N <= 512;
+    L.hp = own ? take(N * 3 * (I + I / 32)) : L.h_hi;
   }
   const size_t tile_bytes = prefill_gemm(d) ? (3 + 2 * static_cast<size_t>(prefill_max_tiles(d))) * 4 : 0;
   if (prefill_mx(d) && !prefill_mx_own_space(d)) {
@@ -381,10 +385,10 @@ int dsk::forward_layer(const dsk_moe_desc* d, const void* x, const void* gate_w,
   // the unfused top-k kernel writes x in the form the gate/up that follows reads (FP8
   // planes for FP4 experts, the factored q3 form for q3 experts; prefill: its MX planes)
   if (!decode && d->tokens > kFusedMaxTokens && !rn && d->x_dtype == DSK_DTYPE_BF16) {
-    const bool pf = prefill_mx(*d);
-    if (pf || (!prefill_gemm(*d) && grouped_path(*d) && (grouped_up_mx(*d) || grouped_x_q3(*d)))) {
+    const bool planes = prefill_mx(*d) || grouped_wide(*d);
+    if (planes || (!prefill_gemm(*d) && grouped_path(*d) && grouped_x_q3(*d))) {
       ra.xp = reinterpret_cast<uint8_t*>(ws + L.xp);
-      ra.xform = pf ? kXPrefillPlanes : d->quant == DSK_QUANT_Q3 ? kXGroupedQ3 : kXGroupedPlanes;
+      ra.xform = planes ? kXPlanes : kXGroupedQ3;
       a.x_planes_ready = 1;
     }
   }

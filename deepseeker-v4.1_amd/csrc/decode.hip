@@ -488,7 +488,8 @@ __global__ __launch_bounds__(kRsW * 64) __attribute__((amdgpu_waves_per_eu(4))) 
       // 16 lanes iterate together: every group of four chunks is exchanged whole)
       const int n = p.T * (p.H / 8), stride = (static_cast<int>(gridDim.x) - 1) * 16;
       for (int c = rt * 16 + tid; c - tid < n; c += stride)
-        x_planes_chunk(static_cast<const uint16_t*>(p.x), p.T, p.H, min(c, n - 1), c < n, p.xp);
+        pf_planes_chunk(static_cast<const uint16_t*>(p.x), p.H, min(c, n - 1), c < n, p.xp,
+                        p.xp + static_cast<size_t>(p.T) * 2 * p.H);
     }
   }
 }
@@ -1807,12 +1808,11 @@ __global__ __launch_bounds__(kDownW * 64) void k_down_decode(DecodeArgs p) {
 }
 
 // The routing kernel of the decode pipeline's non-MX form (k_route_shared) also
-// writes x's FP8 planes for the grouped FP4 gate/up that follows it (saves
+// writes x's FP8 planes for the wide FP4 gate/up that follows it (saves
 // that kernel's own launch): from kDecodeGroupedUpMin tokens, with shared tile
 // blocks to do it.
 bool route_writes_x_planes(const dsk_moe_desc& d) {
-  return d.tokens >= kDecodeGroupedUpMin && d.x_dtype == DSK_DTYPE_BF16 && d.inter_shared > 0 &&
-         grouped_path(d) && grouped_up_mx(d);
+  return d.tokens >= kDecodeGroupedUpMin && d.inter_shared > 0 && grouped_wide(d);
 }
 
 DecodeArgs decode_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a) {
@@ -1986,7 +1986,7 @@ hipError_t launch_experts_decode(const dsk_moe_desc& d, const Workspace& L, cons
   if (d.tokens >= kDecodeGroupedDownMin && grouped_path(d)) {
     // routed and shared down per slot (one output row per dispatch row), then the combine
     // h in FP8 planes where the grouped gate/up wrote it (from kDecodeGroupedUpMin tokens)
-    const bool hpl = d.tokens >= kDecodeGroupedUpMin && grouped_h_planes(d);
+    const bool hpl = d.tokens >= kDecodeGroupedUpMin && grouped_wide(d);
     if ((e = launch_grouped_down(d, L, a, a.route.desc, s, repeat, hpl)) != hipSuccess) return e;
     return launch_combine(d, L, a, s, repeat);
   }

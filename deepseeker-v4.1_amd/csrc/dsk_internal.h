@@ -145,12 +145,12 @@ struct Workspace {
   size_t y;                 // routed outputs          [T*k][H] f32
   size_t ys;                // shared output           [T][H]   f32
   size_t shared_x;          // decode pipeline: shared output [T][H] (x dtype)
-  size_t xp;                // grouped FP4 gate/up: x as FP8 planes [T][2][H] + E8M0 [T][2][H/32];
-                            // MX prefill: x as FP8 planes in stage rows [T][2H] + E8M0 [T][H/32]
+  size_t xp;                // wide and MX prefill gate/up: x as FP8 planes in stage rows [T][2H] +
+                            // E8M0 [T][H/32]
                             // grouped q3: x scaled for the factored gate/up [T][H] bf16 + 64-group
                             // sums [T][H/64][2] f32
-  size_t hp;                // grouped FP4: h as FP8 planes [T*k][3][I] + E8M0 [T*k][3][I/32];
-                            // MX prefill: h in stage rows [T*k][2I] + E8M0 [T*k][I/32]
+  size_t hp;                // h as FP8 planes in stage rows: wide below the prefill sizes [T*k][3I],
+                            // MX prefill [T*k][2I]; + E8M0 [T*k][I/32]
   size_t pf_tiles;          // prefill GEMM tile list  [2 + 2 * prefill_max_tiles] + the MX switch
   size_t total;
 };
@@ -240,9 +240,9 @@ hipError_t launch_route(const dsk_moe_desc& d, const void* x, const void* gate_w
 struct ResNorm;   // resnorm.h: the stack's residual update + RMSNorm, fused into a layer's first kernel
 
 // x as the gate/up after an unfused top-k reads it (written by the top-k's
-// trailing blocks): the grouped FP4 gate/up's FP8 planes, the grouped q3
-// gate/up's factored form, the prefill MX gate/up's FP8 planes.
-enum XForm : int { kXGroupedPlanes = 0, kXGroupedQ3 = 1, kXPrefillPlanes = 2 };
+// trailing blocks): the grouped q3 gate/up's factored form, or the FP8 planes
+// of the wide and prefill MX gate/ups.
+enum XForm : int { kXGroupedQ3 = 0, kXPlanes = 1 };
 
 struct RouteArgs {
   const void* x; const void* gate_w; const float* gate_b;
@@ -337,6 +337,7 @@ struct PrefillArgs {
   char* ws;
   float* rows_out;           // per-row outputs instead of the workspace's (or null)
   int x_planes_ready;        // the routing kernels already wrote x's FP8 planes
+  const ExpertsArgs* call;   // the call's arguments (the wide kernels')
 };
 hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, const PrefillArgs& a,
                                   hipStream_t s, int repeat);
@@ -353,20 +354,38 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
 // Its kernels one at a time, for the decode pipeline: the routed gate/up
 // alone (from kDecodeGroupedUpMin tokens) and the down (routed rows from h,
 // shared from hs; from kDecodeGroupedDownMin tokens).
-// x_planes_ready: the routing kernel already wrote x's FP8 planes (grouped_up_mx).
+// x_planes_ready: the routing kernel already wrote x's FP8 planes (grouped_wide).
 hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                     const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                     int repeat, bool x_planes_ready);
-// The grouped FP4 gate/up takes x as FP8 planes (Workspace::xp).
-bool grouped_up_mx(const dsk_moe_desc& d);
+// Wide FP4 kernels (grouped.hip): a slot's dispatch rows in tiles of up to 64
+// over the whole of K, x and h as FP8 planes in stage rows.
+struct WideCall {
+  int h_planes;              // 3, or 2 of h rounded to bf16 (the prefill GEMM's form, in Workspace::hp)
+  int max_rows;              // slots with more dispatch rows are another kernel's
+  const int32_t* on;         // device switch of the slots' blocks, or null
+  int y_bf16;                // routed rows as bf16
+  bool shared;               // also the shared expert (hs hi / lo planes, float32 ys)
+};
+bool wide_shapes(const dsk_moe_desc& d);
+hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
+                          const int32_t* xrow, const float* wrow, const WideCall& w, hipStream_t s);
+hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
+                            const WideCall& w, hipStream_t s);
+// x [T][H] as FP8 planes in stage rows into Workspace::xp.
+hipError_t launch_pf_planes(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s);
+// The grouped path runs its FP4 slots on the wide kernels.
+bool grouped_wide(const dsk_moe_desc& d);
+// Prefill layers: slots of up to this many dispatch rows run on the wide
+// kernels instead of the GEMM tiles (0: none), and whether the shared expert does.
+int prefill_narrow_rows(const dsk_moe_desc& d);
+bool prefill_shared_wide(const dsk_moe_desc& d);
 // The grouped q3 gate/up takes x scaled for the factored product, with its
 // 64-group sums (Workspace::xp).
 bool grouped_x_q3(const dsk_moe_desc& d);
-// h_planes: the routed h is in FP8 planes (the grouped gate/up ran and grouped_h_planes).
+// h_planes: the routed h is in FP8 planes (the wide gate/up wrote it).
 hipError_t launch_grouped_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                const SlotDesc* desc, hipStream_t s, int repeat, bool h_planes);
-// The grouped FP4 gate/up writes h as FP8 planes and the down reads them on scaled MFMAs.
-bool grouped_h_planes(const dsk_moe_desc& d);
 // out[t] = cast(sum of the token's routed rows y in ascending expert id +
 // shared); the combine stage.
 hipError_t launch_combine(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s,

@@ -588,7 +588,7 @@ hipError_t launch_combine(const dsk_moe_desc& d, const Workspace& L, const Exper
   int mode = Is > 0 ? kSharedF32 : (a.shared_out ? kSharedExt : kNoShared);
   const void* shared_ext = a.shared_out;
   const bool pf = prefill_gemm(d);
-  if (pf && Is > 0) {            // the prefill GEMM wrote the shared output already rounded to bf16
+  if (pf && Is > 0 && !prefill_shared_wide(d)) {   // the prefill GEMM wrote the shared output already rounded to bf16
     mode = kSharedExt;
     shared_ext = ys;
   }
@@ -636,7 +636,8 @@ hipError_t launch_experts(const dsk_moe_desc& d, const Workspace& L, const Exper
   const uint16_t* xb_hi = static_cast<const uint16_t*>(a.x);
   const uint16_t* xb_lo = nullptr;
   if (prefill_gemm(d)) {
-    PrefillArgs pa{desc, a.active, xrow, wrow, a.x, a.ws1, a.ws3, a.ws2, a.ws, a.rows_out, a.x_planes_ready};
+    PrefillArgs pa{desc, a.active, xrow, wrow, a.x, a.ws1, a.ws3, a.ws2, a.ws, a.rows_out, a.x_planes_ready,
+                   &a};
     if ((e = launch_experts_prefill(d, L, pa, s, repeat)) != hipSuccess) return e;
     return a.rows_out ? hipSuccess : launch_combine(d, L, a, s, repeat);
   }

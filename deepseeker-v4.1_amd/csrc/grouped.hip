@@ -48,10 +48,14 @@ struct GroupedArgs {
   int dn_groups, dn_shared;                      // down: the same
   int q3f;                                       // q3 gate/up in the factored form (up_block_q3f)
   int q3fd;                                      // q3 down in the factored form (down_block_q3f)
-  int mx;                                        // FP4 gate/up on scaled MFMAs: blocks per wave, or 0
-  uint8_t* xp;                                   // mx: x as FP8 planes [T][2][H], then E8M0 [T][2][H/32]
-  int hplanes;                                   // FP4 slots' h as FP8 planes, the down on scaled MFMAs
-  uint8_t* hp;                                   // hplanes: [T*k][3][I], then E8M0 [T*k][3][I/32]
+  uint8_t* xp;                                   // q3f: x scaled, [T][H] bf16, then its 64-group sums
+  // wide kernels: x (in xp) and h as FP8 planes in stage rows
+  uint8_t* hp;                                   // [T*k][planes I]
+  const uint8_t* xe; uint8_t* he;                // their E8M0 bytes [T][H/32], [T*k][I/32]
+  int max_rows;                                  // slots with more rows are another kernel's
+  const int32_t* on;                             // device switch of the FP4 slots' blocks, or null (on)
+  int y_bf16;                                    // routed rows rounded to bf16
+  int sh_tg;                                     // shared expert: groups of kGsCols tokens in blocks of their own
 };
 
 // K blocks per weight batch, two batches in flight per wave, within the
@@ -353,28 +357,6 @@ __device__ __forceinline__ void up_block_q3f(const GroupedArgs& p, const void* c
   }
 }
 
-// ---------------------------------------------------------------- MX gate/up (FP4 slots)
-// The FP4 slots' gate/up on v_mfma_scale_f32_16x16x128_f8f6f4 (mx.h): the
-// codes and E8M0 bytes go into the product as loaded, so a wave holds its
-// whole K range of both roles in flight (kGxMaxBlocks 128-code blocks: 16
-// bytes of codes and a 4-byte scale word per block, role and lane) for each
-// column tile.  The activations are two FP8 planes per token,
-// written once per call by k_x_planes in the B-operand layout; a column tile
-// copies its rows' planes into LDS (column 2r + p: plane p of the tile's row
-// r).  K ranges are added in wave order, then a row's two plane columns; h
-// leaves as the bf16 hi / lo pair of the other gate/up paths.
-constexpr int kGxMaxBlocks = 8;     // K blocks per wave held (H <= kGKS * 8 * 128)
-
-// x's two FP8 planes (v ~ q0 2^e + q1 2^(e-4) per 32-value group, e =
-// ilogb(group max) - 7, mx.h) into xp (x_planes_chunk's layout), one thread
-// per 8 values.
-__global__ __launch_bounds__(256) void k_x_planes(const uint16_t* __restrict__ x, int T, int H,
-                                                  uint8_t* __restrict__ xp) {
-  const int n = T * (H / 8);
-  const int c0 = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
-  x_planes_chunk(x, T, H, min(c0, n - 1), c0 < n, xp);   // every lane takes part in the group exchange
-}
-
 // x for the factored q3 gate/up (up_block_q3f), once per call instead of once
 // per block (x_q3_chunk); the blocks copy the rows and sums of their column tile.
 __global__ __launch_bounds__(256) void k_x_q3(const uint16_t* __restrict__ x, int T, int H,
@@ -382,165 +364,6 @@ __global__ __launch_bounds__(256) void k_x_q3(const uint16_t* __restrict__ x, in
   const int n = T * (H / 8);
   const int c = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
   x_q3_chunk(x, H, min(c, n - 1), c < n, xq, xg);   // every lane takes part in the group's sums
-}
-
-// LDS of up_block_mx: the column tile's planes [H/128][16][128] bytes, then
-// their E8M0 words [H/128][16] (4 bytes: the block's four groups); the K-range
-// partial sums [kGI][kGKS][2][64][4] f32 reuse the planes after the products.
-__host__ __device__ inline size_t gx_lds_bytes(int H) { return static_cast<size_t>(H / 128) * 16 * (128 + 4); }
-
-// Gate/up of one FP4 slot block: row tile rt of w1 / w3 for the n dispatch
-// rows base .. base + n - 1.  Every wave's range is PER = H / 128 / kGKS
-// blocks (the launcher's condition), so the weight loads are uniform role
-// pointers + one 32-bit lane offset + an immediate per block.
-template <int PER>
-__device__ __forceinline__ void up_block_mx(const GroupedArgs& p, const void* const* wp, int rt, bool rok, int n,
-                                            int base, uint8_t* lds) {
-  static_assert(PER <= kGxMaxBlocks, "blocks held per wave");
-  const int tid = threadIdx.x, lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r16 = lane & 15, g4 = lane >> 4;
-  const int item = wave / kGKS, ks = wave % kGKS;
-  const int K = p.H, nblk = K / 128;
-  const int k0 = ks * PER;
-  uint8_t* xq = lds;
-  uint32_t* xe = reinterpret_cast<uint32_t*>(lds + static_cast<size_t>(nblk) * 16 * 128);
-  float (*red)[kGKS][2][64][4] = reinterpret_cast<float (*)[kGKS][2][64][4]>(lds);
-  // the wave's range within each role (uniform), this lane's row within it (32 bits: one role < 4 GB)
-  const uint8_t* W1 = static_cast<const uint8_t*>(wp[0]) + k0 * 64;
-  const uint8_t* S1 = static_cast<const uint8_t*>(wp[1]) + k0 * 4;
-  const uint8_t* W3 = static_cast<const uint8_t*>(wp[3]) + k0 * 64;
-  const uint8_t* S3 = static_cast<const uint8_t*>(wp[4]) + k0 * 4;
-  const uint32_t row = rok ? static_cast<uint32_t>(rt * 16 + r16) : 0u;
-  const uint32_t cb = row * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
-  const uint32_t sb = row * static_cast<uint32_t>(K / 32);
-  const uint8_t* xs = p.xp + static_cast<size_t>(p.T) * 2 * K;   // the planes' E8M0 bytes
-  // the h planes' 16-row maxima [kGI][16] f32, past the partial sums
-  float* gmx = reinterpret_cast<float*>(lds + static_cast<size_t>(kGI) * kGKS * 2 * 64 * 4 * sizeof(float));
-  // the wave's whole K range of both roles first (every product waits for it
-  // anyway), held across the slot's column tiles; then per tile its plane rows
-  // (16-byte chunks) and their exponents
-  u32x4 c1[PER], c3[PER];
-  uint32_t s1[PER], s3[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    c1[i] = ldg16(W1 + cb + i * 64);
-    c3[i] = ldg16(W3 + cb + i * 64);
-    s1[i] = ldg<uint32_t>(S1 + sb + i * 4);
-    s3[i] = ldg<uint32_t>(S3 + sb + i * 4);
-  }
-  for (int c0 = 0; c0 < n; c0 += kGNC) {
-    const int cols = min(kGNC, n - c0);
-    asm volatile("" ::: "memory");
-    {
-      const int cpr = K / 16, chunks = 2 * cols * cpr;
-      for (int ch = tid; ch < chunks; ch += 2 * kGW * 64) {   // two chunks per thread in flight
-        u32x4 v[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int cc = min(ch + q * kGW * 64, chunks - 1);   // no condition on the load
-          const int col = cc / cpr, j = cc % cpr;
-          const int tok = p.xrow[base + c0 + (col >> 1)];
-          v[q] = ldg16(p.xp + static_cast<size_t>(2 * tok + (col & 1)) * K + 16 * j);
-        }
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int cc = ch + q * kGW * 64;
-          if (cc < chunks) {
-            const int col = cc / cpr, j = cc % cpr;   // j: 16-byte chunk of the row, block j / 8
-            *reinterpret_cast<u32x4*>(xq + ((j >> 3) * 16 + col) * 128 + 16 * (j & 7)) = v[q];
-          }
-        }
-      }
-      const int words = 2 * cols * nblk;
-      for (int wi = tid; wi < words; wi += kGW * 64) {
-        const int col = wi / nblk, kb = wi % nblk;
-        const int tok = p.xrow[base + c0 + (col >> 1)];
-        xe[kb * 16 + col] = ldg<uint32_t>(xs + static_cast<size_t>(2 * tok + (col & 1)) * (K / 32) + 4 * kb);
-      }
-    }
-    __syncthreads();
-    // B column of this lane: plane r16 & 1 of tile row r16 >> 1 (columns past
-    // the tile's rows repeat its last one; their results are not stored)
-    const int bc = min(r16, 2 * cols - 1);
-    f32x4 ag = {0.f, 0.f, 0.f, 0.f}, au = ag;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int col = (k0 + i) * 16 + bc;
-      const u32x4* src = reinterpret_cast<const u32x4*>(xq + col * 128 + g4 * 32);
-      const u32x4 blo = src[0], bhi = src[1];
-      const uint32_t bs = (xe[col] >> (8 * g4)) & 0xffu;
-      ag = mx_mfma(c1[i], (s1[i] >> (8 * g4)) & 0xffu, blo, bhi, bs, ag);
-      au = mx_mfma(c3[i], (s3[i] >> (8 * g4)) & 0xffu, blo, bhi, bs, au);
-    }
-    __syncthreads();   // every wave is done with the planes
-    *reinterpret_cast<f32x4*>(&red[item][ks][0][lane][0]) = ag;
-    *reinterpret_cast<f32x4*>(&red[item][ks][1][lane][0]) = au;
-    __syncthreads();
-    float hv[4] = {0.f, 0.f, 0.f, 0.f};   // h of this lane's column and rows (ks == 0 waves)
-    if (ks == 0) {
-#pragma unroll
-      for (int w = 1; w < kGKS; ++w) {
-        ag += *reinterpret_cast<const f32x4*>(&red[item][w][0][lane][0]);
-        au += *reinterpret_cast<const f32x4*>(&red[item][w][1][lane][0]);
-      }
-      float g[4], u[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {   // the row's two plane columns (lanes 2r, 2r + 1)
-        g[q] = ag[q] + lane_xor1(ag[q]);
-        u[q] = au[q] + lane_xor1(au[q]);
-      }
-      const int rr = r16 >> 1;
-      const int r = base + c0 + min(rr, cols - 1);   // dispatch row (columns past the tile: its last)
-      const float wr = p.wrow[r];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) hv[q] = silu_clamped(g[q], u[q], p.limit) * wr;
-      if (!p.hplanes && rok && (r16 & 1) == 0 && rr < cols) {
-        uint16_t hh[4], hl[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) split_bf16(hv[q], hh[q], hl[q]);
-        const int64_t off = static_cast<int64_t>(r) * p.I + rt * 16 + 4 * g4;
-        *reinterpret_cast<uint2*>(p.h_hi + off) = uint2{hh[0] | (uint32_t(hh[1]) << 16), hh[2] | (uint32_t(hh[3]) << 16)};
-        *reinterpret_cast<uint2*>(p.h_lo + off) = uint2{hl[0] | (uint32_t(hl[1]) << 16), hl[2] | (uint32_t(hl[3]) << 16)};
-      }
-      if (p.hplanes) {
-        // one exponent per (row, 32-row group): the largest |h| of this tile's 16 rows
-        float m = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) m = fmaxf(m, fabsf(hv[q]));
-        m = max_over_rows(m);
-        // (addresses from a copy of the lane id made here: forms hoisted out of the
-        // column loop stayed live across the weight stream and spilled)
-        int ln = lane;
-        asm volatile("" : "+v"(ln));
-        if (ln < 16) gmx[item * 16 + ln] = m;
-      }
-    }
-    if (p.hplanes) {
-      // h as three FP8 planes per dispatch row (the MX down's B operand): the
-      // block's two row tiles are one 32-row exponent group
-      __syncthreads();
-      int ln = lane;   // (as above)
-      asm volatile("" : "+v"(ln));
-      const int c16 = ln & 15, q4 = ln >> 4, rr = c16 >> 1;
-      if (ks == 0 && rok && (c16 & 1) == 0 && rr < cols) {
-        const int r = base + c0 + rr;
-        const int e = fp8_plane_exp(fmaxf(gmx[c16], gmx[16 + c16]));
-        uint32_t w[3];
-        fp8_planes4<3>(hv, e, w);
-        const int I = p.I, i0 = rt * 16 + 4 * q4;
-        uint8_t* dst = p.hp + static_cast<size_t>(3 * r) * I + (i0 >> 7) * 128 + b_perm(i0 & 127);
-#pragma unroll
-        for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<uint32_t*>(dst + static_cast<size_t>(pl) * I) = w[pl];
-        if (item == 0 && q4 == 0) {
-          uint8_t* sc = p.hp + static_cast<size_t>(p.T) * p.k * 3 * I;
-#pragma unroll
-          for (int pl = 0; pl < 3; ++pl)
-            sc[static_cast<size_t>(3 * r + pl) * (I / 32) + (i0 >> 5)] = static_cast<uint8_t>(e8m0_byte(e - 4 * pl));
-        }
-      }
-    }
-    __syncthreads();   // the next column tile reuses the LDS
-  }
 }
 
 // The shared expert over more than kGNC tokens.  Its weights are 50 MB of
@@ -591,14 +414,16 @@ static_assert(kGW * 64 * 2 * 8 == kGsCols * 128, "two chunks per thread stage on
 // steps ahead, before the weights of block t, so copying them into LDS at
 // step t - 1 waits only for weights already used.  Loads past the end
 // re-read block nb - 1 (unused), so no load in the main loop sits under a
-// condition; the last steps load only what remains.
-template <int NB, typename MM, typename LW, typename LX, typename SX>
-__device__ __forceinline__ void gs_walk(int nb, MM mm, LW ldw, LX ldx, SX stx) {
+// condition; the last steps load only what remains.  mid() runs once the
+// first steps' loads are out.
+template <int NB, typename MM, typename LW, typename LX, typename SX, typename Mid>
+__device__ __forceinline__ void gs_walk(int nb, MM mm, LW ldw, LX ldx, SX stx, Mid mid) {
   constexpr int U = NB % 2 == 0 ? NB : 2 * NB;   // steps per pass: slots and buffers back in phase
 #pragma unroll
   for (int i = 0; i < NB; ++i) ldx(i, min(i, nb - 1));
 #pragma unroll
   for (int i = 0; i < NB; ++i) ldw(i, min(i, nb - 1));
+  mid();
   stx(0, 0);
   __syncthreads();
   int s = 0;
@@ -631,7 +456,7 @@ __device__ __forceinline__ void gs_walk(int nb, MM mm, LW ldw, LX ldx, SX stx) {
 // 2i + 1 take row tile 4b + i of w1 (gate) and of w3 (up), so that a wave
 // holds one role's accumulators and a ring of four weight batches; the up
 // wave hands its sums to the gate wave through LDS for SwiGLU.
-__device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, uint16_t* lds) {
+__device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, int first, int step, uint16_t* lds) {
   constexpr int NB = 3;
   const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
@@ -642,7 +467,7 @@ __device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, uint
   const uint16_t* W = role ? p.ws3 : p.ws1;
   const int K = p.H, nb = K / 128;
   f32x4 (*xch)[kGsCT][64] = reinterpret_cast<f32x4 (*)[kGsCT][64]>(lds);   // [pair][tile][lane], after the walk
-  for (int g0 = 0; g0 < p.T; g0 += kGsCols) {
+  for (int g0 = first; g0 < p.T; g0 += step) {
     const int ncol = min(kGsCols, p.T - g0);
     const int nct = (ncol + 15) / 16;
     RawBF16 w[NB];
@@ -658,7 +483,7 @@ __device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, uint
     auto ldw = [&](int i, int kb) { load_raw_nc(w[i], W, row, K, kb * 128 + g4 * 32); };
     auto ldx = [&](int slot, int kb) { gs_load(xv[slot], p.x, K, g0, ncol, kb); };
     auto stx = [&](int slot, int buf) { gs_store(xv[slot], lds + buf * kGsPlane); };
-    gs_walk<NB>(nb, mm, ldw, ldx, stx);   // ends with a barrier: the buffers are free
+    gs_walk<NB>(nb, mm, ldw, ldx, stx, [] {});   // ends with a barrier: the buffers are free
     if (role) {
 #pragma unroll
       for (int c = 0; c < kGsCT; ++c) xch[pair][c][lane] = acc[c];
@@ -690,14 +515,14 @@ static_assert(size_t{kGW / 2} * kGsCT * 64 * 16 <= gs_up_lds_bytes(), "the SwiGL
 // Down of the shared expert over more than kGNC tokens, as up_shared_wide:
 // block b's eight waves each take one row tile of w2 (16 output rows) over
 // K = Is, the h planes (hi, lo) of up to kGsCols tokens staged per K block.
-__device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, uint16_t* lds) {
+__device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, int first, int step, uint16_t* lds) {
   constexpr int NB = 2;
   const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
   const int rt = b * kDW + wave;
   const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
   const int K = p.Is, nb = K / 128;
-  for (int g0 = 0; g0 < p.T; g0 += kGsCols) {
+  for (int g0 = first; g0 < p.T; g0 += step) {
     const int ncol = min(kGsCols, p.T - g0);
     const int nct = (ncol + 15) / 16;
     RawBF16 w[NB];
@@ -725,7 +550,7 @@ __device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, ui
       gs_store(xh[slot], lds + buf * 2 * kGsPlane);
       gs_store(xl[slot], lds + buf * 2 * kGsPlane + kGsPlane);
     };
-    gs_walk<NB>(nb, mm, ldw, ldx, stx);
+    gs_walk<NB>(nb, mm, ldw, ldx, stx, [] {});
 #pragma unroll
     for (int c = 0; c < kGsCT; ++c) {
       const int t = c * 16 + r16;
@@ -733,6 +558,332 @@ __device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, ui
     }
     __syncthreads();   // the next group restages buffer 0
   }
+}
+
+// ---------------------------------------------------------------- wide FP4 slots
+// FP4 slots on v_mfma_scale_f32_16x16x128_f8f6f4 with the block's eight waves
+// walking all of K together (gs_walk), 256 of K a step: each wave multiplies
+// two weight row tiles (gate/up: the same 16 rows of w1 and w3; down: 32 rows
+// of w2), whose codes go from memory straight into its registers, by up to
+// 16 NCT dispatch rows, whose planes the block stages in LDS, one barrier a
+// step.  A dispatch row is one B column and its planes are products of their
+// own into the same accumulators (plane p's scale is plane 0's times 2^-4p),
+// so 16 rows share a column tile.
+//
+// WidePlanes ("stage rows"): row r of K values in NP FP8 planes takes NP K
+// bytes, NP x 64 per 64-value stage (plane by plane, plain K order), and one
+// E8M0 byte (plane 0's) per 32 values in an array of its own.
+//
+// What bounds it: the weight stream (16 waves of two blocks a CU, NB steps of
+// 4 KB each in flight).  A step is 256 of K so that a row's 128-byte cache line
+// is asked for in one go: with steps of 128 (the line's halves about 2 us
+// apart, when many lines had left the L2 again) the gate/up took 402 us at 200
+// tokens (H 4096, top-8 of 256: 1.8 GB of w1 / w3) against 346 (5.3 TB/s), and
+// 363 at H 5120 and 24 tokens (top-6 of 384) against 306.  The kernels these
+// replace: blocks of one row tile pair whose waves held four K ranges whole
+// and took eight rows a pass (same box, 20 / 64 / 96 tokens at H 4096: gate/up
+// 168 / 345 / 367 -> 161 / 259 / 294 us, down 84 / 176 / 218 -> 88 / 158 / 170;
+// H 5120 had bf16 products there: 407 -> 306 and 162 -> 142 us at 24 tokens),
+// and, from 128 tokens, GEMM tiles of 128 rows (200 tokens: 573 -> 346 and 290
+// -> 204 us, the shared expert included).
+constexpr int kWdWaves = 8;
+constexpr int kWdStep = 256;         // K of a step
+constexpr int kWdScales = 8;         // 8-byte pieces of the weights' scales a lane holds (K up to 4096 at once)
+
+// LDS of a wide block: two buffers of a step's planes (rows padded by 16
+// bytes: 16 rows at one chunk then fall on distinct banks), the dispatch rows'
+// exponents and the weight rows' E8M0 bytes for all of K (rows padded by a
+// word for the same reason).
+constexpr int wd_row(int NP) { return NP * kWdStep + 16; }
+__host__ __device__ constexpr int wd_scale_row(int K) { return K / 32 + 4; }
+constexpr size_t wd_lds_bytes(int NCT, int NP, int K) {
+  return size_t{2} * (16 * NCT) * wd_row(NP) + size_t(16 * NCT + 32 * kWdWaves) * wd_scale_row(K);
+}
+
+// n rows of K / 32 scale bytes each (row r at src(r)) into LDS rows of
+// wd_scale_row(K) by `threads` threads from thread `t`, in pieces of 8 bytes
+// (K % 256 == 0): load() issues the first Q pieces a thread, store() puts them
+// away and copies what is left.
+template <int Q>
+struct WideScales {
+  u32x2 v[Q];
+  // piece c's row: c / (K / 256) through a 16-bit reciprocal (exact: c < 2^11, K / 256 < 2^5)
+  static __device__ __forceinline__ int row(int c, int inv) { return static_cast<int>(__umul24(c, inv) >> 16); }
+  static __device__ __forceinline__ void put(uint8_t* dst, int K, int c, int r, const u32x2& x) {
+    uint32_t* d = reinterpret_cast<uint32_t*>(dst + r * wd_scale_row(K) + 8 * (c - r * (K / 256)));
+    d[0] = x.x;
+    d[1] = x.y;
+  }
+  template <typename Src>
+  static __device__ __forceinline__ u32x2 get(int K, int c, int r, Src src) {
+    return ldg<u32x2>(src(r) + 8 * (c - r * (K / 256)));
+  }
+  template <typename Src>
+  __device__ __forceinline__ void load(int n, int K, int inv, int t, int threads, Src src) {
+    const int last = n * (K / 256) - 1;
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+      const int c = min(t + i * threads, last);   // no condition on the load
+      v[i] = get(K, c, row(c, inv), src);
+    }
+  }
+  template <typename Src>
+  __device__ __forceinline__ void store(uint8_t* dst, int n, int K, int inv, int t, int threads, Src src) {
+    const int total = n * (K / 256);
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+      const int c = t + i * threads;
+      if (c < total) put(dst, K, c, row(c, inv), v[i]);
+    }
+    for (int c = t + Q * threads; c < total; c += threads) {
+      const int r = row(c, inv);
+      put(dst, K, c, r, get(K, c, r, src));
+    }
+  }
+};
+
+// acc[a][c] = row tile a of this wave (16 weight rows, this lane's at W[a] +
+// co[a], their scales at row a of S) by the tile's rows 16 c + [0, 16): n rows
+// from source row src(r) of the planes q / exponents e.
+template <int NCT, int NP, int NB, typename Src>
+__device__ __forceinline__ void wide_mul(const uint8_t* const (&W)[2], const uint8_t* const (&S)[2],
+                                         const uint32_t (&co)[2], const uint32_t (&so)[2], const uint8_t* q,
+                                         const uint8_t* e, int K, int n, Src src, uint8_t* lds,
+                                         f32x4 (&acc)[2][NCT]) {
+  constexpr int kThreads = kWdWaves * 64, kRow = wd_row(NP), kBuf = 16 * NCT * kRow;
+  constexpr int kPer = NP * (kWdStep / 16), kChunks = 16 * NCT * kPer;   // 16-byte pieces of a row, of a step
+  constexpr int Q = (kChunks + kThreads - 1) / kThreads;
+  // (from a copy of the thread id made here: addresses hoisted out of a loop over a
+  // slot's rows would be spilled)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int es = wd_scale_row(K);
+  uint8_t* xe = lds + 2 * kBuf;
+  uint8_t* ws = xe + 16 * NCT * es + wave * 32 * es;
+  // this thread's pieces: row c / kPer, piece c % kPer; rows past n repeat the last
+  uint32_t xs[Q];   // (offsets from q: the planes are below 4 GB, wide_shapes)
+  int xo[Q];
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const int c = min(tid + i * kThreads, kChunks - 1);
+    const int r = c / kPer, j = c - r * kPer;
+    xs[i] = static_cast<uint32_t>(src(min(r, n - 1))) * static_cast<uint32_t>(NP * K) + 16 * j;
+    xo[i] = r * kRow + 16 * j;
+  }
+  const int inv = (65536 + K / 256 - 1) / (K / 256);
+  auto esrc = [&](int r) { return e + static_cast<uint32_t>(src(r)) * static_cast<uint32_t>(K / 32); };
+  auto wsrc = [&](int r) { return (r < 16 ? S[0] + so[0] : S[1] + so[1]) + (r & 15) * (K / 32); };
+  WideScales<NCT> esc;
+  WideScales<kWdScales> wsc;
+  wsc.load(32, K, inv, lane, 64, wsrc);
+  esc.load(n, K, inv, tid, kThreads, esrc);
+  u32x4 w[NB][2][2];   // [slot][row tile][K block]: a row's 128 bytes in one go (whole cache lines)
+  u32x4 xv[NB][Q];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) acc[a][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint8_t* wsl = ws + r16 * es + g4;                    // + 8 per step
+  const uint8_t* xel = xe + min(r16, n - 1) * es + g4;
+  const int xn = max(n - 1 - r16, 0);                         // column tile c reads row min(16 c, xn) further
+  auto mm = [&](int i, int buf) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint8_t* xb = lds + buf * kBuf + r16 * kRow + 16 * g4 + b * 128 * NP;
+      const uint32_t s0 = wsl[4 * b], s1 = wsl[16 * es + 4 * b];
+#pragma unroll
+      for (int c = 0; c < NCT; ++c) {
+        // the operands of one column tile at a time, its products here (left to the
+        // compiler they sink to the end of a pass of steps, all operands live, and spill)
+        asm volatile("" : "+v"(acc[0][c]), "+v"(acc[1][c])::"memory");
+        const uint32_t bs = xel[min(16 * c, xn) * es + 4 * b];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          const uint8_t* x = xb + c * 16 * kRow + 64 * p;
+          const u32x4 lo = *reinterpret_cast<const u32x4*>(x), hi = *reinterpret_cast<const u32x4*>(x + 64 * NP);
+          acc[0][c] = mx_mfma(w[i][0][b], s0, lo, hi, bs - 4u * p, acc[0][c]);
+          acc[1][c] = mx_mfma(w[i][1][b], s1, lo, hi, bs - 4u * p, acc[1][c]);
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) asm volatile("" : "+v"(acc[0][c]), "+v"(acc[1][c])::"memory");
+    wsl += 8;
+    xel += 8;
+  };
+  auto ldw = [&](int i, int kb) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      w[i][a][0] = ldg16(W[a] + kb * (kWdStep / 2) + co[a]);
+      w[i][a][1] = ldg16(W[a] + kb * (kWdStep / 2) + co[a] + 64);
+    }
+  };
+  auto ldx = [&](int i, int kb) {
+#pragma unroll
+    for (int j = 0; j < Q; ++j) xv[i][j] = ldg16(q + kb * (NP * kWdStep) + xs[j]);
+  };
+  auto stx = [&](int i, int buf) {
+#pragma unroll
+    for (int j = 0; j < Q; ++j)
+      if (kChunks % kThreads == 0 || tid + j * kThreads < kChunks)
+        *reinterpret_cast<u32x4*>(lds + buf * kBuf + xo[j]) = xv[i][j];
+  };
+  // the scales' loads go out ahead of the first steps' and are put away behind them
+  gs_walk<NB>(K / kWdStep, mm, ldw, ldx, stx, [&] {
+    asm volatile("" ::: "memory");
+    wsc.store(ws, 32, K, inv, lane, 64, wsrc);
+    esc.store(xe, n, K, inv, tid, kThreads, esrc);
+  });   // ends with a barrier: the buffers are free
+}
+
+// Gate/up of one FP4 slot: rows 128 grp + [0, 128) of w1 and w3 for dispatch
+// rows base + c0 + [0, min(n - c0, 16 NCT)); h in NPH planes (two: of h rounded
+// to bf16, as the prefill GEMM rounds it).
+template <int NCT, int NB, int NPH>
+__device__ __forceinline__ void up_wide_tile(const GroupedArgs& p, const void* const* wp, int grp, int n, int base,
+                                             uint8_t* lds) {
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int rt = grp * kWdWaves + wave;
+  const bool rok = rt < p.I / 16;
+  const int K = p.H;
+  const uint32_t row = rok ? static_cast<uint32_t>(rt * 16 + r16) : 0u;
+  const uint8_t* const W[2] = {static_cast<const uint8_t*>(wp[0]), static_cast<const uint8_t*>(wp[2])};
+  const uint8_t* const S[2] = {static_cast<const uint8_t*>(wp[1]), static_cast<const uint8_t*>(wp[3])};
+  const uint32_t c0 = row * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
+  const uint32_t s0 = (rok ? static_cast<uint32_t>(rt * 16) : 0u) * static_cast<uint32_t>(K / 32);   // (the tile's first row)
+  const uint32_t co[2] = {c0, c0}, so[2] = {s0, s0};
+  f32x4 acc[2][NCT];
+  wide_mul<NCT, 2, NB>(W, S, co, so, p.xp, p.xe, K, n, [&](int r) { return p.xrow[base + r]; }, lds, acc);
+  float (*gmx)[NCT][16] = reinterpret_cast<float (*)[NCT][16]>(lds);   // [wave][tile][row]: largest of its 16 features
+  float hv[NCT][4];
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) {
+    const float wr = p.wrow[base + min(16 * c + r16, n - 1)];
+    float m = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v = silu_clamped(acc[0][c][q], acc[1][c][q], p.limit) * wr;
+      if constexpr (NPH == 2) v = bf16_bits_to_f32(f32_to_bf16_bits(v));
+      hv[c][q] = rok ? v : 0.0f;
+      m = fmaxf(m, fabsf(hv[c][q]));
+    }
+    m = max_over_rows(m);
+    if (g4 == 0) gmx[wave][c][r16] = m;
+  }
+  __syncthreads();
+  // one exponent per dispatch row and 32 features (waves 2j, 2j + 1)
+  const int i0 = rt * 16 + 4 * g4;
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) {
+    const int ex = fp8_plane_exp(fmaxf(gmx[wave][c][r16], gmx[wave ^ 1][c][r16]));
+    uint32_t pl[NPH];
+    fp8_planes4<NPH>(hv[c], ex, pl);
+    if (rok && 16 * c + r16 < n) {
+      const int64_t r = base + 16 * c + r16;
+      uint8_t* dst = p.hp + r * (NPH * p.I) + (i0 >> 6) * (64 * NPH) + (i0 & 63);
+#pragma unroll
+      for (int i = 0; i < NPH; ++i) *reinterpret_cast<uint32_t*>(dst + 64 * i) = pl[i];
+      if ((wave & 1) == 0 && g4 == 0) p.he[r * (p.I / 32) + (i0 >> 5)] = static_cast<uint8_t>(e8m0_byte(ex));
+    }
+  }
+  __syncthreads();   // the next rows reuse the LDS
+}
+
+// Down of one FP4 slot: output rows 256 grp + [0, 256) of w2 for n dispatch
+// rows from base; h in NPH planes.
+template <int NCT, int NB, int NPH>
+__device__ __forceinline__ void down_wide_tile(const GroupedArgs& p, int slot, int grp, int n, int base,
+                                               uint8_t* lds) {
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int rt = (grp * kWdWaves + wave) * 2;
+  const int K = p.I;
+  const uint8_t* W2 = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 6));
+  const uint8_t* S2 = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 7));
+  const uint8_t* const W[2] = {W2, W2};
+  const uint8_t* const S[2] = {S2, S2};
+  const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
+  const uint32_t c0 = row * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
+  const uint32_t s0 = static_cast<uint32_t>(rt * 16) * static_cast<uint32_t>(K / 32);
+  const uint32_t co[2] = {c0, c0 + static_cast<uint32_t>(8 * K)}, so[2] = {s0, s0 + static_cast<uint32_t>(K / 2)};
+  f32x4 acc[2][NCT];
+  wide_mul<NCT, NPH, NB>(W, S, co, so, p.hp, p.he, K, n, [&](int r) { return base + r; }, lds, acc);
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) {
+    if (16 * c + r16 >= n) continue;
+    const int64_t o = static_cast<int64_t>(base + 16 * c + r16) * p.H + rt * 16 + 4 * g4;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      if (p.y_bf16) {
+        uint16_t b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b[q] = f32_to_bf16_bits(acc[a][c][q]);
+        *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.y) + o + 16 * a) =
+            uint2{b[0] | (uint32_t(b[1]) << 16), b[2] | (uint32_t(b[3]) << 16)};
+      } else {
+        *reinterpret_cast<f32x4*>(p.y + o + 16 * a) = acc[a][c];
+      }
+    }
+  }
+}
+
+// Rows of a slot in passes of the widest tile the remaining ones fill.
+// Column tiles of a pass and steps in flight.  Of one column tile three steps:
+// two took 289 us of gate/up at 64 tokens (H 4096, top-8 of 256) against 259,
+// four 307 (12 KB in flight per wave then overrun the XCD's L2: a 128-byte row
+// piece is two loads).  Two column tiles leave registers for two steps; four
+// spill.
+constexpr int kWdMaxCT = 2;
+constexpr int kWdNB1 = 3, kWdNB2 = 2;
+
+// Blocks [0, up_shared): the shared expert, sh_tg groups of kGsCols tokens
+// each; the others: up_groups blocks per slot.
+template <int NPH>
+__global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_up_wide(GroupedArgs p) {
+  extern __shared__ __align__(16) uint16_t lds_g[];
+  uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
+  const int b = static_cast<int>(blockIdx.x);
+  if (b < p.up_shared) {
+    up_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    return;
+  }
+  const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
+  if (slot >= p.active[0] || (p.on && !*p.on)) return;
+  const SlotDesc* d = p.desc + slot;
+  const int n = d->n_tok, base = d->tok_base;
+  if (n > p.max_rows) return;
+  const void* const wp[4] = {desc_ptr(p.desc, slot, 0), desc_ptr(p.desc, slot, 1), desc_ptr(p.desc, slot, 3),
+                             desc_ptr(p.desc, slot, 4)};
+  int r = 0;
+  for (; n - r > 32; r += 16 * kWdMaxCT)
+    up_wide_tile<kWdMaxCT, kWdNB2, NPH>(p, wp, grp, min(n - r, 16 * kWdMaxCT), base + r, lds);
+  if (n - r > 16) up_wide_tile<2, kWdNB2, NPH>(p, wp, grp, n - r, base + r, lds);
+  else if (n > r) up_wide_tile<1, kWdNB1, NPH>(p, wp, grp, n - r, base + r, lds);
+}
+
+template <int NPH>
+__global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_down_wide(GroupedArgs p) {
+  extern __shared__ __align__(16) uint16_t lds_g[];
+  uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
+  const int b = static_cast<int>(blockIdx.x);
+  if (b < p.dn_shared) {
+    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    return;
+  }
+  const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
+  if (slot >= p.active[0] || (p.on && !*p.on)) return;
+  const SlotDesc* d = p.desc + slot;
+  const int n = d->n_tok, base = d->tok_base;
+  if (n > p.max_rows) return;
+  int r = 0;
+  for (; n - r > 32; r += 16 * kWdMaxCT)
+    down_wide_tile<kWdMaxCT, kWdNB2, NPH>(p, slot, grp, min(n - r, 16 * kWdMaxCT), base + r, lds);
+  if (n - r > 16) down_wide_tile<2, kWdNB2, NPH>(p, slot, grp, n - r, base + r, lds);
+  else
+  if (n > r) down_wide_tile<1, kWdNB1, NPH>(p, slot, grp, n - r, base + r, lds);
 }
 
 // Blocks [0, up_shared): the shared expert (bf16 w1/w3, all T tokens); the
@@ -744,7 +895,7 @@ __global__ __launch_bounds__(kGW * 64) __attribute__((amdgpu_waves_per_eu(4))) v
   const int item = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kGKS;
   if (b < p.up_shared) {
     if (p.T > kGNC) {
-      up_shared_wide(p, b, lds_g);
+      up_shared_wide(p, b, 0, kGsCols, lds_g);
       return;
     }
     const int rt = b * kGI + item;
@@ -763,19 +914,6 @@ __global__ __launch_bounds__(kGW * 64) __attribute__((amdgpu_waves_per_eu(4))) v
     if (p.q3f) {   // one row tile per block (up_groups = I / 16)
       const int rt1 = rb % p.up_groups;
       up_block_q3f(p, wp, rt1, rt1 < p.I / 16, d->n_tok, d->tok_base, lds_g);
-      return;
-    }
-  }
-  if constexpr (std::is_same_v<Raw, RawFP4>) {
-    if (p.mx) {
-      uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
-      const bool rok = rt < p.I / 16;
-      switch (p.mx) {   // blocks per wave: H / 128 / kGKS
-        case 2: up_block_mx<2>(p, wp, rt, rok, d->n_tok, d->tok_base, lds); break;
-        case 4: up_block_mx<4>(p, wp, rt, rok, d->n_tok, d->tok_base, lds); break;
-        case 6: up_block_mx<6>(p, wp, rt, rok, d->n_tok, d->tok_base, lds); break;
-        default: up_block_mx<8>(p, wp, rt, rok, d->n_tok, d->tok_base, lds); break;
-      }
       return;
     }
   }
@@ -876,91 +1014,6 @@ __device__ __forceinline__ void down_block(const GroupedArgs& p, LoadW load_w, W
       float* out = shared ? p.ys : p.y;
       *reinterpret_cast<f32x4*>(out + static_cast<int64_t>(base + c0 + r16) * p.H + rt * 16 + 4 * g4) = acc;
     }
-    __syncthreads();   // the next column tile reuses the LDS
-  }
-}
-
-// Down of one FP4 slot block on scaled MFMAs: row tile rt (output rows
-// 16 rt ..) of w2 over K = I = 128 NKB, for the n dispatch rows base ..
-// base + n - 1, h as the gate/up's three FP8 planes per row (B column 3r + p:
-// five rows per column tile).  The wave's whole range of w2 codes and E8M0
-// words is issued first, then the tile's plane rows are copied into LDS;
-// one MFMA per block, a row's three plane columns added in order.  Writes
-// one float32 output row per dispatch row, as down_block.
-constexpr int kGdRows = 5;   // dispatch rows of an MX down column tile (15 B columns)
-
-__host__ __device__ inline size_t gd_lds_bytes(int I) { return static_cast<size_t>(I / 128) * 16 * (128 + 4); }
-
-template <int NKB>
-__device__ __forceinline__ void down_block_mx(const GroupedArgs& p, int slot, int rt, int n, int base,
-                                              uint8_t* lds) {
-  const int tid = threadIdx.x, lane = __lane_id();
-  const int r16 = lane & 15, g4 = lane >> 4;
-  const int I = p.I;
-  uint8_t* hq = lds;
-  uint32_t* he = reinterpret_cast<uint32_t*>(lds + static_cast<size_t>(NKB) * 16 * 128);
-  const uint8_t* W = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 6));
-  const uint8_t* S = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 7));
-  const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
-  const uint32_t cb = row * static_cast<uint32_t>(I / 2) + static_cast<uint32_t>(g4 * 16);
-  const uint32_t sb = row * static_cast<uint32_t>(I / 32);
-  const uint8_t* hs = p.hp + static_cast<size_t>(p.T) * p.k * 3 * I;   // the planes' E8M0 bytes
-  for (int c0 = 0; c0 < n; c0 += kGdRows) {
-    const int cols = min(kGdRows, n - c0);
-    u32x4 c[NKB];
-    uint32_t sc[NKB];
-#pragma unroll
-    for (int i = 0; i < NKB; ++i) {
-      c[i] = ldg16(W + cb + i * 64);
-      sc[i] = ldg<uint32_t>(S + sb + i * 4);
-    }
-    asm volatile("" ::: "memory");
-    {
-      const int cpr = I / 16, chunks = 3 * cols * cpr;
-      for (int ch = tid; ch < chunks; ch += 4 * kDW * 64) {
-        u32x4 v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int cc = min(ch + q * kDW * 64, chunks - 1);   // no condition on the load
-          const int col = cc / cpr, j = cc % cpr;
-          v[q] = ldg16(p.hp + static_cast<size_t>(3 * (base + c0) + col) * I + 16 * j);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int cc = ch + q * kDW * 64;
-          if (cc < chunks) {
-            const int col = cc / cpr, j = cc % cpr;
-            *reinterpret_cast<u32x4*>(hq + ((j >> 3) * 16 + col) * 128 + 16 * (j & 7)) = v[q];
-          }
-        }
-      }
-      const int words = 3 * cols * NKB;
-      for (int wi = tid; wi < words; wi += kDW * 64) {
-        const int col = wi / NKB, kb = wi % NKB;
-        he[kb * 16 + col] = ldg<uint32_t>(hs + static_cast<size_t>(3 * (base + c0) + col) * (I / 32) + 4 * kb);
-      }
-    }
-    __syncthreads();
-    // B column of this lane: plane r16 % 3 of tile row r16 / 3 (columns past
-    // the tile's rows repeat its last one; their results are not stored)
-    const int bc = min(r16, 3 * cols - 1);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < NKB; ++i) {
-      const int col = i * 16 + bc;
-      const u32x4* src = reinterpret_cast<const u32x4*>(hq + col * 128 + g4 * 32);
-      const u32x4 blo = src[0], bhi = src[1];
-      const uint32_t bs = (he[col] >> (8 * g4)) & 0xffu;
-      acc = mx_mfma(c[i], (sc[i] >> (8 * g4)) & 0xffu, blo, bhi, bs, acc);
-    }
-    // row t = r16 of this lane group: columns 3t .. 3t + 2, added in order
-    const int t = min(r16, cols - 1), gb = lane & 48;
-    f32x4 ra;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      ra[q] = (__shfl(acc[q], gb + 3 * t, 64) + __shfl(acc[q], gb + 3 * t + 1, 64)) + __shfl(acc[q], gb + 3 * t + 2, 64);
-    if (r16 < cols)
-      *reinterpret_cast<f32x4*>(p.y + static_cast<int64_t>(base + c0 + r16) * p.H + rt * 16 + 4 * g4) = ra;
     __syncthreads();   // the next column tile reuses the LDS
   }
 }
@@ -1090,7 +1143,7 @@ k_down_grouped(GroupedArgs p) {
   const int item = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kDKS;
   if (b < p.dn_shared) {
     if (p.T > kGNC) {
-      down_shared_wide(p, b, lds_g);
+      down_shared_wide(p, b, 0, kGsCols, lds_g);
       return;
     }
     const int rt = b * kDI + item;
@@ -1109,17 +1162,6 @@ k_down_grouped(GroupedArgs p) {
       return;
     }
   }
-  if constexpr (std::is_same_v<Raw, RawFP4>) {
-    if (p.hplanes) {
-      uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
-      switch (p.I / 128) {   // blocks of K per wave (grouped_h_planes)
-        case 4: down_block_mx<4>(p, slot, rt, d->n_tok, d->tok_base, lds); break;
-        case 8: down_block_mx<8>(p, slot, rt, d->n_tok, d->tok_base, lds); break;
-        default: down_block_mx<16>(p, slot, rt, d->n_tok, d->tok_base, lds); break;
-      }
-      return;
-    }
-  }
   auto load_w = [&](Raw& r, uint32_t row, int kc) { load_w2_nc(r, p.desc, slot, row, p.I, kc); };
   auto wptr = [&](int i) { return desc_ptr(p.desc, slot, 6 + i); };   // 0: w2 codes, 1: w2 scales
   down_block<Raw>(p, load_w, wptr, rt, d->n_tok, d->tok_base, false, lds_g);
@@ -1130,30 +1172,9 @@ bool up_q3f(const dsk_moe_desc& d) {
   return d.quant == DSK_QUANT_Q3 && d.hidden % (kQ3gKS * 512) == 0 && d.hidden <= kQ3gMaxGroups * 64;
 }
 
-// The FP4 gate/up on scaled MFMAs: bf16 x (planes made from it), every wave's
-// K range 2, 4, 6 or 8 whole blocks (up_block_mx's instances).
-bool up_mx(const dsk_moe_desc& d) {
-  const int per = d.hidden / 128 / kGKS;
-  return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_BF16 && d.hidden % (kGKS * 256) == 0 &&
-         per >= 2 && per <= kGxMaxBlocks;
-}
-
 }  // namespace
 
-// h as FP8 planes and the FP4 down on scaled MFMAs: the gate/up on scaled MFMAs
-// (up_mx), I a whole 4, 8 or 16 blocks (down_block_mx's instances), and at most
-// 512 dispatch rows (measured up to there): at 8 and 20 tokens (top-8) the down
-// went 57.9 -> 50.5 and 102.8 -> 88.6 us; at 64 (once the shared expert's weights
-// streamed once per call) 173.3 -> 157.7 us while the planes epilogue added
-// 11.5 us to the gate/up.
-bool grouped_up_mx(const dsk_moe_desc& d) { return up_mx(d); }
-
 bool grouped_x_q3(const dsk_moe_desc& d) { return up_q3f(d); }
-
-bool grouped_h_planes(const dsk_moe_desc& d) {
-  return up_mx(d) && (d.inter == 512 || d.inter == 1024 || d.inter == 2048) &&
-         static_cast<int64_t>(d.tokens) * d.top_k <= 512;
-}
 
 namespace {
 
@@ -1163,7 +1184,6 @@ size_t up_lds(const dsk_moe_desc& d) {
   // factored q3: the x tile, its group sums [H/128][8][2][2] f32, 64 zero bytes
   const size_t q3f = x_tile + static_cast<size_t>(d.hidden / 128) * kQ3fMaxTokens * 16 + 64;
   size_t base = x_tile > red ? x_tile : red;
-  if (up_mx(d) && gx_lds_bytes(d.hidden) > base) base = gx_lds_bytes(d.hidden);
   if (d.tokens > kGNC && d.inter_shared > 0 && gs_up_lds_bytes() > base) base = gs_up_lds_bytes();
   return up_q3f(d) && q3f > base ? q3f : base;
 }
@@ -1173,12 +1193,6 @@ hipError_t launch_x_q3(const dsk_moe_desc& d, const GroupedArgs& p, hipStream_t 
   uint16_t* xq = reinterpret_cast<uint16_t*>(p.xp);
   float* xg = reinterpret_cast<float*>(p.xp + static_cast<size_t>(d.tokens) * d.hidden * 2);
   launch_kernel(k_x_q3, static_cast<unsigned>((n + 255) / 256), 256, 0, s, p.x, d.tokens, d.hidden, xq, xg);
-  return hipGetLastError();
-}
-
-hipError_t launch_x_planes(const dsk_moe_desc& d, const GroupedArgs& p, hipStream_t s) {
-  const int64_t n = static_cast<int64_t>(d.tokens) * (d.hidden / 8);
-  launch_kernel(k_x_planes, static_cast<unsigned>((n + 255) / 256), 256, 0, s, p.x, d.tokens, d.hidden, p.xp);
   return hipGetLastError();
 }
 
@@ -1193,8 +1207,7 @@ size_t down_lds(const dsk_moe_desc& d) {
   // factored q3: the h tile of I, its group sums [I/128][8][2][2] f32, 64 zero bytes
   const size_t q3f = 2 * static_cast<size_t>(kGNC) * (d.inter + 8) * 2 +
                      static_cast<size_t>(d.inter / 128) * kQ3fMaxTokens * 16 + 64;
-  const size_t mx = grouped_h_planes(d) ? gd_lds_bytes(d.inter) : 0;
-  size_t b2 = mx > base ? mx : base;
+  size_t b2 = base;
   if (d.tokens > kGNC && d.inter_shared > 0 && gs_down_lds_bytes() > b2) b2 = gs_down_lds_bytes();
   return down_q3f(d) && q3f > b2 ? q3f : b2;
 }
@@ -1230,9 +1243,7 @@ GroupedArgs grouped_args(const dsk_moe_desc& d, const Workspace& L, const Expert
   p.ys = reinterpret_cast<float*>(a.ws + L.ys);
   p.q3f = up_q3f(d) ? 1 : 0;
   p.q3fd = down_q3f(d) ? 1 : 0;
-  p.mx = up_mx(d) ? d.hidden / 128 / kGKS : 0;
   p.xp = reinterpret_cast<uint8_t*>(a.ws + L.xp);
-  p.hplanes = 0;   // set by the launchers where the grouped gate/up writes h
   p.hp = reinterpret_cast<uint8_t*>(a.ws + L.hp);
   p.up_groups = p.q3f ? d.inter / 16 : d.inter / 16 / kGI;   // factored q3: one row tile per block
   // shared gate/up: past kGNC tokens, four row tiles per block (up_shared_wide)
@@ -1261,14 +1272,24 @@ hipError_t grouped_down(const dsk_moe_desc& d, const GroupedArgs& p, hipStream_t
 hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                   const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                   int repeat) {
+  hipError_t e;
+  if (grouped_wide(d)) {
+    const WideCall w{3, d.tokens, nullptr, 0, d.inter_shared > 0};
+    if ((e = stage_open(kStageUp)) != hipSuccess) return e;
+    for (int r = 0; r < repeat; ++r) {
+      if (!a.x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
+      if ((e = launch_wide_up(d, L, a, desc, xrow, wrow, w, s)) != hipSuccess) return e;
+    }
+    if ((e = stage_open(kStageDown)) != hipSuccess) return e;
+    for (int r = 0; r < repeat; ++r)
+      if ((e = launch_wide_down(d, L, a, desc, w, s)) != hipSuccess) return e;
+    return e;
+  }
   GroupedArgs p = grouped_args(d, L, a, desc, xrow, wrow);
-  p.hplanes = grouped_h_planes(d) ? 1 : 0;
   const unsigned up_blocks = static_cast<unsigned>(p.up_shared + max_slots(d) * p.up_groups);
   const size_t ul = up_lds(d);
-  hipError_t e;
   if ((e = stage_open(kStageUp)) != hipSuccess) return e;
   for (int r = 0; r < repeat; ++r) {
-    if (p.mx && !a.x_planes_ready && (e = launch_x_planes(d, p, s)) != hipSuccess) return e;
     if (p.q3f && !a.x_planes_ready && (e = launch_x_q3(d, p, s)) != hipSuccess) return e;
     if (d.quant == DSK_QUANT_Q3) launch_kernel(k_up_grouped<RawQ3>, up_blocks, kGW * 64, ul, s, p);
     else launch_kernel(k_up_grouped<RawFP4>, up_blocks, kGW * 64, ul, s, p);
@@ -1278,35 +1299,99 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
   return grouped_down(d, p, s, repeat);
 }
 
+// The wide kernels' rows (max_rows: of the largest slot they may get) and planes fit the LDS.
+size_t wide_lds(int rows, int planes, int K) {
+  return rows <= 16 ? wd_lds_bytes(1, planes, K) : wd_lds_bytes(kWdMaxCT, planes, K);
+}
+
+bool grouped_wide(const dsk_moe_desc& d) { return wide_shapes(d) && grouped_path(d) && !prefill_gemm(d); }
+
+bool wide_shapes(const dsk_moe_desc& d) {
+  return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_BF16 && d.hidden % kWdStep == 0 &&
+         d.inter % kWdStep == 0 && d.inter_shared % 128 == 0 && d.hidden < 8192 && d.inter < 8192 &&
+         int64_t{d.tokens} * d.top_k * 3 * d.inter < (int64_t{1} << 32) &&
+         int64_t{d.tokens} * 2 * d.hidden < (int64_t{1} << 32) && wide_lds(64, 3, d.inter) <= kMaxLds &&
+         wide_lds(64, 2, d.hidden) <= kMaxLds;
+}
+
+namespace {
+
+GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
+                      const int32_t* xrow, const float* wrow, const WideCall& w) {
+  GroupedArgs p = grouped_args(d, L, a, desc, xrow, wrow);
+  p.xe = p.xp + static_cast<size_t>(d.tokens) * 2 * d.hidden;
+  p.he = p.hp + static_cast<size_t>(d.tokens) * d.top_k * w.h_planes * d.inter;
+  p.max_rows = w.max_rows;
+  p.on = w.on;
+  p.y_bf16 = w.y_bf16;
+  p.sh_tg = (d.tokens + kGsCols - 1) / kGsCols;
+  p.up_groups = (d.inter / 16 + kWdWaves - 1) / kWdWaves;
+  p.up_shared = w.shared ? (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2) * p.sh_tg : 0;
+  p.dn_groups = d.hidden / 256;
+  p.dn_shared = w.shared && d.inter_shared > 0 ? d.hidden / 128 * p.sh_tg : 0;
+  return p;
+}
+
+}  // namespace
+
+hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
+                          const int32_t* xrow, const float* wrow, const WideCall& w, hipStream_t s) {
+  const GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, w);
+  const unsigned blocks = static_cast<unsigned>(p.up_shared + max_slots(d) * p.up_groups);
+  const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
+  size_t lds = wide_lds(rows, 2, d.hidden);
+  if (p.up_shared > 0 && gs_up_lds_bytes() > lds) lds = gs_up_lds_bytes();
+  if (w.h_planes == 2) launch_kernel(k_up_wide<2>, blocks, kWdWaves * 64, lds, s, p);
+  else launch_kernel(k_up_wide<3>, blocks, kWdWaves * 64, lds, s, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
+                            const WideCall& w, hipStream_t s) {
+  const GroupedArgs p = wide_args(d, L, a, desc, nullptr, nullptr, w);
+  const unsigned blocks = static_cast<unsigned>(p.dn_shared + max_slots(d) * p.dn_groups);
+  const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
+  size_t lds = wide_lds(rows, w.h_planes, d.inter);
+  if (p.dn_shared > 0 && gs_down_lds_bytes() > lds) lds = gs_down_lds_bytes();
+  if (w.h_planes == 2) launch_kernel(k_down_wide<2>, blocks, kWdWaves * 64, lds, s, p);
+  else launch_kernel(k_down_wide<3>, blocks, kWdWaves * 64, lds, s, p);
+  return hipGetLastError();
+}
+
 hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                     const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                     int repeat, bool x_planes_ready) {
+  const bool wide = grouped_wide(d);
   GroupedArgs p = grouped_args(d, L, a, desc, xrow, wrow);
   p.up_shared = 0;
-  p.hplanes = grouped_h_planes(d) ? 1 : 0;
   const unsigned blocks = static_cast<unsigned>(max_slots(d) * p.up_groups);
   const size_t lds = up_lds(d);
   for (int r = 0; r < repeat; ++r) {
-    if (p.mx && !x_planes_ready) {
-      const hipError_t e = launch_x_planes(d, p, s);
-      if (e != hipSuccess) return e;
+    hipError_t e = hipSuccess;
+    if (wide) {
+      if (!x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
+      if ((e = launch_wide_up(d, L, a, desc, xrow, wrow, WideCall{3, d.tokens, nullptr, 0, false}, s)) != hipSuccess)
+        return e;
+      continue;
     }
-    if (p.q3f) {
-      const hipError_t e = launch_x_q3(d, p, s);
-      if (e != hipSuccess) return e;
-    }
+    if (p.q3f && (e = launch_x_q3(d, p, s)) != hipSuccess) return e;
     if (d.quant == DSK_QUANT_Q3) launch_kernel(k_up_grouped<RawQ3>, blocks, kGW * 64, lds, s, p);
     else launch_kernel(k_up_grouped<RawFP4>, blocks, kGW * 64, lds, s, p);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   return hipSuccess;
 }
 
 hipError_t launch_grouped_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                const SlotDesc* desc, hipStream_t s, int repeat, bool h_planes) {
-  GroupedArgs p = grouped_args(d, L, a, desc, nullptr, nullptr);
-  p.hplanes = h_planes ? 1 : 0;
+  if (h_planes) {
+    for (int r = 0; r < repeat; ++r) {
+      const hipError_t e = launch_wide_down(d, L, a, desc, WideCall{3, d.tokens, nullptr, 0, d.inter_shared > 0}, s);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  const GroupedArgs p = grouped_args(d, L, a, desc, nullptr, nullptr);
   return grouped_down(d, p, s, repeat);
 }
 

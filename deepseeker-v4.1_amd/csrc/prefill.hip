@@ -1143,7 +1143,7 @@ __global__ __launch_bounds__(256) void k_pf_planes(const uint16_t* __restrict__ 
 // the 8-wave kernels (kPfToks rows each); tiles[2 + 2 max_tiles] says which.
 __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ desc,
                                                    const int32_t* __restrict__ active, int E, int T,
-                                                   int with_shared, int max_tiles, int mx,
+                                                   int with_shared, int max_tiles, int mx, int narrow,
                                                    int32_t* __restrict__ tiles) {
   __shared__ int32_t wsum[16];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -1155,7 +1155,8 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   }
   const bool on = mx && __syncthreads_and(ok ? 1 : 0);
   const int rtoks = on ? kPfToksMx : kPfToks;
-  const int cnt = t < n_act ? (desc[t].n_tok + rtoks - 1) / rtoks : 0;
+  const int rows = t < n_act ? desc[t].n_tok : 0;
+  const int cnt = on && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;   // (narrow slots: the wide kernels)
   int incl = cnt;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
@@ -1196,6 +1197,33 @@ int prefill_max_tiles(const dsk_moe_desc& d) {
   return (n + rtoks - 1) / rtoks + slots + shared;
 }
 
+// Slots of up to 32 rows (two column tiles, one pass over the weights) go to the
+// wide kernels, which stream the weights at 4.5 TB/s where a GEMM tile, most
+// of its columns empty, takes 3.5: at H 5120 and 2000 tokens (31 rows a slot
+// on average) gate/up + down 2087 us without, 2010 up to 16 rows, 1976 up to
+// 24, 1905 up to 32.  Where a slot has more than 96 rows on average few are
+// that small, and their launches would cost more than they save.
+int prefill_narrow_rows(const dsk_moe_desc& d) {
+  return prefill_mx(d) && wide_shapes(d) && int64_t{d.tokens} * d.top_k <= int64_t{96} * d.n_experts ? 32 : 0;
+}
+
+// The shared expert's GEMM tiles are one block per 128 features and 256 tokens:
+// 16 blocks at 200 tokens, 107 us beside idle CUs for its gate/up (59 for its
+// down).  Up to 512 tokens it runs as blocks of the wide kernels instead (64
+// tokens and 64 features each), under the routed slots' stream.
+bool prefill_shared_wide(const dsk_moe_desc& d) {
+  return prefill_narrow_rows(d) > 0 && d.inter_shared > 0 && d.tokens <= 512;
+}
+
+hipError_t launch_pf_planes(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s) {
+  const int64_t chunks = static_cast<int64_t>(d.tokens) * (d.hidden / 8);
+  uint8_t* xp = reinterpret_cast<uint8_t*>(a.ws + L.xp);
+  launch_kernel(k_pf_planes, static_cast<unsigned>((chunks + 255) / 256), 256, 0, s,
+                static_cast<const uint16_t*>(a.x), chunks, d.hidden, xp,
+                xp + static_cast<size_t>(d.tokens) * 2 * d.hidden);
+  return hipGetLastError();
+}
+
 hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, const PrefillArgs& a,
                                   hipStream_t s, int repeat) {
   const int T = d.tokens, H = d.hidden, I = d.inter, Is = d.inter_shared;
@@ -1203,8 +1231,11 @@ hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, con
   const int max_tiles = prefill_max_tiles(d);
   int32_t* tiles = reinterpret_cast<int32_t*>(a.ws + L.pf_tiles);
   const bool mx = prefill_mx(d);
-  launch_kernel(k_pf_tiles, 1, 1024, 0, s, a.desc, a.active, d.n_experts, T, Is > 0 ? 1 : 0, max_tiles,
-                mx ? 1 : 0, tiles);
+  const int narrow = prefill_narrow_rows(d);
+  const bool sh_wide = prefill_shared_wide(d);
+  const WideCall wide{2, narrow, tiles + 2 + 2 * max_tiles, prefill_rows_bf16(d, a.rows_out) ? 1 : 0, sh_wide};
+  launch_kernel(k_pf_tiles, 1, 1024, 0, s, a.desc, a.active, d.n_experts, T, Is > 0 && !sh_wide ? 1 : 0, max_tiles,
+                mx ? 1 : 0, narrow, tiles);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
 
@@ -1236,14 +1267,9 @@ hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, con
   // covers its units for either tile size (k_pf_tiles decides on the device)
   if ((e = stage_open(kStageUp)) != hipSuccess) return e;
   const int up_rows = (I > Is ? I : Is) / 128;
-  const int64_t x_chunks = static_cast<int64_t>(T) * (H / 8);
   for (int r = 0; r < repeat; ++r) {
-    if (mx && !a.x_planes_ready) {
-      launch_kernel(k_pf_planes, static_cast<unsigned>((x_chunks + 255) / 256), 256, 0, s,
-                    static_cast<const uint16_t*>(a.x), x_chunks, H, const_cast<uint8_t*>(p.xq),
-                    const_cast<uint8_t*>(p.xe));
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
+    if (mx && !a.x_planes_ready && (e = launch_pf_planes(d, L, *a.call, s)) != hipSuccess) return e;
+    if (narrow && (e = launch_wide_up(d, L, *a.call, a.desc, a.xrow, a.wrow, wide, s)) != hipSuccess) return e;
     if (mx) {
       p.row_tiles = I / 128;
       launch_kernel(k_pf_mx_up, static_cast<unsigned>(max_tiles * p.row_tiles), kMxThreads, kMxLdsBytes, s, p);
@@ -1259,6 +1285,7 @@ hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, con
   p.row_tiles = H / kPfRows;
   const unsigned down_blocks = static_cast<unsigned>(max_tiles * p.row_tiles);
   for (int r = 0; r < repeat; ++r) {
+    if (narrow && (e = launch_wide_down(d, L, *a.call, a.desc, wide, s)) != hipSuccess) return e;
     if (mx) {
       launch_kernel(k_pf_mx_down, down_blocks, kMxThreads, kMxLdsBytes, s, p);
       if ((e = hipGetLastError()) != hipSuccess) return e;

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void k_gate(GateArgs g) {
 // One wave per token: biased top-k + normalised weights (unfused path).
 // With xp, the blocks after the top-k's ((T + 3) / 4) write x in the form
 // of the gate/up that follows, one 8-value chunk per thread (XForm: the work
-// of k_x_planes, k_x_q3 or k_pf_planes, without a launch of its own).
+// of k_x_q3 or k_pf_planes, without a launch of its own).
 __global__ __launch_bounds__(256) void k_topk(const float* __restrict__ scores,
                                               const float* __restrict__ bias, int T, int E,
                                               int k, float route_scale,
@@ -132,10 +132,8 @@ __global__ __launch_bounds__(256) void k_topk(const float* __restrict__ scores,
     if (form == kXGroupedQ3)
       x_q3_chunk(x, H, min(c, n - 1), c < n, reinterpret_cast<uint16_t*>(xp),
                  reinterpret_cast<float*>(xp + plane_bytes));
-    else if (form == kXPrefillPlanes)
-      pf_planes_chunk(x, H, min(c, n - 1), c < n, xp, xp + plane_bytes);
     else
-      x_planes_chunk(x, T, H, min(c, n - 1), c < n, xp);
+      pf_planes_chunk(x, H, min(c, n - 1), c < n, xp, xp + plane_bytes);
     return;
   }
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);

@@ -1,0 +1,59 @@
+"""GPU parity of the wide FP4 kernels (a slot's dispatch rows in passes of up to 32
+over the whole of K) against the oracle, where their tiles can go wrong: one row,
+15 / 16 / 17 rows (a column tile and its edge), 31 / 32 / 33 (a pass and its edge),
+an intermediate that fills its last block of row tiles in part, and, from 128
+tokens, slots on both sides of the rows the GEMM tiles take over at."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import dsk_moe
+from oracle import layer as L
+from oracle import synth
+from conftest import assert_layer_close
+from test_gpu_layer import to_bank, to_shared
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _check(spec, T, hot, seed, label, shared=True):
+    print(f"wide {label} T={T} hot={hot}", flush=True)
+    d = synth.make_layer(spec, seed, T)
+    if hot:
+        d["gate_b"] = d["gate_b"].clone()
+        d["gate_b"][:hot] += 10.0          # every token goes to experts 0 .. hot - 1
+    r = L.moe_forward(d["x"], d["gate_w"], d["gate_b"], d["bank"], d["shared"] if shared else None, spec)
+    idx = torch.empty((T, spec.k), dtype=torch.int32, device=DEV)
+    layer = dsk_moe.MoELayer(d["gate_w"].to(DEV), d["gate_b"].to(DEV), to_bank(d["bank"]),
+                             to_shared(d["shared"]) if shared else None, spec.k)
+    x = d["x"].to(DEV)
+    out = layer(x, idx=idx)
+    again = layer(x)
+    assert torch.equal(out.view(torch.int16), again.view(torch.int16))
+    np.testing.assert_array_equal(idx.cpu().numpy(), r["idx"])
+    c, rel = assert_layer_close(out.cpu().float(), r["y_ref"])
+    print(f"cos={c:.9f} rel={rel:.2e} rows {sorted(set(int(v) for v in r['counts']))}", flush=True)
+    return r
+
+
+@pytest.mark.parametrize("T,hot", [(9, 0), (15, 4), (16, 4), (17, 4), (31, 4), (32, 4), (33, 4), (127, 4)])
+def test_wide_rows_of_a_slot(T, hot):
+    _check(L.LayerSpec(H=1024, E=24, k=4, I=512, I_shared=256), T, hot, 310 + T, "rows")
+
+
+@pytest.mark.parametrize("H,I,Is", [(1024, 256, 128), (5120, 768, 384), (2048, 2304, 0)])
+def test_wide_shapes(H, I, Is):
+    """Two K steps, an odd number of them, and rows of scales of 8-byte pieces."""
+    _check(L.LayerSpec(H=H, E=6, k=2, I=I, I_shared=Is or 128), 20, 0, 330, f"H {H} I {I}", shared=Is > 0)
+
+
+@pytest.mark.parametrize("T,E,k", [(128, 64, 4), (150, 16, 4), (300, 24, 4), (520, 64, 2)])
+def test_wide_slots_beside_gemm_tiles(T, E, k):
+    """From 128 tokens: slots of up to 32 rows beside GEMM tiles of 64 and 128 columns,
+    the shared expert in the wide kernels (up to 512 tokens) and in GEMM tiles."""
+    r = _check(L.LayerSpec(H=1024, E=E, k=k, I=768, I_shared=256), T, 0, 350, f"E {E} k {k}")
+    assert int(r["counts"].min()) <= 32 or E == 24
