@@ -79,12 +79,17 @@ Workspace workspace_layout(const dsk_moe_desc& d) {
   L.h_lo = take(N * I * 2);
   L.hs_hi = take(T * Is * 2);
   L.hs_lo = take(T * Is * 2);
-  const bool mx = mx_decode(d);
+  const bool mx = mx_decode(d) && mx_own_space(d);
   L.hq = take(mx ? N * 3 * T * I : 0);
   L.hqs = take(mx ? N * 3 * T * (I / 32) : 0);
   L.y = take(N * H * 4);
   L.ys = take(T * H * 4);
   L.shared_x = take(mx && Is > 0 ? T * H * 2 : 0);
+  if (mx_decode(d) && !mx) {
+    L.hq = L.y;
+    L.hqs = L.y + align_up(N * 3 * T * I);
+    L.shared_x = L.ys;
+  }
   // the grouped FP4 gate/up's x planes: every batch the grouped path may take (below the
   // prefill GEMM), bf16 x
   if (prefill_mx_own_space(d)) {

@@ -661,7 +661,6 @@ __global__ __launch_bounds__(kUpW * 64) __attribute__((amdgpu_waves_per_eu(kF32 
 // [kUpItems][kMxMaxTokens] f32, then the activation planes xq [H/128][2T][128]
 // and their E8M0 bytes xe [H/128][2T][4].
 static_assert(kUpItems * 16 == 32, "a gate/up block's row tiles are one 32-row exponent group of h");
-static_assert(kStW * kStKB * 128 == kMxInter, "the MX down kernel's waves cover the intermediate");
 constexpr size_t kMxUpRedBytes = kUpItems * kUpKS * 2 * 64 * 4 * 4;
 constexpr size_t kMxUpXchOffset = kMxUpRedBytes;
 constexpr size_t kMxUpMaxOffset = kMxUpXchOffset + kUpW * 640;
@@ -708,15 +707,15 @@ __device__ __forceinline__ void put_x_mx(uint8_t* xq, uint8_t* xe, int T, int t,
 // up) * route weight (0 for a token not routed to the slot) leaves as three
 // FP8 planes per (slot, token) with one exponent per 32-row group -- the two
 // row tiles of a block -- in the B-operand layout of k_down_mx.
-template <int G>
+// kI: the intermediate (0: p.I).
+template <int G, int kI>
 __global__ __launch_bounds__(kUpW * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_up_mx(DecodeArgs p) {
   extern __shared__ __align__(16) uint16_t lds_up[];
   const int tid = threadIdx.x, lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
-  // the intermediate is kMxInter (the launcher's condition), so the block ->
-  // slot map needs no argument
-  constexpr int kTiles = kMxInter / 16;
-  constexpr int groups = (kTiles + kUpItems - 1) / kUpItems;
+  // (a fixed intermediate: the block -> slot map then needs no argument)
+  const int kTiles = (kI ? kI : p.I) / 16;
+  const int groups = (kTiles + kUpItems - 1) / kUpItems;
   const int rb = static_cast<int>(blockIdx.x);
   const int slot = rb / groups;
   // the argument words the first loads address, read in one go
@@ -1333,17 +1332,18 @@ constexpr int kMxSlots = 8;   // routed experts per round of k_down_mx (all of t
 // Wave-private LDS of k_down_mx, after the wave partial sums: the round's h
 // planes of the wave's two K blocks [kMxSlots][3T][256 B] (B-operand order)
 // and their E8M0 windows [kMxSlots][3T][8 B] (rounded up to 256 B).
-constexpr int kMxDnRedBytes = kStW * 64 * 4 * 4;   // wave partial sums
+constexpr int mx_dn_red_bytes(int waves) { return waves * 64 * 4 * 4; }   // wave partial sums
 constexpr int mx_dn_h_bytes(int T) { return kMxSlots * 3 * T * 256; }
 constexpr int mx_dn_s_bytes(int T) { return (kMxSlots * 3 * T * 8 + 255) / 256 * 256; }
 constexpr int mx_dn_wave_bytes(int T) { return mx_dn_h_bytes(T) + mx_dn_s_bytes(T); }
 static_assert((kMxSlots * 3) % 4 == 0, "h DMA instructions cover whole (slot, column) pairs");
 
 // Down + combine of the decode pipeline for FP4 experts and T (one or two)
-// tokens on scaled FP4 x FP8 MFMAs.  Block = 16 output rows, kStW waves;
-// wave w owns the K blocks [kStKB*w, kStKB*w + kStKB) of every active
+// tokens on scaled FP4 x FP8 MFMAs.  Block = 16 output rows, I / 256 waves (at
+// most NW); wave w owns the K blocks [kStKB*w, kStKB*w + kStKB) of every active
 // expert's w2 rows.  Everything of a round of kMxSlots experts is in flight
-// at once: first the wave's slices of the FP8 h planes k_up_mx wrote (B
+// at once (kS of them in the weights: a token's top-k, so that no slot is read
+// for nothing): first the wave's slices of the FP8 h planes k_up_mx wrote (B
 // column 3t + p: plane p of token t; zero planes for a token not routed to
 // the slot) and of their E8M0 windows, 16 contiguous bytes per lane, then
 // every expert's w2 codes and scale windows.  The h loads do not wait for
@@ -1360,11 +1360,13 @@ static_assert((kMxSlots * 3) % 4 == 0, "h DMA instructions cover whole (slot, co
 // the chains added in order, the waves in order, then a token's plane columns
 // ((p0 + p1) + p2) and the final add of the precomputed shared output and
 // cast.
-template <int T>
-__global__ __launch_bounds__(kStW * 64) void k_down_mx(DecodeArgs p) {
+template <int T, int NW, int kS>
+__global__ __launch_bounds__(NW * 64) void k_down_mx(DecodeArgs p) {
+  static_assert(kS <= kMxSlots, "the round's h planes cover its slots");
   extern __shared__ __align__(16) uint8_t lds_mx[];
   constexpr int C = 3 * T;
   float (*red)[64][4] = reinterpret_cast<float (*)[64][4]>(lds_mx);
+  const int waves = NW == kStW ? kStW : p.I / (kStKB * 128);
   const int tid = threadIdx.x, lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
   const int row0 = blockIdx.x * 16;
@@ -1373,7 +1375,7 @@ __global__ __launch_bounds__(kStW * 64) void k_down_mx(DecodeArgs p) {
   const int ms = min(p.E, T * p.k);   // slots of the h planes the gate/up grid covers
   const int I = p.I;
   const int kb0 = wave * kStKB;
-  uint8_t* hl = lds_mx + kMxDnRedBytes + wave * mx_dn_wave_bytes(T);   // [kMxSlots][C][256]
+  uint8_t* hl = lds_mx + mx_dn_red_bytes(waves) + wave * mx_dn_wave_bytes(T);   // [kMxSlots][C][256]
   uint8_t* sl = hl + mx_dn_h_bytes(T);                                  // [kMxSlots][C][8]
   // B column of this lane (past the last one, repeats of it; their results are not used)
   const int bc = min(r16, C - 1);
@@ -1406,7 +1408,8 @@ __global__ __launch_bounds__(kStW * 64) void k_down_mx(DecodeArgs p) {
     // 1. the round's h planes and E8M0 windows (slot indices past the gate/up
     // grid re-read its last slot; a slot past the count is not used):
     // lane l takes 16 bytes of (slot, column) pair 4q + l / 16, 4 bytes of pair 32q + l / 2
-    constexpr int NH = kMxSlots * C / 4, NS = mx_dn_s_bytes(T) / 256;
+    constexpr int kH = kS * C % 4 == 0 ? kS : kMxSlots;   // slots whose planes are loaded: whole instructions
+    constexpr int NH = kH * C / 4, NS = mx_dn_s_bytes(T) / 256;
     u32x4 hv[NH];
     uint32_t sv[NS];
 #pragma unroll
@@ -1428,10 +1431,10 @@ __global__ __launch_bounds__(kStW * 64) void k_down_mx(DecodeArgs p) {
                  "s"(Sr[7]));
     static_assert(kMxSlots == 8, "one operand per slot above");
     // 2. every expert's w2 codes and scale windows
-    u32x4 wc[kMxSlots][kStKB];
-    u32x2 ws[kMxSlots];
+    u32x4 wc[kS][kStKB];
+    u32x2 ws[kS];
 #pragma unroll
-    for (int i = 0; i < kMxSlots; ++i) {
+    for (int i = 0; i < kS; ++i) {
       const bool live = u0 + i < U;
       const uint8_t* W = live ? Wr[i] : W0;
       const uint8_t* S = live ? Sr[i] : S0;
@@ -1455,7 +1458,7 @@ __global__ __launch_bounds__(kStW * 64) void k_down_mx(DecodeArgs p) {
     }
     // 4. the experts in slot order as they land
 #pragma unroll
-    for (int i = 0; i < kMxSlots; ++i) {
+    for (int i = 0; i < kS; ++i) {
 #pragma unroll
       for (int j = 0; j < kStKB; ++j) {
         const uint8_t* src = hl + (i * C + bc) * 256 + j * 128 + g4 * 32;
@@ -1466,14 +1469,14 @@ __global__ __launch_bounds__(kStW * 64) void k_down_mx(DecodeArgs p) {
         acc[j] = mx_mfma(wc[i][j], wsb, lo, hi, hs, acc[j]);
       }
     }
-    u0 += kMxSlots;
+    u0 += kS;
   } while (u0 < U);
   static_assert(kStKB == 2, "two K-block chains");
   *reinterpret_cast<f32x4*>(&red[wave][lane][0]) = acc[0] + acc[1];
   __syncthreads();
   if (wave == 0) {
     f32x4 a = z;
-    for (int w = 0; w < kStW; ++w) a += *reinterpret_cast<const f32x4*>(&red[w][lane][0]);
+    for (int w = 0; w < waves; ++w) a += *reinterpret_cast<const f32x4*>(&red[w][lane][0]);
     // token t = r16 of this lane group: columns 3t .. 3t + 2
     const int t = min(r16, T - 1), gb = lane & 48;
     f32x4 ra;
@@ -1970,7 +1973,8 @@ hipError_t launch_experts_decode(const dsk_moe_desc& d, const Workspace& L, cons
         else if (!p.x_f32) launch_kernel(k_up_q3<false, false, true>, q3f_blocks, kQ3fW * 64, q3f_lds, s, p);
         else launch_kernel(k_up_q3<false, true, true>, q3f_blocks, kQ3fW * 64, q3f_lds, s, p);
       }
-      else if (mx) launch_kernel(k_up_mx<kUpBatch>, up_blocks, kUpW * 64, up_mx_lds_bytes(p), s, p);
+      else if (mx && d.inter == kMxInter) launch_kernel(k_up_mx<kUpBatch, kMxInter>, up_blocks, kUpW * 64, up_mx_lds_bytes(p), s, p);
+      else if (mx) launch_kernel(k_up_mx<kUpBatch, 0>, up_blocks, kUpW * 64, up_mx_lds_bytes(p), s, p);
       else if (q3 && q3win && !p.x_f32) launch_kernel(k_up_stream<kUpBatch, true, false, true>, up_blocks, kUpW * 64, up_lds, s, p);
       else if (q3 && q3win) launch_kernel(k_up_stream<kUpBatch, true, true, true>, up_blocks, kUpW * 64, up_lds, s, p);
       else if (q3 && !p.x_f32) launch_kernel(k_up_stream<kUpBatch, false, false, true>, up_blocks, kUpW * 64, up_lds, s, p);
@@ -1994,9 +1998,20 @@ hipError_t launch_experts_decode(const dsk_moe_desc& d, const Workspace& L, cons
     // the shared expert's down ran beside the routing (no shared intermediate here)
     if (d.inter_shared != 0) return hipErrorInvalidValue;
     for (int r = 0; r < repeat; ++r) {
-      const size_t lds = kMxDnRedBytes + kStW * mx_dn_wave_bytes(d.tokens);
-      if (d.tokens == 1) launch_kernel(k_down_mx<1>, static_cast<unsigned>(d.hidden / 16), kStW * 64, lds, s, p);
-      else launch_kernel(k_down_mx<2>, static_cast<unsigned>(d.hidden / 16), kStW * 64, lds, s, p);
+      const int waves = d.inter / (kStKB * 128);
+      const size_t lds = mx_dn_red_bytes(waves) + waves * mx_dn_wave_bytes(d.tokens);
+      const unsigned blocks = static_cast<unsigned>(d.hidden / 16);
+      // rounds of eight experts in the eight-wave form (a token's top-8 at once; nine
+      // waves have the registers of six), of six where six are all there are: at
+      // H 5120, I 2304, top-6 the down of one token in 13.0 us (50.3 without the
+      // scaled MFMAs), of two in 28.4 (93.2; 45.9 in rounds of eight, which spill)
+      if (d.inter == kMxInter && d.top_k > 6) {
+        if (d.tokens == 1) launch_kernel(k_down_mx<1, kStW, kMxSlots>, blocks, waves * 64, lds, s, p);
+        else launch_kernel(k_down_mx<2, kStW, kMxSlots>, blocks, waves * 64, lds, s, p);
+      } else {
+        if (d.tokens == 1) launch_kernel(k_down_mx<1, kMxMaxWaves, 6>, blocks, waves * 64, lds, s, p);
+        else launch_kernel(k_down_mx<2, kMxMaxWaves, 6>, blocks, waves * 64, lds, s, p);
+      }
       if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return hipSuccess;

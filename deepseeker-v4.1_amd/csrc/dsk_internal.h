@@ -218,15 +218,26 @@ inline bool decode_pipeline(const dsk_moe_desc& d) {
 // FP4 experts, bf16 activations and one or two tokens: the decode gate/up and
 // down kernels run the routed products as scaled FP4 x FP8 MFMAs, with the
 // activations split into FP8 planes (two for x, three for h) on the B side.
-// The down kernel's eight waves take two K blocks each of an intermediate of
-// kMxInter (the shared expert runs in the decode pipeline's first two kernels).
+// The down kernel's waves take two K blocks each of the intermediate, so I is a
+// multiple of 256 up to kMxMaxWaves of them; kMxInter, the eight-wave form, has
+// kernels of its own.  (The shared expert runs in the decode pipeline's first
+// two kernels.)  At H 5120, I 2304, top-6 of 384 one
+// token took 99.5 us without these kernels, 67.7 with; two 164 and 107 of kernels.
 constexpr int kMxMaxTokens = 2;
 constexpr int kMxInter = 2048;
+constexpr int kMxMaxWaves = 9;
+// h's planes and the shared output have workspace of their own at I = kMxInter;
+// for other I they lie in regions this pipeline does not use (y and ys), so that
+// workspaces keep their sizes.
+inline bool mx_own_space(const dsk_moe_desc& d) { return d.inter == kMxInter; }
 inline bool mx_decode(const dsk_moe_desc& d) {
   // gate/up LDS: 21.5 KB of partial sums and exchange tiles, 2.07 T H bytes of activation planes
   const size_t up_lds = 32768 + static_cast<size_t>(d.tokens) * d.hidden * 3;
+  // (the same shapes at one token and at two, whose rows are those of two calls of one)
+  const bool fits = mx_own_space(d) || int64_t{4} * d.hidden >= int64_t{3} * kMxMaxTokens * (d.inter + d.inter / 32) + 512;
   return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_BF16 && d.tokens <= kMxMaxTokens &&
-         decode_pipeline(d) && d.hidden % 128 == 0 && d.inter == kMxInter && up_lds <= kMaxLds;
+         decode_pipeline(d) && d.hidden % 128 == 0 && d.inter % 256 == 0 && d.inter <= 256 * kMxMaxWaves && fits &&
+         up_lds <= kMaxLds;
 }
 
 // ---------------------------------------------------------------- launchers

@@ -144,3 +144,17 @@ def test_mx_decode_two_tokens_equal_two_single_calls():
         assert union > 8
         assert torch.equal(both[0:1].view(torch.int16), one0.view(torch.int16))
         assert torch.equal(both[1:2].view(torch.int16), one1.view(torch.int16))
+
+
+@pytest.mark.parametrize("H,I,E,k", [(5120, 2304, 24, 6), (1024, 256, 16, 2), (2048, 768, 24, 8), (1536, 1024, 8, 8)])
+def test_mx_decode_intermediates(H, I, E, k):
+    """Intermediates other than 2048 (one to nine waves in the down kernel, rounds of six
+    experts and a part of one); two tokens give the rows of two one-token calls."""
+    print(f"mx decode H={H} I={I} E={E} k={k}", flush=True)
+    layer = gsynth.make_layer(hidden=H, n_experts=E, top_k=k, inter=I, inter_shared=256, seed=800 + I, device=DEV)
+    spec = L.LayerSpec(H=H, E=E, k=k, I=I, I_shared=256)
+    x = torch.randn((2, H), generator=torch.Generator(device=DEV).manual_seed(I), device=DEV).to(torch.bfloat16)
+    _check(layer, x, spec)
+    both = layer(x)
+    for t in range(2):
+        assert torch.equal(layer(x[t:t + 1]).view(torch.int16), both[t:t + 1].view(torch.int16))
