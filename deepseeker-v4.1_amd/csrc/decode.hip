@@ -1812,10 +1812,10 @@ __global__ __launch_bounds__(kDownW * 64) void k_down_decode(DecodeArgs p) {
 
 // The routing kernel of the decode pipeline's non-MX form (k_route_shared) also
 // writes x's FP8 planes for the wide FP4 gate/up that follows it (saves
-// that kernel's own launch): from kDecodeGroupedUpMin tokens, with shared tile
+// that kernel's own launch): from decode_grouped_up_min tokens, with shared tile
 // blocks to do it.
 bool route_writes_x_planes(const dsk_moe_desc& d) {
-  return d.tokens >= kDecodeGroupedUpMin && d.inter_shared > 0 && grouped_wide(d);
+  return d.tokens >= decode_grouped_up_min(d) && d.inter_shared > 0 && grouped_wide(d);
 }
 
 DecodeArgs decode_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a) {
@@ -1949,7 +1949,13 @@ hipError_t launch_experts_decode(const dsk_moe_desc& d, const Workspace& L, cons
   const unsigned q3f_blocks = static_cast<unsigned>(max_slots * ((p.up_tiles + kQ3fItems - 1) / kQ3fItems));
   const unsigned q3f2_blocks = static_cast<unsigned>(max_slots * ((p.up_tiles + 2 * kQ3fItems - 1) / (2 * kQ3fItems)));
   if ((e = stage_open(kStageUp)) != hipSuccess) return e;
-  if (d.tokens >= kDecodeGroupedUpMin && grouped_path(d)) {
+  if (d.tokens >= kDecodeGroupedDownMin && wide_pair(d)) {
+    if ((e = launch_split_x(d, L, a, s)) != hipSuccess) return e;
+    e = launch_experts_wide_pair(d, L, a, a.route.desc, a.route.xrow, a.route.wrow, s, repeat, true);
+    return e != hipSuccess ? e : launch_combine(d, L, a, s, repeat);
+  }
+  const bool gup = d.tokens >= decode_grouped_up_min(d) && grouped_path(d);
+  if (gup) {
     e = launch_grouped_up_routed(d, L, a, a.route.desc, a.route.xrow, a.route.wrow, s, repeat,
                                  route_writes_x_planes(d));
     if (e != hipSuccess) return e;
@@ -1989,8 +1995,8 @@ hipError_t launch_experts_decode(const dsk_moe_desc& d, const Workspace& L, cons
   if ((e = stage_open(kStageDown)) != hipSuccess) return e;
   if (d.tokens >= kDecodeGroupedDownMin && grouped_path(d)) {
     // routed and shared down per slot (one output row per dispatch row), then the combine
-    // h in FP8 planes where the grouped gate/up wrote it (from kDecodeGroupedUpMin tokens)
-    const bool hpl = d.tokens >= kDecodeGroupedUpMin && grouped_wide(d);
+    // h in FP8 planes where the wide gate/up wrote it
+    const bool hpl = gup && grouped_wide(d);
     if ((e = launch_grouped_down(d, L, a, a.route.desc, s, repeat, hpl)) != hipSuccess) return e;
     return launch_combine(d, L, a, s, repeat);
   }

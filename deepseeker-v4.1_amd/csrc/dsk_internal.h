@@ -167,7 +167,8 @@ constexpr int kDecodeMaxTokens = 16;
 // From this many tokens the decode pipeline runs the grouped down kernel and
 // the combine instead of its fused down + combine kernel.
 constexpr int kDecodeGroupedDownMin = 3;
-// ... and from this many its routed gate/up in the grouped kernel.
+// ... and from this many its routed gate/up in the grouped kernel (the wide
+// kernels: decode_grouped_up_min).
 constexpr int kDecodeGroupedUpMin = 8;
 constexpr int kDecodeMaxPositions = 64;
 constexpr size_t kMaxLds = 163840;          // LDS bytes one gfx950 workgroup may use
@@ -383,6 +384,17 @@ hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const Exper
                           const int32_t* xrow, const float* wrow, const WideCall& w, hipStream_t s);
 hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                             const WideCall& w, hipStream_t s);
+// The same walk for float32 x below the prefill sizes (bf16 hi / lo pairs: x in
+// Workspace::xb_hi / xb_lo, already split): gate/up and down with the shared
+// expert.  Opens the down stage (the gate/up's is open).
+bool wide_pair(const dsk_moe_desc& d);
+hipError_t launch_experts_wide_pair(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
+                                    const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
+                                    int repeat, bool hs_ready);
+// float32 x [T][H] as a bf16 hi / lo pair into Workspace::xb_hi / xb_lo.
+hipError_t launch_split_x(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s);
+// Tokens from which the decode pipeline's routed gate/up is the grouped path's.
+int decode_grouped_up_min(const dsk_moe_desc& d);
 // x [T][H] as FP8 planes in stage rows into Workspace::xp.
 hipError_t launch_pf_planes(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s);
 // The grouped path runs its FP4 slots on the wide kernels.

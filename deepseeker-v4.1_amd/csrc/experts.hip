@@ -613,6 +613,13 @@ hipError_t launch_combine(const dsk_moe_desc& d, const Workspace& L, const Exper
   return e;
 }
 
+hipError_t launch_split_x(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s) {
+  const int64_t n = static_cast<int64_t>(d.tokens) * d.hidden;
+  launch_kernel(k_split_x, static_cast<unsigned>((n + 255) / 256), 256, 0, s, static_cast<const float*>(a.x), n,
+                reinterpret_cast<uint16_t*>(a.ws + L.xb_hi), reinterpret_cast<uint16_t*>(a.ws + L.xb_lo));
+  return hipGetLastError();
+}
+
 hipError_t launch_experts(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                           hipStream_t s, int repeat) {
   const int T = d.tokens, H = d.hidden, I = d.inter, Is = d.inter_shared, k = d.top_k;
@@ -647,13 +654,13 @@ hipError_t launch_experts(const dsk_moe_desc& d, const Workspace& L, const Exper
   }
   if ((e = stage_open(kStageUp)) != hipSuccess) return e;
   if (x_f32) {
-    uint16_t* hi = reinterpret_cast<uint16_t*>(a.ws + L.xb_hi);
-    uint16_t* lo = reinterpret_cast<uint16_t*>(a.ws + L.xb_lo);
-    const int64_t n = static_cast<int64_t>(T) * H;
-    launch_kernel(k_split_x, static_cast<unsigned>((n + 255) / 256), 256, 0, s, static_cast<const float*>(a.x), n, hi, lo);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    xb_hi = hi;
-    xb_lo = lo;
+    if ((e = launch_split_x(d, L, a, s)) != hipSuccess) return e;
+    xb_hi = reinterpret_cast<const uint16_t*>(a.ws + L.xb_hi);
+    xb_lo = reinterpret_cast<const uint16_t*>(a.ws + L.xb_lo);
+    if (wide_pair(d)) {
+      if ((e = launch_experts_wide_pair(d, L, a, desc, xrow, wrow, s, repeat, false)) != hipSuccess) return e;
+      return a.rows_out ? hipSuccess : launch_combine(d, L, a, s, repeat);
+    }
   }
   const int nt = (T <= 16) ? 1 : (T <= 32 ? 2 : 4);
 

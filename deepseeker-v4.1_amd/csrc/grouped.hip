@@ -37,7 +37,8 @@ struct GroupedArgs {
   float limit;
   const SlotDesc* desc; const int32_t* active;   // active[0] = number of descriptors
   const int32_t* xrow; const float* wrow;        // per dispatch row: token, route weight
-  const uint16_t* x;                             // [T][H] bf16
+  const uint16_t* x;                             // [T][H] bf16 (float32 x: its hi part)
+  const uint16_t* x_lo;                          // float32 x: its lo part
   const uint16_t* ws1; const uint16_t* ws3;      // shared [Is][H] bf16
   const uint16_t* ws2;                           // shared [H][Is] bf16
   uint16_t* h_hi; uint16_t* h_lo;                // [T*k][I] by dispatch row
@@ -456,8 +457,10 @@ __device__ __forceinline__ void gs_walk(int nb, MM mm, LW ldw, LX ldx, SX stx, M
 // 2i + 1 take row tile 4b + i of w1 (gate) and of w3 (up), so that a wave
 // holds one role's accumulators and a ring of four weight batches; the up
 // wave hands its sums to the gate wave through LDS for SwiGLU.
+// kPair: x as a bf16 hi / lo pair (two planes staged and multiplied, as in the down).
+template <bool kPair>
 __device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, int first, int step, uint16_t* lds) {
-  constexpr int NB = 3;
+  constexpr int NB = kPair ? 2 : 3, NX = kPair ? 2 : 1;
   const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
   const int role = wave & 1, pair = wave >> 1;
@@ -471,18 +474,28 @@ __device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, int 
     const int ncol = min(kGsCols, p.T - g0);
     const int nct = (ncol + 15) / 16;
     RawBF16 w[NB];
-    u32x4 xv[NB][2];
+    u32x4 xv[NB][NX][2];
     f32x4 acc[kGsCT];
 #pragma unroll
     for (int c = 0; c < kGsCT; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto mm = [&](int i, int buf) {
 #pragma unroll
       for (int c = 0; c < kGsCT; ++c)
-        if (c < nct) mma_block(w[i], lds + buf * kGsPlane + (c * 16 + r16) * kGsStride, g4 * 32, true, acc[c]);
+        if (c < nct) {
+          const uint16_t* x = lds + buf * NX * kGsPlane + (c * 16 + r16) * kGsStride;
+          mma_block(w[i], x, g4 * 32, true, acc[c]);
+          if constexpr (kPair) mma_block(w[i], x + kGsPlane, g4 * 32, true, acc[c]);
+        }
     };
     auto ldw = [&](int i, int kb) { load_raw_nc(w[i], W, row, K, kb * 128 + g4 * 32); };
-    auto ldx = [&](int slot, int kb) { gs_load(xv[slot], p.x, K, g0, ncol, kb); };
-    auto stx = [&](int slot, int buf) { gs_store(xv[slot], lds + buf * kGsPlane); };
+    auto ldx = [&](int slot, int kb) {
+      gs_load(xv[slot][0], p.x, K, g0, ncol, kb);
+      if constexpr (kPair) gs_load(xv[slot][NX - 1], p.x_lo, K, g0, ncol, kb);
+    };
+    auto stx = [&](int slot, int buf) {
+#pragma unroll
+      for (int i = 0; i < NX; ++i) gs_store(xv[slot][i], lds + (buf * NX + i) * kGsPlane);
+    };
     gs_walk<NB>(nb, mm, ldw, ldx, stx, [] {});   // ends with a barrier: the buffers are free
     if (role) {
 #pragma unroll
@@ -847,7 +860,7 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.up_shared) {
-    up_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    up_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
     return;
   }
   const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
@@ -886,6 +899,168 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   if (n > r) down_wide_tile<1, kWdNB1, NPH>(p, slot, grp, n - r, base + r, lds);
 }
 
+// ---------------------------------------------------------------- wide FP4 slots, float32 x
+// The same walk for activations as bf16 hi / lo pairs (float32 x, whose products
+// keep 2^-17 and float32 sums: the scaled MFMA would sum to 2^-14): per 128-code
+// block, row tile and plane four v_mfma_f32_16x16x32_bf16, the codes converted
+// to bf16 with their scale once for both planes; 16 dispatch rows a pass.  Bound
+// by the weight stream.  H 4096, top-8 of 256, 20 tokens: gate/up
+// 490 -> 177 us, down 230 -> 100 against tiles of 16 rows by 16 tokens that read
+// their activations from memory per wave; 60 tokens 1011 -> 302 and 460 -> 168;
+// H 5120, top-6 of 384, 30 tokens 1080 -> 386 and 457 -> 191.  Three steps in
+// flight spill (209 and 119 at 20 tokens).
+constexpr int kWpNB = 2;                              // steps in flight
+constexpr int kWpRow = 2 * kWdStep * 2 + 16;          // LDS bytes of a row's step: hi, lo, padding
+constexpr size_t wp_lds_bytes(int K) { return size_t{2} * 16 * kWpRow + size_t(32 * kWdWaves) * wd_scale_row(K); }
+
+template <typename Src>
+__device__ __forceinline__ void wide_mul_pair(const uint8_t* const (&W)[2], const uint8_t* const (&S)[2],
+                                              const uint32_t (&co)[2], const uint32_t (&so)[2], const uint16_t* hi,
+                                              const uint16_t* lo, int K, int n, Src src, uint8_t* lds,
+                                              f32x4 (&acc)[2]) {
+  constexpr int kThreads = kWdWaves * 64, kBuf = 16 * kWpRow, NB = kWpNB;
+  constexpr int Q = 16 * 64 / kThreads;               // 16-byte pieces a thread stages (64 a row)
+  static_assert(Q == 2, "piece i of a thread: plane i");
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (see wide_mul)
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int es = wd_scale_row(K);
+  uint8_t* ws = lds + 2 * kBuf + wave * 32 * es;
+  // this thread's pieces: row tid / 32, piece tid % 32 of each plane
+  const uint32_t xs = static_cast<uint32_t>(src(min(tid >> 5, n - 1))) * static_cast<uint32_t>(K) + 8 * (tid & 31);
+  const int xo = (tid >> 5) * kWpRow + 16 * (tid & 31);
+  const int inv = (65536 + K / 256 - 1) / (K / 256);
+  auto wsrc = [&](int r) { return (r < 16 ? S[0] + so[0] : S[1] + so[1]) + (r & 15) * (K / 32); };
+  WideScales<kWdScales> wsc;
+  wsc.load(32, K, inv, lane, 64, wsrc);
+  u32x4 w[NB][2][2];   // [slot][row tile][K block]
+  u32x4 xv[NB][Q];
+  acc[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+  acc[1] = acc[0];
+  const uint8_t* wsl = ws + r16 * es + g4;
+  auto mm = [&](int i, int buf) {
+    // a step's products in a sum of their own: chains as short as the K splits of
+    // the general path's kernels (one chain over all of K was 1.5 % less exact)
+    f32x4 st[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint8_t* xb = lds + buf * kBuf + r16 * kWpRow + b * 256 + g4 * 64;
+      const float s0 = e8m0_to_f32(wsl[4 * b]), s1 = e8m0_to_f32(wsl[16 * es + 4 * b]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        asm volatile("" : "+v"(st[0]), "+v"(st[1])::"memory");   // (see wide_mul)
+        const bf16x8 xh = as_bf16x8(*reinterpret_cast<const u32x4*>(xb + 16 * j));
+        const bf16x8 xl = as_bf16x8(*reinterpret_cast<const u32x4*>(xb + 2 * kWdStep + 16 * j));
+        const bf16x8 a0 = fp4_word_to_bf16x8(w[i][0][b][j], s0), a1 = fp4_word_to_bf16x8(w[i][1][b][j], s1);
+        st[0] = mfma16(a0, xh, st[0]);
+        st[1] = mfma16(a1, xh, st[1]);
+        st[0] = mfma16(a0, xl, st[0]);
+        st[1] = mfma16(a1, xl, st[1]);
+      }
+    }
+    acc[0] += st[0];
+    acc[1] += st[1];
+    asm volatile("" : "+v"(acc[0]), "+v"(acc[1])::"memory");
+    wsl += 8;
+  };
+  auto ldw = [&](int i, int kb) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      w[i][a][0] = ldg16(W[a] + kb * (kWdStep / 2) + co[a]);
+      w[i][a][1] = ldg16(W[a] + kb * (kWdStep / 2) + co[a] + 64);
+    }
+  };
+  auto ldx = [&](int i, int kb) {
+    xv[i][0] = ldg16(hi + kb * kWdStep + xs);
+    xv[i][1] = ldg16(lo + kb * kWdStep + xs);
+  };
+  auto stx = [&](int i, int buf) {
+    *reinterpret_cast<u32x4*>(lds + buf * kBuf + xo) = xv[i][0];
+    *reinterpret_cast<u32x4*>(lds + buf * kBuf + xo + 2 * kWdStep) = xv[i][1];
+  };
+  gs_walk<NB>(K / kWdStep, mm, ldw, ldx, stx, [&] {
+    asm volatile("" ::: "memory");
+    wsc.store(ws, 32, K, inv, lane, 64, wsrc);
+  });
+}
+
+// Blocks as in k_up_wide; h as the bf16 hi / lo pair by dispatch row.
+__global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_up_wide_pair(GroupedArgs p) {
+  extern __shared__ __align__(16) uint16_t lds_g[];
+  uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
+  const int b = static_cast<int>(blockIdx.x);
+  if (b < p.up_shared) {
+    up_shared_wide<true>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    return;
+  }
+  const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
+  if (slot >= p.active[0]) return;
+  const SlotDesc* d = p.desc + slot;
+  const int n = d->n_tok, base = d->tok_base;
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int rt = grp * kWdWaves + wave, K = p.H;
+  const bool rok = rt < p.I / 16;
+  const uint8_t* const W[2] = {static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 0)),
+                               static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3))};
+  const uint8_t* const S[2] = {static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 1)),
+                               static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 4))};
+  const uint32_t row0 = rok ? static_cast<uint32_t>(rt * 16) : 0u;
+  const uint32_t c0 = (row0 + r16) * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
+  const uint32_t s0 = row0 * static_cast<uint32_t>(K / 32);
+  const uint32_t co[2] = {c0, c0}, so[2] = {s0, s0};
+  for (int r = 0; r < n; r += 16) {
+    const int m = min(n - r, 16);
+    f32x4 acc[2];
+    wide_mul_pair(W, S, co, so, p.x, p.x_lo, K, m, [&](int i) { return p.xrow[base + r + i]; }, lds, acc);
+    if (rok && r16 < m) {
+      const int64_t row = base + r + r16;
+      const float wr = p.wrow[row];
+      uint16_t hh[4], hl[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) split_bf16(silu_clamped(acc[0][q], acc[1][q], p.limit) * wr, hh[q], hl[q]);
+      const int64_t off = row * p.I + rt * 16 + 4 * g4;
+      *reinterpret_cast<uint2*>(p.h_hi + off) = uint2{hh[0] | (uint32_t(hh[1]) << 16), hh[2] | (uint32_t(hh[3]) << 16)};
+      *reinterpret_cast<uint2*>(p.h_lo + off) = uint2{hl[0] | (uint32_t(hl[1]) << 16), hl[2] | (uint32_t(hl[3]) << 16)};
+    }
+  }
+}
+
+__global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_down_wide_pair(GroupedArgs p) {
+  extern __shared__ __align__(16) uint16_t lds_g[];
+  uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
+  const int b = static_cast<int>(blockIdx.x);
+  if (b < p.dn_shared) {
+    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    return;
+  }
+  const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
+  if (slot >= p.active[0]) return;
+  const SlotDesc* d = p.desc + slot;
+  const int n = d->n_tok, base = d->tok_base;
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int rt = (grp * kWdWaves + wave) * 2, K = p.I;
+  const uint8_t* W2 = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 6));
+  const uint8_t* S2 = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 7));
+  const uint8_t* const W[2] = {W2, W2};
+  const uint8_t* const S[2] = {S2, S2};
+  const uint32_t c0 = static_cast<uint32_t>(rt * 16 + r16) * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
+  const uint32_t s0 = static_cast<uint32_t>(rt * 16) * static_cast<uint32_t>(K / 32);
+  const uint32_t co[2] = {c0, c0 + static_cast<uint32_t>(8 * K)}, so[2] = {s0, s0 + static_cast<uint32_t>(K / 2)};
+  for (int r = 0; r < n; r += 16) {
+    const int m = min(n - r, 16);
+    f32x4 acc[2];
+    wide_mul_pair(W, S, co, so, p.h_hi, p.h_lo, K, m, [&](int i) { return base + r + i; }, lds, acc);
+    if (r16 < m) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+        *reinterpret_cast<f32x4*>(p.y + static_cast<int64_t>(base + r + r16) * p.H + (rt + a) * 16 + 4 * g4) = acc[a];
+    }
+  }
+}
+
 // Blocks [0, up_shared): the shared expert (bf16 w1/w3, all T tokens); the
 // others: up_groups blocks per slot.
 template <typename Raw>
@@ -895,7 +1070,7 @@ __global__ __launch_bounds__(kGW * 64) __attribute__((amdgpu_waves_per_eu(4))) v
   const int item = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kGKS;
   if (b < p.up_shared) {
     if (p.T > kGNC) {
-      up_shared_wide(p, b, 0, kGsCols, lds_g);
+      up_shared_wide<false>(p, b, 0, kGsCols, lds_g);
       return;
     }
     const int rt = b * kGI + item;
@@ -1304,6 +1479,11 @@ size_t wide_lds(int rows, int planes, int K) {
   return rows <= 16 ? wd_lds_bytes(1, planes, K) : wd_lds_bytes(kWdMaxCT, planes, K);
 }
 
+// The wide kernels from four tokens (gate/up + down: H 4096, top-8 of 256 at three
+// tokens 88 us against 81 on the streaming kernels, at five 114 and 118, H 5120,
+// top-6 of 384 at six 155 and 225), the others of the grouped path from eight.
+int decode_grouped_up_min(const dsk_moe_desc& d) { return grouped_wide(d) ? 4 : kDecodeGroupedUpMin; }
+
 bool grouped_wide(const dsk_moe_desc& d) { return wide_shapes(d) && grouped_path(d) && !prefill_gemm(d); }
 
 bool wide_shapes(const dsk_moe_desc& d) {
@@ -1356,6 +1536,35 @@ hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const Exp
   if (w.h_planes == 2) launch_kernel(k_down_wide<2>, blocks, kWdWaves * 64, lds, s, p);
   else launch_kernel(k_down_wide<3>, blocks, kWdWaves * 64, lds, s, p);
   return hipGetLastError();
+}
+
+bool wide_pair(const dsk_moe_desc& d) {
+  return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_F32 && d.tokens < kPrefillMinTokens &&
+         d.hidden % kWdStep == 0 && d.inter % kWdStep == 0 && d.inter_shared % 128 == 0 && d.hidden < 8192 &&
+         d.inter < 8192 && wp_lds_bytes(d.hidden) <= kMaxLds && wp_lds_bytes(d.inter) <= kMaxLds;
+}
+
+hipError_t launch_experts_wide_pair(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
+                                    const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
+                                    int repeat, bool hs_ready) {
+  GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, WideCall{3, d.tokens, nullptr, 0, d.inter_shared > 0});
+  if (hs_ready) p.up_shared = 0;
+  p.x = reinterpret_cast<const uint16_t*>(a.ws + L.xb_hi);
+  p.x_lo = reinterpret_cast<const uint16_t*>(a.ws + L.xb_lo);
+  const size_t sh = d.inter_shared > 0 ? gs_down_lds_bytes() : 0;
+  const size_t ul = wp_lds_bytes(d.hidden) > sh ? wp_lds_bytes(d.hidden) : sh;
+  const size_t dl = wp_lds_bytes(d.inter) > sh ? wp_lds_bytes(d.inter) : sh;
+  hipError_t e;
+  for (int r = 0; r < repeat; ++r) {
+    launch_kernel(k_up_wide_pair, static_cast<unsigned>(p.up_shared + max_slots(d) * p.up_groups), kWdWaves * 64, ul, s, p);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if ((e = stage_open(kStageDown)) != hipSuccess) return e;
+  for (int r = 0; r < repeat; ++r) {
+    launch_kernel(k_down_wide_pair, static_cast<unsigned>(p.dn_shared + max_slots(d) * p.dn_groups), kWdWaves * 64, dl, s, p);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,

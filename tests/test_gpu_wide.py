@@ -20,9 +20,11 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-def _check(spec, T, hot, seed, label, shared=True):
+def _check(spec, T, hot, seed, label, shared=True, f32=False):
     print(f"wide {label} T={T} hot={hot}", flush=True)
     d = synth.make_layer(spec, seed, T)
+    if f32:
+        d["x"] = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(seed))
     if hot:
         d["gate_b"] = d["gate_b"].clone()
         d["gate_b"][:hot] += 10.0          # every token goes to experts 0 .. hot - 1
@@ -33,9 +35,11 @@ def _check(spec, T, hot, seed, label, shared=True):
     x = d["x"].to(DEV)
     out = layer(x, idx=idx)
     again = layer(x)
-    assert torch.equal(out.view(torch.int16), again.view(torch.int16))
+    assert torch.equal(out, again)
     np.testing.assert_array_equal(idx.cpu().numpy(), r["idx"])
     c, rel = assert_layer_close(out.cpu().float(), r["y_ref"])
+    if f32:        # hi / lo pairs hold 2^-17, h and x each: well inside 1e-4 of the largest output
+        assert rel < 1e-4
     print(f"cos={c:.9f} rel={rel:.2e} rows {sorted(set(int(v) for v in r['counts']))}", flush=True)
     return r
 
@@ -43,6 +47,20 @@ def _check(spec, T, hot, seed, label, shared=True):
 @pytest.mark.parametrize("T,hot", [(9, 0), (15, 4), (16, 4), (17, 4), (31, 4), (32, 4), (33, 4), (127, 4)])
 def test_wide_rows_of_a_slot(T, hot):
     _check(L.LayerSpec(H=1024, E=24, k=4, I=512, I_shared=256), T, hot, 310 + T, "rows")
+
+
+@pytest.mark.parametrize("T,hot,H,I", [(3, 0, 1024, 512), (9, 0, 512, 256), (17, 4, 1024, 768), (70, 0, 5120, 256),
+                                       (127, 4, 1024, 512)])
+def test_wide_float32_pairs(T, hot, H, I):
+    """float32 x: passes of 16 rows and a part of one, the shared expert over one and two
+    groups of 64 tokens, the decode pipeline's form (3 tokens)."""
+    _check(L.LayerSpec(H=H, E=16, k=4, I=I, I_shared=256), T, hot, 370 + T, f"f32 H {H} I {I}", f32=True)
+
+
+@pytest.mark.parametrize("T", [4, 7])
+def test_wide_in_the_decode_pipeline(T):
+    _check(L.LayerSpec(H=1024, E=32, k=4, I=512, I_shared=256), T, 0, 390 + T, "decode")
+    _check(L.LayerSpec(H=1024, E=32, k=4, I=512, I_shared=256), T, 0, 390 + T, "decode, no shared", shared=False)
 
 
 @pytest.mark.parametrize("H,I,Is", [(1024, 256, 128), (5120, 768, 384), (2048, 2304, 0)])
