@@ -391,7 +391,7 @@ int dsk::forward_layer(const dsk_moe_desc* d, const void* x, const void* gate_w,
   // planes for FP4 experts, the factored q3 form for q3 experts; prefill: its MX planes)
   if (!decode && d->tokens > kFusedMaxTokens && !rn && d->x_dtype == DSK_DTYPE_BF16) {
     const bool planes = prefill_mx(*d) || grouped_wide(*d);
-    if (planes || (!prefill_gemm(*d) && grouped_path(*d) && grouped_x_q3(*d))) {
+    if (planes || (!prefill_gemm(*d) && grouped_path(*d) && grouped_x_q3(*d) && !grouped_wide_q3(*d))) {
       ra.xp = reinterpret_cast<uint8_t*>(ws + L.xp);
       ra.xform = planes ? kXPlanes : kXGroupedQ3;
       a.x_planes_ready = 1;

@@ -1996,7 +1996,7 @@ hipError_t launch_experts_decode(const dsk_moe_desc& d, const Workspace& L, cons
   if (d.tokens >= kDecodeGroupedDownMin && grouped_path(d)) {
     // routed and shared down per slot (one output row per dispatch row), then the combine
     // h in FP8 planes where the wide gate/up wrote it
-    const bool hpl = gup && grouped_wide(d);
+    const bool hpl = gup && (grouped_wide(d) || grouped_wide_q3(d));
     if ((e = launch_grouped_down(d, L, a, a.route.desc, s, repeat, hpl)) != hipSuccess) return e;
     return launch_combine(d, L, a, s, repeat);
   }

@@ -397,8 +397,12 @@ hipError_t launch_split_x(const dsk_moe_desc& d, const Workspace& L, const Exper
 int decode_grouped_up_min(const dsk_moe_desc& d);
 // x [T][H] as FP8 planes in stage rows into Workspace::xp.
 hipError_t launch_pf_planes(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s);
-// The grouped path runs its FP4 slots on the wide kernels.
+// q3 experts' wide kernels take these shapes (launch_wide_up / _down dispatch on
+// the format; h as the bf16 hi / lo pair, rows float32).
+bool wide_q3(const dsk_moe_desc& d);
+// The grouped path runs its FP4 / q3 slots on the wide kernels.
 bool grouped_wide(const dsk_moe_desc& d);
+bool grouped_wide_q3(const dsk_moe_desc& d);
 // Prefill layers: slots of up to this many dispatch rows run on the wide
 // kernels instead of the GEMM tiles (0: none), and whether the shared expert does.
 int prefill_narrow_rows(const dsk_moe_desc& d);

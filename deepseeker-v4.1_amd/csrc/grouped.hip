@@ -1061,6 +1061,252 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   }
 }
 
+// ---------------------------------------------------------------- wide q3 slots
+// The walk for q3 experts in the factored form (x . W = s sum(q x) + b sum(x) per
+// 64-group), 512 of K a step, one row tile a wave: the A operand is the
+// activations (row 2t + h: dispatch row t of eight on a block's h-th 64-group;
+// the other half's lanes read a row of zeros), the B operand the codes as 128 +
+// q, and a product with ones gives the group sums where the kernels of
+// up_block_q3f read prepared ones, so x and h are staged as they lie (h as its
+// hi / lo pair).  All codes are shifted down to bits 0..2 for that: six shifts
+// a block more than the 128 + 8q form.  Up to 16 dispatch rows a pass.
+//
+// Bound by the weight stream and, near it, by the masking.  Gate/up and down at H 4096, top-8 of 256
+// (against blocks of eight K ranges and eight rows a pass): 16 tokens 226 -> 220 and
+// 121 -> 124 us, 64 tokens 416 -> 371 and 212 -> 210, 100 tokens 507 -> 426 and 262
+// -> 256. At H 5120, I 2304, top-6 of 384, where the other kernels dequantise every
+// weight: 24 tokens 696 -> 361 and 369 -> 199, 6 tokens 367 -> 108 and 121 -> 72.
+constexpr int kWqStep = 512;                                // K of a step: a superblock
+constexpr int kWqNB = 2;                                    // steps in flight
+constexpr int kWqUpTiles = 4;                               // gate/up: row tiles of a block (w1 and w3 in waves 2i, 2i + 1)
+constexpr int wq_row(int NPL) { return NPL * kWqStep * 2 + 16; }
+constexpr int wq_buf(int NPL) { return 17 * wq_row(NPL); }  // 16 rows and one of zeros
+constexpr size_t wq_lds_bytes(int NPL) { return size_t{2} * wq_buf(NPL); }
+
+// Pair P of a lane's 32 codes as two bf16 128 + q (see q3m_pair).
+template <int P>
+__device__ __forceinline__ uint32_t q3_pair128(const uint32_t (&w)[3], const Q3Masks& k) {
+  if constexpr (P < 15) return ((w[P / 5] >> (3 * (P % 5))) & k.m7) | k.magic;
+  else return q3m_pair<15>(w, k);
+}
+
+template <int M>
+__device__ __forceinline__ bf16x8 q3_operand128(const uint32_t (&w)[3], const Q3Masks& k) {
+  return as_bf16x8(u32x4{q3_pair128<4 * M>(w, k), q3_pair128<4 * M + 1>(w, k), q3_pair128<4 * M + 2>(w, k),
+                         q3_pair128<4 * M + 3>(w, k)});
+}
+
+// acc[s][i]: dispatch row 8 s + 2 g4 + i of the n rows (row r from source row
+// src(r) of the NPL planes) by this lane's weight row (codes W + co, scales and
+// biases S / B + so), K in whole 128-code blocks.
+template <int NS, int NPL, typename Src>
+__device__ __forceinline__ void wide_mul_q3(const uint8_t* W, const uint8_t* S, const uint8_t* B, uint32_t co,
+                                            uint32_t so, const uint16_t* hi, const uint16_t* lo, int K, int n, Src src,
+                                            uint8_t* lds, float (&acc)[NS][2]) {
+  constexpr int kRow = wq_row(NPL), kBuf = wq_buf(NPL), NB = kWqNB;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (see wide_mul)
+  const int lane = tid & 63;
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int nsb = K / kWqStep, tb = (K / 128) & 3;   // superblocks, blocks after them
+  // this thread's pieces: rows tid / 64 + 8 i, piece tid % 64 of each plane
+  uint32_t xs[NS];
+#pragma unroll
+  for (int i = 0; i < NS; ++i)
+    xs[i] = static_cast<uint32_t>(src(min((tid >> 6) + 8 * i, n - 1))) * static_cast<uint32_t>(K);
+  const int xp = tid & 63, xo = (tid >> 6) * kRow + 16 * xp;
+  if (tid < kRow / 16) {   // the zero rows
+    *reinterpret_cast<u32x4*>(lds + 16 * kRow + 16 * tid) = u32x4{0u, 0u, 0u, 0u};
+    *reinterpret_cast<u32x4*>(lds + kBuf + 16 * kRow + 16 * tid) = u32x4{0u, 0u, 0u, 0u};
+  }
+  struct Sb { uint32_t c[4][3]; u32x4 s, b; } w[NB];
+  u32x4 xv[NB][NS][NPL];
+#pragma unroll
+  for (int s2 = 0; s2 < NS; ++s2) acc[s2][0] = acc[s2][1] = 0.0f;
+  const Q3Masks km = q3_masks();
+  const bf16x8 ones = as_bf16x8(u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+  const bool av = (r16 & 1) == (g4 >> 1);
+  // one block: codes c, scale / bias words, activations at byte offset `at` of a row
+  auto block = [&](const uint32_t (&c)[3], uint32_t sw, uint32_t bw, const uint8_t* xb, int at) {
+#pragma unroll
+    for (int s2 = 0; s2 < NS; ++s2) {
+      asm volatile("" : "+v"(acc[s2][0]), "+v"(acc[s2][1])::"memory");   // (see wide_mul)
+      const uint8_t* x = xb + (av ? 8 * s2 + (r16 >> 1) : 16) * kRow + at + 64 * g4;
+      f32x4 d = {0.f, 0.f, 0.f, 0.f}, sum = d;
+#define DSK_WQ3_STEP(M)                                                                             \
+      {                                                                                             \
+        const bf16x8 q = q3_operand128<M>(c, km);                                                   \
+        _Pragma("unroll") for (int pl = 0; pl < NPL; ++pl) {                                        \
+          const bf16x8 xa = as_bf16x8(*reinterpret_cast<const u32x4*>(x + pl * 2 * kWqStep + 16 * M)); \
+          d = mfma16(xa, q, d);                                                                     \
+          sum = mfma16(xa, ones, sum);                                                              \
+        }                                                                                           \
+      }
+      DSK_WQ3_STEP(0) DSK_WQ3_STEP(1) DSK_WQ3_STEP(2) DSK_WQ3_STEP(3)
+#undef DSK_WQ3_STEP
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        acc[s2][i] = fmaf(f16_half<0>(sw), fmaf(-128.0f, sum[2 * i], d[2 * i]), acc[s2][i]);
+        acc[s2][i] = fmaf(f16_half<0>(bw), sum[2 * i], acc[s2][i]);
+        acc[s2][i] = fmaf(f16_half<1>(sw), fmaf(-128.0f, sum[2 * i + 1], d[2 * i + 1]), acc[s2][i]);
+        acc[s2][i] = fmaf(f16_half<1>(bw), sum[2 * i + 1], acc[s2][i]);
+      }
+    }
+  };
+  auto mm = [&](int i, int buf) {
+    const uint32_t sw[4] = {w[i].s.x, w[i].s.y, w[i].s.z, w[i].s.w}, bw[4] = {w[i].b.x, w[i].b.y, w[i].b.z, w[i].b.w};
+#pragma unroll
+    for (int b = 0; b < 4; ++b) block(w[i].c[b], sw[b], bw[b], lds + buf * kBuf, b * 256);
+#pragma unroll
+    for (int s2 = 0; s2 < NS; ++s2) asm volatile("" : "+v"(acc[s2][0]), "+v"(acc[s2][1])::"memory");
+  };
+  auto ldw = [&](int i, int sb) {
+    const auto c = gptr<u32x4>(W + sb * 192 + co + 48 * g4);
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      const u32x4 a = c[v];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[i].c[(4 * v + j) / 3][(4 * v + j) % 3] = a[j];
+    }
+    w[i].s = ldg16(S + sb * 16 + so);
+    w[i].b = ldg16(B + sb * 16 + so);
+  };
+  auto ldx_at = [&](int i, int k0, int piece) {
+#pragma unroll
+    for (int r = 0; r < NS; ++r) {
+      xv[i][r][0] = ldg16(hi + k0 + 8 * piece + xs[r]);
+      if constexpr (NPL == 2) xv[i][r][NPL - 1] = ldg16(lo + k0 + 8 * piece + xs[r]);
+    }
+  };
+  auto stx = [&](int i, int buf) {
+#pragma unroll
+    for (int r = 0; r < NS; ++r)
+#pragma unroll
+      for (int pl = 0; pl < NPL; ++pl)
+        *reinterpret_cast<u32x4*>(lds + buf * kBuf + 8 * r * kRow + xo + pl * 2 * kWqStep) = xv[i][r][pl];
+  };
+  gs_walk<NB>(nsb, mm, ldw, [&](int i, int sb) { ldx_at(i, sb * kWqStep, xp); }, stx, [] {});
+  if (tb) {
+    // the blocks after the last superblock (plain 48-byte blocks)
+    uint32_t tw[3][3], ts[3], tbi[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int kb = min(nsb * 4 + i, K / 128 - 1);
+      const auto c = gptr<uint32_t>(W + kb * 48 + co + 12 * g4);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) tw[i][j] = c[j];
+      ts[i] = ldg<uint32_t>(S + kb * 4 + so);
+      tbi[i] = ldg<uint32_t>(B + kb * 4 + so);
+    }
+    // (pieces past the blocks repeat the last one; nothing reads them)
+    ldx_at(0, nsb * kWqStep, min(xp, tb * 16 - 1));
+    stx(0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i < tb) block(tw[i], ts[i], tbi[i], lds, i * 256);
+    __syncthreads();
+  }
+}
+
+// Gate/up of one q3 slot, NS sets of eight dispatch rows: row tile 4 grp + wave / 2
+// of w1 (even waves) and w3 (odd); h as the hi / lo pair by dispatch row.
+template <int NS>
+__device__ __forceinline__ void up_wide_q3(const GroupedArgs& p, int slot, int grp, int n, int base, uint8_t* lds) {
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int role = wave & 1, pair = wave >> 1, rt = grp * kWqUpTiles + pair, K = p.H;
+  const bool rok = rt < p.I / 16;
+  const uint32_t row = rok ? static_cast<uint32_t>(rt * 16 + r16) : 0u;
+  const uint8_t* W = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3 * role));
+  const uint8_t* S = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3 * role + 1));
+  const uint8_t* B = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3 * role + 2));
+  float acc[NS][2];
+  wide_mul_q3<NS, 1>(W, S, B, row * static_cast<uint32_t>(K / 8 * 3), row * static_cast<uint32_t>(K / 32), p.x, p.x, K, n,
+                     [&](int r) { return p.xrow[base + r]; }, lds, acc);
+  float (*xch)[NS][2][64] = reinterpret_cast<float (*)[NS][2][64]>(lds);   // [pair]: the up sums
+  if (role) {
+#pragma unroll
+    for (int s2 = 0; s2 < NS; ++s2)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) xch[pair][s2][i][lane] = acc[s2][i];
+  }
+  __syncthreads();
+  if (!role && rok) {
+#pragma unroll
+    for (int s2 = 0; s2 < NS; ++s2)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int t = 8 * s2 + 2 * g4 + i;
+        if (t < n) {
+          const int64_t r = base + t;
+          uint16_t hh, hl;
+          split_bf16(silu_clamped(acc[s2][i], xch[pair][s2][i][lane], p.limit) * p.wrow[r], hh, hl);
+          p.h_hi[r * p.I + rt * 16 + r16] = hh;
+          p.h_lo[r * p.I + rt * 16 + r16] = hl;
+        }
+      }
+  }
+  __syncthreads();   // the next rows reuse the LDS
+}
+
+template <int NS>
+__device__ __forceinline__ void down_wide_q3(const GroupedArgs& p, int slot, int grp, int n, int base, uint8_t* lds) {
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int rt = grp * kWdWaves + wave, K = p.I;
+  const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
+  const uint8_t* W = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 6));
+  const uint8_t* S = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 7));
+  const uint8_t* B = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 8));
+  float acc[NS][2];
+  wide_mul_q3<NS, 2>(W, S, B, row * static_cast<uint32_t>(K / 8 * 3), row * static_cast<uint32_t>(K / 32), p.h_hi, p.h_lo,
+                     K, n, [&](int r) { return base + r; }, lds, acc);
+#pragma unroll
+  for (int s2 = 0; s2 < NS; ++s2)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int t = 8 * s2 + 2 * g4 + i;
+      if (t < n) p.y[static_cast<int64_t>(base + t) * p.H + rt * 16 + r16] = acc[s2][i];
+    }
+}
+
+__global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_up_wide_q3(GroupedArgs p) {
+  extern __shared__ __align__(16) uint16_t lds_g[];
+  uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
+  const int b = static_cast<int>(blockIdx.x);
+  if (b < p.up_shared) {
+    up_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    return;
+  }
+  const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
+  if (slot >= p.active[0]) return;
+  const SlotDesc* d = p.desc + slot;
+  const int n = d->n_tok, base = d->tok_base;
+  if (n > p.max_rows) return;
+  int r = 0;
+  for (; n - r > 8; r += 16) up_wide_q3<2>(p, slot, grp, min(n - r, 16), base + r, lds);
+  if (n > r) up_wide_q3<1>(p, slot, grp, n - r, base + r, lds);
+}
+
+__global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_down_wide_q3(GroupedArgs p) {
+  extern __shared__ __align__(16) uint16_t lds_g[];
+  uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
+  const int b = static_cast<int>(blockIdx.x);
+  if (b < p.dn_shared) {
+    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    return;
+  }
+  const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
+  if (slot >= p.active[0]) return;
+  const SlotDesc* d = p.desc + slot;
+  const int n = d->n_tok, base = d->tok_base;
+  if (n > p.max_rows) return;
+  int r = 0;
+  for (; n - r > 8; r += 16) down_wide_q3<2>(p, slot, grp, min(n - r, 16), base + r, lds);
+  if (n > r) down_wide_q3<1>(p, slot, grp, n - r, base + r, lds);
+}
+
 // Blocks [0, up_shared): the shared expert (bf16 w1/w3, all T tokens); the
 // others: up_groups blocks per slot.
 template <typename Raw>
@@ -1448,11 +1694,12 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
                                   const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                   int repeat) {
   hipError_t e;
-  if (grouped_wide(d)) {
+  if (grouped_wide(d) || grouped_wide_q3(d)) {
+    const bool planes = d.quant == DSK_QUANT_FP4;
     const WideCall w{3, d.tokens, nullptr, 0, d.inter_shared > 0};
     if ((e = stage_open(kStageUp)) != hipSuccess) return e;
     for (int r = 0; r < repeat; ++r) {
-      if (!a.x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
+      if (planes && !a.x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
       if ((e = launch_wide_up(d, L, a, desc, xrow, wrow, w, s)) != hipSuccess) return e;
     }
     if ((e = stage_open(kStageDown)) != hipSuccess) return e;
@@ -1481,10 +1728,15 @@ size_t wide_lds(int rows, int planes, int K) {
 
 // The wide kernels from four tokens (gate/up + down: H 4096, top-8 of 256 at three
 // tokens 88 us against 81 on the streaming kernels, at five 114 and 118, H 5120,
-// top-6 of 384 at six 155 and 225), the others of the grouped path from eight.
-int decode_grouped_up_min(const dsk_moe_desc& d) { return grouped_wide(d) ? 4 : kDecodeGroupedUpMin; }
+// top-6 of 384 at six 155 and 225; q3 at five 147 and 158, at six 180 and 487), the
+// others of the grouped path from eight.
+int decode_grouped_up_min(const dsk_moe_desc& d) {
+  return grouped_wide(d) || grouped_wide_q3(d) ? 4 : kDecodeGroupedUpMin;
+}
 
 bool grouped_wide(const dsk_moe_desc& d) { return wide_shapes(d) && grouped_path(d) && !prefill_gemm(d); }
+
+bool grouped_wide_q3(const dsk_moe_desc& d) { return wide_q3(d) && grouped_path(d) && !prefill_gemm(d); }
 
 bool wide_shapes(const dsk_moe_desc& d) {
   return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_BF16 && d.hidden % kWdStep == 0 &&
@@ -1506,8 +1758,12 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
   p.y_bf16 = w.y_bf16;
   p.sh_tg = (d.tokens + kGsCols - 1) / kGsCols;
   p.up_groups = (d.inter / 16 + kWdWaves - 1) / kWdWaves;
-  p.up_shared = w.shared ? (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2) * p.sh_tg : 0;
   p.dn_groups = d.hidden / 256;
+  if (d.quant == DSK_QUANT_Q3) {
+    p.up_groups = (d.inter / 16 + kWqUpTiles - 1) / kWqUpTiles;
+    p.dn_groups = d.hidden / 128;
+  }
+  p.up_shared = w.shared ? (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2) * p.sh_tg : 0;
   p.dn_shared = w.shared && d.inter_shared > 0 ? d.hidden / 128 * p.sh_tg : 0;
   return p;
 }
@@ -1519,9 +1775,11 @@ hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const Exper
   const GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, w);
   const unsigned blocks = static_cast<unsigned>(p.up_shared + max_slots(d) * p.up_groups);
   const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
-  size_t lds = wide_lds(rows, 2, d.hidden);
+  const bool q3 = d.quant == DSK_QUANT_Q3;
+  size_t lds = q3 ? wq_lds_bytes(1) : wide_lds(rows, 2, d.hidden);
   if (p.up_shared > 0 && gs_up_lds_bytes() > lds) lds = gs_up_lds_bytes();
-  if (w.h_planes == 2) launch_kernel(k_up_wide<2>, blocks, kWdWaves * 64, lds, s, p);
+  if (q3) launch_kernel(k_up_wide_q3, blocks, kWdWaves * 64, lds, s, p);
+  else if (w.h_planes == 2) launch_kernel(k_up_wide<2>, blocks, kWdWaves * 64, lds, s, p);
   else launch_kernel(k_up_wide<3>, blocks, kWdWaves * 64, lds, s, p);
   return hipGetLastError();
 }
@@ -1531,11 +1789,19 @@ hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const Exp
   const GroupedArgs p = wide_args(d, L, a, desc, nullptr, nullptr, w);
   const unsigned blocks = static_cast<unsigned>(p.dn_shared + max_slots(d) * p.dn_groups);
   const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
-  size_t lds = wide_lds(rows, w.h_planes, d.inter);
+  const bool q3 = d.quant == DSK_QUANT_Q3;
+  size_t lds = q3 ? wq_lds_bytes(2) : wide_lds(rows, w.h_planes, d.inter);
   if (p.dn_shared > 0 && gs_down_lds_bytes() > lds) lds = gs_down_lds_bytes();
-  if (w.h_planes == 2) launch_kernel(k_down_wide<2>, blocks, kWdWaves * 64, lds, s, p);
+  if (q3) launch_kernel(k_down_wide_q3, blocks, kWdWaves * 64, lds, s, p);
+  else if (w.h_planes == 2) launch_kernel(k_down_wide<2>, blocks, kWdWaves * 64, lds, s, p);
   else launch_kernel(k_down_wide<3>, blocks, kWdWaves * 64, lds, s, p);
   return hipGetLastError();
+}
+
+bool wide_q3(const dsk_moe_desc& d) {
+  return d.quant == DSK_QUANT_Q3 && d.x_dtype == DSK_DTYPE_BF16 && d.hidden >= kWqStep && d.inter >= kWqStep &&
+         d.inter_shared % 128 == 0 && int64_t{d.tokens} * d.top_k * d.inter < (int64_t{1} << 31) &&
+         int64_t{d.tokens} * d.hidden < (int64_t{1} << 31);
 }
 
 bool wide_pair(const dsk_moe_desc& d) {
@@ -1570,7 +1836,7 @@ hipError_t launch_experts_wide_pair(const dsk_moe_desc& d, const Workspace& L, c
 hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                     const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                     int repeat, bool x_planes_ready) {
-  const bool wide = grouped_wide(d);
+  const bool wide = grouped_wide(d) || grouped_wide_q3(d);
   GroupedArgs p = grouped_args(d, L, a, desc, xrow, wrow);
   p.up_shared = 0;
   const unsigned blocks = static_cast<unsigned>(max_slots(d) * p.up_groups);
@@ -1578,7 +1844,7 @@ hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, c
   for (int r = 0; r < repeat; ++r) {
     hipError_t e = hipSuccess;
     if (wide) {
-      if (!x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
+      if (d.quant == DSK_QUANT_FP4 && !x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
       if ((e = launch_wide_up(d, L, a, desc, xrow, wrow, WideCall{3, d.tokens, nullptr, 0, false}, s)) != hipSuccess)
         return e;
       continue;

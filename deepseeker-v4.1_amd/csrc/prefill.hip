@@ -1156,7 +1156,7 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   const bool on = mx && __syncthreads_and(ok ? 1 : 0);
   const int rtoks = on ? kPfToksMx : kPfToks;
   const int rows = t < n_act ? desc[t].n_tok : 0;
-  const int cnt = on && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;   // (narrow slots: the wide kernels)
+  const int cnt = (on || !mx) && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;   // (narrow slots: the wide kernels)
   int incl = cnt;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
@@ -1202,9 +1202,13 @@ int prefill_max_tiles(const dsk_moe_desc& d) {
 // of its columns empty, takes 3.5: at H 5120 and 2000 tokens (31 rows a slot
 // on average) gate/up + down 2087 us without, 2010 up to 16 rows, 1976 up to
 // 24, 1905 up to 32.  Where a slot has more than 96 rows on average few are
-// that small, and their launches would cost more than they save.
+// that small, and their launches would cost more than they save.  q3 slots up to
+// 16 rows (one pass): 300 tokens at H 4096, top-8 of 256, gate/up + down 1868 us
+// on GEMM tiles alone, 1213 with, 1327 with slots of up to 32 rows.
 int prefill_narrow_rows(const dsk_moe_desc& d) {
-  return prefill_mx(d) && wide_shapes(d) && int64_t{d.tokens} * d.top_k <= int64_t{96} * d.n_experts ? 32 : 0;
+  if (int64_t{d.tokens} * d.top_k > int64_t{96} * d.n_experts) return 0;
+  if (d.quant == DSK_QUANT_Q3) return prefill_gemm(d) && wide_q3(d) ? 16 : 0;
+  return prefill_mx(d) && wide_shapes(d) ? 32 : 0;
 }
 
 // The shared expert's GEMM tiles are one block per 128 features and 256 tokens:

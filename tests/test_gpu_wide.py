@@ -1,4 +1,4 @@
-"""GPU parity of the wide FP4 kernels (a slot's dispatch rows in passes of up to 32
+"""GPU parity of the wide kernels (a slot's dispatch rows in passes of up to 32
 over the whole of K) against the oracle, where their tiles can go wrong: one row,
 15 / 16 / 17 rows (a column tile and its edge), 31 / 32 / 33 (a pass and its edge),
 an intermediate that fills its last block of row tiles in part, and, from 128
@@ -55,6 +55,15 @@ def test_wide_float32_pairs(T, hot, H, I):
     """float32 x: passes of 16 rows and a part of one, the shared expert over one and two
     groups of 64 tokens, the decode pipeline's form (3 tokens)."""
     _check(L.LayerSpec(H=H, E=16, k=4, I=I, I_shared=256), T, hot, 370 + T, f"f32 H {H} I {I}", f32=True)
+
+
+@pytest.mark.parametrize("T,hot,H,I", [(4, 0, 512, 512), (9, 4, 1024, 640), (16, 4, 768, 768), (17, 4, 1024, 896),
+                                       (40, 4, 5120, 512), (150, 0, 1024, 768), (300, 4, 512, 1024)])
+def test_wide_q3(T, hot, H, I):
+    """q3: sets of eight rows and a part of one, passes of sixteen, one to three blocks
+    after the last superblock, the decode pipeline's form (4 tokens), and, from 128
+    tokens, slots beside the GEMM tiles (300: none of them narrow)."""
+    _check(L.LayerSpec(H=H, E=16, k=4, I=I, I_shared=256, quant=L.QUANT_Q3), T, hot, 410 + T, f"q3 H {H} I {I}")
 
 
 @pytest.mark.parametrize("T", [4, 7])
