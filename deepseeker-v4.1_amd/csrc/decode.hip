@@ -1993,7 +1993,7 @@ hipError_t launch_experts_decode(const dsk_moe_desc& d, const Workspace& L, cons
     }
   }
   if ((e = stage_open(kStageDown)) != hipSuccess) return e;
-  if (d.tokens >= kDecodeGroupedDownMin && grouped_path(d)) {
+  if ((gup || d.tokens >= kDecodeGroupedDownMin) && grouped_path(d)) {
     // routed and shared down per slot (one output row per dispatch row), then the combine
     // h in FP8 planes where the wide gate/up wrote it
     const bool hpl = gup && (grouped_wide(d) || grouped_wide_q3(d));

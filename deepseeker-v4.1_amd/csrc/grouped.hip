@@ -1731,6 +1731,11 @@ size_t wide_lds(int rows, int planes, int K) {
 // top-6 of 384 at six 155 and 225; q3 at five 147 and 158, at six 180 and 487), the
 // others of the grouped path from eight.
 int decode_grouped_up_min(const dsk_moe_desc& d) {
+  // q3 shapes without the factored decode kernels: k_up_q3 with one superblock a wave (H
+  // a multiple of 4096), k_down_q3 (I 2048).  Gate/up + down of one token at H 5120, I
+  // 2304: 151 -> 63 us; layer at H 2048, I 1024: 53.5 -> 39.5 us; at H 4096, I 512 one
+  // token is faster on k_up_q3 (41.3 against 45.5), two are not (61.1, 47.9)
+  if (grouped_wide_q3(d) && (d.hidden % 4096 != 0 || d.inter != 2048)) return d.hidden % 4096 != 0 ? 1 : 2;
   return grouped_wide(d) || grouped_wide_q3(d) ? 4 : kDecodeGroupedUpMin;
 }
 

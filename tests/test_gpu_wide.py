@@ -57,11 +57,11 @@ def test_wide_float32_pairs(T, hot, H, I):
     _check(L.LayerSpec(H=H, E=16, k=4, I=I, I_shared=256), T, hot, 370 + T, f"f32 H {H} I {I}", f32=True)
 
 
-@pytest.mark.parametrize("T,hot,H,I", [(4, 0, 512, 512), (9, 4, 1024, 640), (16, 4, 768, 768), (17, 4, 1024, 896),
+@pytest.mark.parametrize("T,hot,H,I", [(1, 0, 1024, 640), (2, 0, 4096, 512), (4, 0, 512, 512), (9, 4, 1024, 640), (16, 4, 768, 768), (17, 4, 1024, 896),
                                        (40, 4, 5120, 512), (150, 0, 1024, 768), (300, 4, 512, 1024)])
 def test_wide_q3(T, hot, H, I):
     """q3: sets of eight rows and a part of one, passes of sixteen, one to three blocks
-    after the last superblock, the decode pipeline's form (4 tokens), and, from 128
+    after the last superblock, the decode pipeline's form (1, 2, 4 tokens), and, from 128
     tokens, slots beside the GEMM tiles (300: none of them narrow)."""
     _check(L.LayerSpec(H=H, E=16, k=4, I=I, I_shared=256, quant=L.QUANT_Q3), T, hot, 410 + T, f"q3 H {H} I {I}")
 
