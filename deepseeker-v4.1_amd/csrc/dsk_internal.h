@@ -378,6 +378,7 @@ struct WideCall {
   const int32_t* on;         // device switch of the slots' blocks, or null
   int y_bf16;                // routed rows as bf16
   bool shared;               // also the shared expert (hs hi / lo planes, float32 ys)
+  bool sh_on = false;        // ... under the same switch, ys rounded to bf16 (q3)
 };
 bool wide_shapes(const dsk_moe_desc& d);
 hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,

@@ -588,7 +588,8 @@ hipError_t launch_combine(const dsk_moe_desc& d, const Workspace& L, const Exper
   int mode = Is > 0 ? kSharedF32 : (a.shared_out ? kSharedExt : kNoShared);
   const void* shared_ext = a.shared_out;
   const bool pf = prefill_gemm(d);
-  if (pf && Is > 0 && !prefill_shared_wide(d)) {   // the prefill GEMM wrote the shared output already rounded to bf16
+  // the prefill GEMM (q3: the wide kernels too) wrote the shared output already rounded to bf16
+  if (pf && Is > 0 && (d.quant == DSK_QUANT_Q3 || !prefill_shared_wide(d))) {
     mode = kSharedExt;
     shared_ext = ys;
   }

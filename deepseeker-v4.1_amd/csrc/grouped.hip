@@ -56,6 +56,7 @@ struct GroupedArgs {
   int max_rows;                                  // slots with more rows are another kernel's
   const int32_t* on;                             // device switch of the FP4 slots' blocks, or null (on)
   int y_bf16;                                    // routed rows rounded to bf16
+  int sh_on;                                     // shared blocks under the switch too, ys rounded to bf16
   int sh_tg;                                     // shared expert: groups of kGsCols tokens in blocks of their own
 };
 
@@ -567,7 +568,17 @@ __device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, in
 #pragma unroll
     for (int c = 0; c < kGsCT; ++c) {
       const int t = c * 16 + r16;
-      if (t < ncol) *reinterpret_cast<f32x4*>(p.ys + static_cast<int64_t>(g0 + t) * p.H + rt * 16 + 4 * g4) = acc[c];
+      const int64_t at = static_cast<int64_t>(g0 + t) * p.H + rt * 16 + 4 * g4;
+      if (t < ncol && p.sh_on) {
+        ushort4 b;
+        b.x = f32_to_bf16_bits(acc[c][0]);
+        b.y = f32_to_bf16_bits(acc[c][1]);
+        b.z = f32_to_bf16_bits(acc[c][2]);
+        b.w = f32_to_bf16_bits(acc[c][3]);
+        *reinterpret_cast<ushort4*>(reinterpret_cast<uint16_t*>(p.ys) + at) = b;
+      } else if (t < ncol) {
+        *reinterpret_cast<f32x4*>(p.ys + at) = acc[c];
+      }
     }
     __syncthreads();   // the next group restages buffer 0
   }
@@ -1276,11 +1287,12 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.up_shared) {
+    if (p.sh_on && !*p.on) return;
     up_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
     return;
   }
   const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
-  if (slot >= p.active[0]) return;
+  if (slot >= p.active[0] || (p.on && !*p.on)) return;
   const SlotDesc* d = p.desc + slot;
   const int n = d->n_tok, base = d->tok_base;
   if (n > p.max_rows) return;
@@ -1294,11 +1306,12 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.dn_shared) {
+    if (p.sh_on && !*p.on) return;
     down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
     return;
   }
   const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
-  if (slot >= p.active[0]) return;
+  if (slot >= p.active[0] || (p.on && !*p.on)) return;
   const SlotDesc* d = p.desc + slot;
   const int n = d->n_tok, base = d->tok_base;
   if (n > p.max_rows) return;
@@ -1728,20 +1741,32 @@ size_t wide_lds(int rows, int planes, int K) {
 
 // The wide kernels from four tokens (gate/up + down: H 4096, top-8 of 256 at three
 // tokens 88 us against 81 on the streaming kernels, at five 114 and 118, H 5120,
-// top-6 of 384 at six 155 and 225; q3 at five 147 and 158, at six 180 and 487), the
+// top-6 of 384 at six 155 and 225), the
 // others of the grouped path from eight.
 int decode_grouped_up_min(const dsk_moe_desc& d) {
   // q3 shapes without the factored decode kernels: k_up_q3 with one superblock a wave (H
   // a multiple of 4096), k_down_q3 (I 2048).  Gate/up + down of one token at H 5120, I
   // 2304: 151 -> 63 us; layer at H 2048, I 1024: 53.5 -> 39.5 us; at H 4096, I 512 one
   // token is faster on k_up_q3 (41.3 against 45.5), two are not (61.1, 47.9)
-  if (grouped_wide_q3(d) && (d.hidden % 4096 != 0 || d.inter != 2048)) return d.hidden % 4096 != 0 ? 1 : 2;
-  return grouped_wide(d) || grouped_wide_q3(d) ? 4 : kDecodeGroupedUpMin;
+  if (grouped_wide_q3(d)) return d.hidden % 4096 != 0 ? 1 : 2;
+  return grouped_wide(d) ? 4 : kDecodeGroupedUpMin;
 }
 
 bool grouped_wide(const dsk_moe_desc& d) { return wide_shapes(d) && grouped_path(d) && !prefill_gemm(d); }
 
-bool grouped_wide_q3(const dsk_moe_desc& d) { return wide_q3(d) && grouped_path(d) && !prefill_gemm(d); }
+// Below 24 tokens the column tiles' factored products (H a multiple of 4096, I of
+// 512) keep their shapes: a layer of H 4096, I 2048, top-8 of 256 takes 8 / 12 / 16
+// tokens in 215 / 280 / 340 us there and 218 / 284 / 329 in the wide kernels, but 86 /
+// 114 / 127 and 95 / 120 / 130 when the routing is skewed (Zipf, 15 experts: few blocks,
+// each with all of K to walk); 32 tokens skewed 196 and 154.  So does the decode
+// pipeline's factored gate/up (4 tokens 140 and 141, skewed 75 and 92).
+static bool q3_tiles(const dsk_moe_desc& d) {
+  return d.hidden % 4096 == 0 && d.inter % 512 == 0 && d.tokens < 24 && (d.tokens >= 3 || d.inter == 2048);
+}
+
+bool grouped_wide_q3(const dsk_moe_desc& d) {
+  return wide_q3(d) && grouped_path(d) && !prefill_gemm(d) && !q3_tiles(d);
+}
 
 bool wide_shapes(const dsk_moe_desc& d) {
   return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_BF16 && d.hidden % kWdStep == 0 &&
@@ -1760,6 +1785,7 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
   p.he = p.hp + static_cast<size_t>(d.tokens) * d.top_k * w.h_planes * d.inter;
   p.max_rows = w.max_rows;
   p.on = w.on;
+  p.sh_on = w.on && w.sh_on ? 1 : 0;
   p.y_bf16 = w.y_bf16;
   p.sh_tg = (d.tokens + kGsCols - 1) / kGsCols;
   p.up_groups = (d.inter / 16 + kWdWaves - 1) / kWdWaves;

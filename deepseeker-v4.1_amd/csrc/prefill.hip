@@ -747,7 +747,7 @@ __device__ __forceinline__ bool pf_unit_2d(const PfArgs& p, int t0, int n, int& 
 // The shared expert's units when the MX kernels take every routed tile
 // (2-D per XCD where the shapes allow), else every unit (1-D per XCD).
 __device__ __forceinline__ bool pf_unit(const PfArgs& p, int& tile, int& rt) {
-  if (*p.mx_on) {
+  if (*p.mx_on == 1) {
     const int n = p.tiles[0] - p.tiles[1];
     return n % 4 == 0 && p.row_tiles % 2 == 0 ? pf_unit_2d(p, p.tiles[1], n, tile, rt)
                                                : pf_unit_in(p, p.tiles[1], n, tile, rt);
@@ -1140,10 +1140,14 @@ __global__ __launch_bounds__(256) void k_pf_planes(const uint16_t* __restrict__ 
 // expert's tiles of kPfToks tokens.  The routed tiles run on the MX kernels
 // (kPfToksMx rows each) when the layer allows it (mx) and every active
 // slot's six FP4 arrays are 16-byte aligned (the LDS DMA's pieces), else on
-// the 8-wave kernels (kPfToks rows each); tiles[2 + 2 max_tiles] says which.
+// the 8-wave kernels (kPfToks rows each).  Slots of at most `narrow` rows are
+// the wide kernels' with the MX kernels, and of q3 layers when at least
+// min_narrow slots are that small.  with_shared: the shared expert's tiles
+// (2: only if the narrow q3 slots stay here; it is the wide kernels' else).
+// tiles[2 + 2 max_tiles]: 1 on the MX kernels, 2 narrow q3 slots on the wide ones, 0.
 __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ desc,
                                                    const int32_t* __restrict__ active, int E, int T,
-                                                   int with_shared, int max_tiles, int mx, int narrow,
+                                                   int with_shared, int max_tiles, int mx, int narrow, int min_narrow,
                                                    int32_t* __restrict__ tiles) {
   __shared__ int32_t wsum[16];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -1156,7 +1160,9 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   const bool on = mx && __syncthreads_and(ok ? 1 : 0);
   const int rtoks = on ? kPfToksMx : kPfToks;
   const int rows = t < n_act ? desc[t].n_tok : 0;
-  const int cnt = (on || !mx) && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;   // (narrow slots: the wide kernels)
+  const bool few = __syncthreads_count(rows > 0 && rows <= narrow) < min_narrow;
+  const bool wide_q3 = !mx && narrow > 0 && !few;
+  const int cnt = (on || wide_q3) && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;
   int incl = cnt;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
@@ -1175,7 +1181,7 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
     tiles[2 + off + j] = t;
     tiles[2 + max_tiles + off + j] = j * rtoks;
   }
-  const int sh = with_shared ? (T + kPfToks - 1) / kPfToks : 0;
+  const int sh = with_shared == 1 || (with_shared && !wide_q3) ? (T + kPfToks - 1) / kPfToks : 0;
   for (int j = t; j < sh; j += 1024) {
     tiles[2 + total + j] = -1;
     tiles[2 + max_tiles + total + j] = j * kPfToks;
@@ -1183,7 +1189,7 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   if (t == 0) {
     tiles[0] = total + sh;
     tiles[1] = total;
-    tiles[2 + 2 * max_tiles] = on ? 1 : 0;
+    tiles[2 + 2 * max_tiles] = on ? 1 : wide_q3 ? 2 : 0;
   }
 }
 
@@ -1205,6 +1211,10 @@ int prefill_max_tiles(const dsk_moe_desc& d) {
 // that small, and their launches would cost more than they save.  q3 slots up to
 // 16 rows (one pass): 300 tokens at H 4096, top-8 of 256, gate/up + down 1868 us
 // on GEMM tiles alone, 1213 with, 1327 with slots of up to 32 rows.
+// Few such slots (skewed routing) are better left to the tiles (they fill the
+// same launch; the wide kernels' walk over K takes its 40 us and more however few
+// blocks it has: 128 tokens on 15 experts, 220 us a layer without, 288 with), so
+// k_pf_tiles counts them: from two tiles a CU on (prefill_min_narrow).
 int prefill_narrow_rows(const dsk_moe_desc& d) {
   if (int64_t{d.tokens} * d.top_k > int64_t{96} * d.n_experts) return 0;
   if (d.quant == DSK_QUANT_Q3) return prefill_gemm(d) && wide_q3(d) ? 16 : 0;
@@ -1214,7 +1224,12 @@ int prefill_narrow_rows(const dsk_moe_desc& d) {
 // The shared expert's GEMM tiles are one block per 128 features and 256 tokens:
 // 16 blocks at 200 tokens, 107 us beside idle CUs for its gate/up (59 for its
 // down).  Up to 512 tokens it runs as blocks of the wide kernels instead (64
-// tokens and 64 features each), under the routed slots' stream.
+// tokens and 64 features each), under the routed slots' stream (q3: where the
+// narrow slots do, its output rounded to bf16 as the GEMM tiles write it).
+static int prefill_min_narrow(const dsk_moe_desc& d) {
+  return d.quant == DSK_QUANT_Q3 ? (2 * 256 * 128 + d.inter - 1) / d.inter : 0;
+}
+
 bool prefill_shared_wide(const dsk_moe_desc& d) {
   return prefill_narrow_rows(d) > 0 && d.inter_shared > 0 && d.tokens <= 512;
 }
@@ -1237,9 +1252,10 @@ hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, con
   const bool mx = prefill_mx(d);
   const int narrow = prefill_narrow_rows(d);
   const bool sh_wide = prefill_shared_wide(d);
-  const WideCall wide{2, narrow, tiles + 2 + 2 * max_tiles, prefill_rows_bf16(d, a.rows_out) ? 1 : 0, sh_wide};
-  launch_kernel(k_pf_tiles, 1, 1024, 0, s, a.desc, a.active, d.n_experts, T, Is > 0 && !sh_wide ? 1 : 0, max_tiles,
-                mx ? 1 : 0, narrow, tiles);
+  const WideCall wide{2, narrow, tiles + 2 + 2 * max_tiles, prefill_rows_bf16(d, a.rows_out) ? 1 : 0, sh_wide,
+                      q3};
+  launch_kernel(k_pf_tiles, 1, 1024, 0, s, a.desc, a.active, d.n_experts, T, Is == 0 ? 0 : !sh_wide ? 1 : q3 ? 2 : 0,
+                max_tiles, mx ? 1 : 0, narrow, prefill_min_narrow(d), tiles);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
 

@@ -84,3 +84,11 @@ def test_wide_slots_beside_gemm_tiles(T, E, k):
     the shared expert in the wide kernels (up to 512 tokens) and in GEMM tiles."""
     r = _check(L.LayerSpec(H=1024, E=E, k=k, I=768, I_shared=256), T, 0, 350, f"E {E} k {k}")
     assert int(r["counts"].min()) <= 32 or E == 24
+
+
+@pytest.mark.parametrize("T,hot,E", [(130, 0, 64), (150, 40, 64), (150, 0, 40), (513, 0, 256)])
+def test_wide_q3_prefill_slots(T, hot, E):
+    """q3 from 128 tokens: from 32 slots of at most 16 rows these and (up to 512 tokens)
+    the shared expert on the wide kernels beside GEMM tiles (64 and 256 experts), with
+    fewer all on GEMM tiles (40 experts)."""
+    _check(L.LayerSpec(H=512, E=E, k=4, I=2048, I_shared=256, quant=L.QUANT_Q3), T, hot, 470 + T, f"q3 E {E}")
