@@ -56,6 +56,7 @@ struct GroupedArgs {
   int max_rows;                                  // slots with more rows are another kernel's
   const int32_t* on;                             // device switch of the FP4 slots' blocks, or null (on)
   int y_bf16;                                    // routed rows rounded to bf16
+  int slot_step;                                 // wide q3: a block takes every slot_step-th slot
   int sh_on;                                     // shared blocks under the switch too, ys rounded to bf16
   int sh_tg;                                     // shared expert: groups of kGsCols tokens in blocks of their own
 };
@@ -1291,14 +1292,17 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     up_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
     return;
   }
-  const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
-  if (slot >= p.active[0] || (p.on && !*p.on)) return;
-  const SlotDesc* d = p.desc + slot;
-  const int n = d->n_tok, base = d->tok_base;
-  if (n > p.max_rows) return;
-  int r = 0;
-  for (; n - r > 8; r += 16) up_wide_q3<2>(p, slot, grp, min(n - r, 16), base + r, lds);
-  if (n > r) up_wide_q3<1>(p, slot, grp, n - r, base + r, lds);
+  const int rb = b - p.up_shared, first = rb / p.up_groups, grp = rb % p.up_groups;
+  const int n_act = p.active[0];
+  if (p.on && !*p.on) return;
+  for (int slot = first; slot < n_act; slot += p.slot_step) {
+    const SlotDesc* d = p.desc + slot;
+    const int n = d->n_tok, base = d->tok_base;
+    if (n > p.max_rows) continue;
+    int r = 0;
+    for (; n - r > 8; r += 16) up_wide_q3<2>(p, slot, grp, min(n - r, 16), base + r, lds);
+    if (n > r) up_wide_q3<1>(p, slot, grp, n - r, base + r, lds);
+  }
 }
 
 __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_down_wide_q3(GroupedArgs p) {
@@ -1310,14 +1314,17 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
     return;
   }
-  const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
-  if (slot >= p.active[0] || (p.on && !*p.on)) return;
-  const SlotDesc* d = p.desc + slot;
-  const int n = d->n_tok, base = d->tok_base;
-  if (n > p.max_rows) return;
-  int r = 0;
-  for (; n - r > 8; r += 16) down_wide_q3<2>(p, slot, grp, min(n - r, 16), base + r, lds);
-  if (n > r) down_wide_q3<1>(p, slot, grp, n - r, base + r, lds);
+  const int rb = b - p.dn_shared, first = rb / p.dn_groups, grp = rb % p.dn_groups;
+  const int n_act = p.active[0];
+  if (p.on && !*p.on) return;
+  for (int slot = first; slot < n_act; slot += p.slot_step) {
+    const SlotDesc* d = p.desc + slot;
+    const int n = d->n_tok, base = d->tok_base;
+    if (n > p.max_rows) continue;
+    int r = 0;
+    for (; n - r > 8; r += 16) down_wide_q3<2>(p, slot, grp, min(n - r, 16), base + r, lds);
+    if (n > r) down_wide_q3<1>(p, slot, grp, n - r, base + r, lds);
+  }
 }
 
 // Blocks [0, up_shared): the shared expert (bf16 w1/w3, all T tokens); the
@@ -1794,6 +1801,12 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
     p.up_groups = (d.inter / 16 + kWqUpTiles - 1) / kWqUpTiles;
     p.dn_groups = d.hidden / 128;
   }
+  // q3 under the device switch: blocks for 64 slots, each walking every 64th.  Skewed
+  // routing switches them off, and a block per slot then costs what it takes to launch
+  // 8192 that only look (layer of 300 tokens, top-8 of 256: 406 us, 395 so, 390
+  // without the wide kernels; even routing 200 tokens: 982 and 1029, without 1801)
+  p.slot_step = max_slots(d);
+  if (d.quant == DSK_QUANT_Q3 && w.on && p.slot_step > 64) p.slot_step = 64;
   p.up_shared = w.shared ? (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2) * p.sh_tg : 0;
   p.dn_shared = w.shared && d.inter_shared > 0 ? d.hidden / 128 * p.sh_tg : 0;
   return p;
@@ -1804,7 +1817,7 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
 hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                           const int32_t* xrow, const float* wrow, const WideCall& w, hipStream_t s) {
   const GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, w);
-  const unsigned blocks = static_cast<unsigned>(p.up_shared + max_slots(d) * p.up_groups);
+  const unsigned blocks = static_cast<unsigned>(p.up_shared + p.slot_step * p.up_groups);
   const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
   const bool q3 = d.quant == DSK_QUANT_Q3;
   size_t lds = q3 ? wq_lds_bytes(1) : wide_lds(rows, 2, d.hidden);
@@ -1818,7 +1831,7 @@ hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const Exper
 hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                             const WideCall& w, hipStream_t s) {
   const GroupedArgs p = wide_args(d, L, a, desc, nullptr, nullptr, w);
-  const unsigned blocks = static_cast<unsigned>(p.dn_shared + max_slots(d) * p.dn_groups);
+  const unsigned blocks = static_cast<unsigned>(p.dn_shared + p.slot_step * p.dn_groups);
   const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
   const bool q3 = d.quant == DSK_QUANT_Q3;
   size_t lds = q3 ? wq_lds_bytes(2) : wide_lds(rows, w.h_planes, d.inter);

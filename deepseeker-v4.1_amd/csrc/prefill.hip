@@ -1217,7 +1217,8 @@ int prefill_max_tiles(const dsk_moe_desc& d) {
 // k_pf_tiles counts them: from two tiles a CU on (prefill_min_narrow).
 int prefill_narrow_rows(const dsk_moe_desc& d) {
   if (int64_t{d.tokens} * d.top_k > int64_t{96} * d.n_experts) return 0;
-  if (d.quant == DSK_QUANT_Q3) return prefill_gemm(d) && wide_q3(d) ? 16 : 0;
+  if (d.quant == DSK_QUANT_Q3)   // (with more than 16 rows a slot on average few are that small)
+    return prefill_gemm(d) && wide_q3(d) && int64_t{d.tokens} * d.top_k <= int64_t{16} * d.n_experts ? 16 : 0;
   return prefill_mx(d) && wide_shapes(d) ? 32 : 0;
 }
 
