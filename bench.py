@@ -607,10 +607,14 @@ def main() -> int:
         routed_us = float(np.mean(r["stage_us"][:, 2] + r["stage_us"][:, 3]))
         achieved = rs["bytes_mean"] / (routed_us * 1e-6)
         mx = mx_decode(T, args.quant)
-        up_k = ("k_up_grouped" if T >= 8 else "k_up_q3" if args.quant == "q3" else
-                "k_up_mx" if mx else "k_up_stream")
-        dn_k = ("k_down_q3" if args.quant == "q3" and T <= 4 else "k_down_mx" if mx else
-                "k_down_decode_staged" if T <= 2 else "k_down_grouped + k_combine")
+        if args.quant == "q3":
+            up_k = "k_up_wide_q3" if T >= 24 else "k_up_grouped" if T >= 8 else "k_up_q3"
+            dn_k = ("k_down_wide_q3 + k_combine" if T >= 24 else
+                    "k_down_grouped + k_combine" if T >= 3 else "k_down_q3")
+        else:
+            up_k = "k_up_wide" if T >= 4 else "k_up_mx" if mx else "k_up_stream"
+            dn_k = ("k_down_wide + k_combine" if T >= 4 else
+                    "k_down_mx" if mx else "k_down_grouped + k_combine")
         roofline = {"bound": "hbm", "achieved": round(achieved / 1e9, 1), "peak": PEAK_HBM / 1e9,
                     "unit": "GB/s", "frac": round(achieved / PEAK_HBM, 4),
                     **traffic_fields([up_k, dn_k], workload),

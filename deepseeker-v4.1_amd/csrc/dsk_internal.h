@@ -364,8 +364,8 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
                                   const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                   int repeat);
 // Its kernels one at a time, for the decode pipeline: the routed gate/up
-// alone (from kDecodeGroupedUpMin tokens) and the down (routed rows from h,
-// shared from hs; from kDecodeGroupedDownMin tokens).
+// alone (from decode_grouped_up_min tokens) and the down (routed rows from h,
+// shared from hs; from kDecodeGroupedDownMin tokens, or where the gate/up ran here).
 // x_planes_ready: the routing kernel already wrote x's FP8 planes (grouped_wide).
 hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                     const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,

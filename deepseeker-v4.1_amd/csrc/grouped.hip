@@ -4,10 +4,16 @@
 // moe_layer (src/deepseeker/mlx_forward.py:388-406) and its shared expert
 // (src/deepseeker/mlx_runner.py:765-783) when each active expert sees only a
 // handful of tokens: every expert's weights must be streamed from HBM once,
-// and the MFMA B operand (16 columns) is mostly empty.  A block takes one
-// slot (an active expert, or the shared expert as a pseudo-slot over all T
-// tokens) and a group of row tiles; it walks the slot's dispatch rows in
-// column tiles of kGNC.  For each column tile the block gathers only that
+// and the MFMA B operand (16 columns) is mostly empty.
+//
+// The wide kernels (k_up_wide, k_down_wide and their float32 and q3 forms)
+// take most shapes: a block's waves walk all of K of one slot together with the
+// weights straight in registers and all of the slot's rows of a pass staged.
+// The others (k_up_grouped, k_down_grouped: FP4 with H or I out of the wide
+// kernels' range, q3 below one superblock or 24 tokens, the decode pipeline's
+// down at three tokens) are column tiles: a block takes one slot (an active expert, or the
+// shared expert as a pseudo-slot over all T tokens) and a group of row tiles;
+// it walks the slot's dispatch rows in column tiles of kGNC.  For each column tile the block gathers only that
 // tile's activation rows into LDS (x for gate/up, the h planes for down), the
 // waves issue their first weight batches behind those loads (not in front of
 // them, where the LDS stores would wait for the weights too), and each wave

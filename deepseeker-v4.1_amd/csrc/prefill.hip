@@ -37,8 +37,9 @@
 // bf16 products' rate for the same work.  k_pf_planes writes x's planes
 // before the gate/up; the gate/up's epilogue writes h's.
 //
-// Tile list: one entry per 256 dispatch rows of every active expert, then the
-// shared expert's token tiles.  Workgroup b runs on XCD b mod 8; blocks are
+// Tile list: one entry per 256 dispatch rows (MX kernels: 128, and 64 where at
+// most 64 are left) of every active expert with more rows than the wide kernels
+// take (prefill_narrow_rows), then the shared expert's token tiles.  Workgroup b runs on XCD b mod 8; blocks are
 // mapped to (tile, weight-row tile) so that each XCD walks a contiguous range
 // with the row tiles of one token tile adjacent, which keeps that tile's
 // activations in the XCD's L2 while they are reused.
