@@ -370,8 +370,9 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
 hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                     const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                     int repeat, bool x_planes_ready);
-// Wide FP4 kernels (grouped.hip): a slot's dispatch rows in tiles of up to 64
+// Wide FP4 kernels (grouped.hip): a slot's dispatch rows in passes of up to 32
 // over the whole of K, x and h as FP8 planes in stage rows.
+constexpr int kAllRows = 0x7fffffff;   // WideCall::max_rows: every slot, whatever its rows
 struct WideCall {
   int h_planes;              // 3, or 2 of h rounded to bf16 (the prefill GEMM's form, in Workspace::hp)
   int max_rows;              // slots with more dispatch rows are another kernel's

@@ -861,7 +861,6 @@ __device__ __forceinline__ void down_wide_tile(const GroupedArgs& p, int slot, i
   }
 }
 
-// Rows of a slot in passes of the widest tile the remaining ones fill.
 // Column tiles of a pass and steps in flight.  Of one column tile three steps:
 // two took 289 us of gate/up at 64 tokens (H 4096, top-8 of 256) against 259,
 // four 307 (12 KB in flight per wave then overrun the XCD's L2: a 128-byte row
@@ -871,8 +870,10 @@ constexpr int kWdMaxCT = 2;
 constexpr int kWdNB1 = 3, kWdNB2 = 2;
 
 // Blocks [0, up_shared): the shared expert, sh_tg groups of kGsCols tokens
-// each; the others: up_groups blocks per slot.
-template <int NPH>
+// each; the others: up_groups blocks per slot, which walk its rows in passes of
+// up to CT column tiles.  (A slot has more rows than the call has tokens where a
+// caller's routing names an expert twice in a row.)
+template <int NPH, int CT>
 __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_up_wide(GroupedArgs p) {
   extern __shared__ __align__(16) uint16_t lds_g[];
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
@@ -889,13 +890,13 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   const void* const wp[4] = {desc_ptr(p.desc, slot, 0), desc_ptr(p.desc, slot, 1), desc_ptr(p.desc, slot, 3),
                              desc_ptr(p.desc, slot, 4)};
   int r = 0;
-  for (; n - r > 32; r += 16 * kWdMaxCT)
-    up_wide_tile<kWdMaxCT, kWdNB2, NPH>(p, wp, grp, min(n - r, 16 * kWdMaxCT), base + r, lds);
-  if (n - r > 16) up_wide_tile<2, kWdNB2, NPH>(p, wp, grp, n - r, base + r, lds);
-  else if (n > r) up_wide_tile<1, kWdNB1, NPH>(p, wp, grp, n - r, base + r, lds);
+  if (CT == 2 || n > 16)
+    for (; n - r > 16 * (CT - 1); r += 16 * CT)
+      up_wide_tile<CT, kWdNB2, NPH>(p, wp, grp, min(n - r, 16 * CT), base + r, lds);
+  if (n > r) up_wide_tile<1, kWdNB1, NPH>(p, wp, grp, n - r, base + r, lds);
 }
 
-template <int NPH>
+template <int NPH, int CT>
 __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_down_wide(GroupedArgs p) {
   extern __shared__ __align__(16) uint16_t lds_g[];
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
@@ -910,10 +911,9 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   const int n = d->n_tok, base = d->tok_base;
   if (n > p.max_rows) return;
   int r = 0;
-  for (; n - r > 32; r += 16 * kWdMaxCT)
-    down_wide_tile<kWdMaxCT, kWdNB2, NPH>(p, slot, grp, min(n - r, 16 * kWdMaxCT), base + r, lds);
-  if (n - r > 16) down_wide_tile<2, kWdNB2, NPH>(p, slot, grp, n - r, base + r, lds);
-  else
+  if (CT == 2 || n > 16)
+    for (; n - r > 16 * (CT - 1); r += 16 * CT)
+      down_wide_tile<CT, kWdNB2, NPH>(p, slot, grp, min(n - r, 16 * CT), base + r, lds);
   if (n > r) down_wide_tile<1, kWdNB1, NPH>(p, slot, grp, n - r, base + r, lds);
 }
 
@@ -1722,7 +1722,7 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
   hipError_t e;
   if (grouped_wide(d) || grouped_wide_q3(d)) {
     const bool planes = d.quant == DSK_QUANT_FP4;
-    const WideCall w{3, d.tokens, nullptr, 0, d.inter_shared > 0};
+    const WideCall w{3, kAllRows, nullptr, 0, d.inter_shared > 0};
     if ((e = stage_open(kStageUp)) != hipSuccess) return e;
     for (int r = 0; r < repeat; ++r) {
       if (planes && !a.x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
@@ -1745,11 +1745,6 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
   }
   if ((e = stage_open(kStageDown)) != hipSuccess) return e;
   return grouped_down(d, p, s, repeat);
-}
-
-// The wide kernels' rows (max_rows: of the largest slot they may get) and planes fit the LDS.
-size_t wide_lds(int rows, int planes, int K) {
-  return rows <= 16 ? wd_lds_bytes(1, planes, K) : wd_lds_bytes(kWdMaxCT, planes, K);
 }
 
 // The wide kernels from four tokens (gate/up + down: H 4096, top-8 of 256 at three
@@ -1785,8 +1780,8 @@ bool wide_shapes(const dsk_moe_desc& d) {
   return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_BF16 && d.hidden % kWdStep == 0 &&
          d.inter % kWdStep == 0 && d.inter_shared % 128 == 0 && d.hidden < 8192 && d.inter < 8192 &&
          int64_t{d.tokens} * d.top_k * 3 * d.inter < (int64_t{1} << 32) &&
-         int64_t{d.tokens} * 2 * d.hidden < (int64_t{1} << 32) && wide_lds(64, 3, d.inter) <= kMaxLds &&
-         wide_lds(64, 2, d.hidden) <= kMaxLds;
+         int64_t{d.tokens} * 2 * d.hidden < (int64_t{1} << 32) && wd_lds_bytes(kWdMaxCT, 3, d.inter) <= kMaxLds &&
+         wd_lds_bytes(kWdMaxCT, 2, d.hidden) <= kMaxLds;
 }
 
 namespace {
@@ -1824,13 +1819,14 @@ hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const Exper
                           const int32_t* xrow, const float* wrow, const WideCall& w, hipStream_t s) {
   const GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, w);
   const unsigned blocks = static_cast<unsigned>(p.up_shared + p.slot_step * p.up_groups);
-  const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
+  const int ct = d.tokens <= 16 ? 1 : kWdMaxCT;   // column tiles of a pass
   const bool q3 = d.quant == DSK_QUANT_Q3;
-  size_t lds = q3 ? wq_lds_bytes(1) : wide_lds(rows, 2, d.hidden);
+  size_t lds = q3 ? wq_lds_bytes(1) : wd_lds_bytes(ct, 2, d.hidden);
   if (p.up_shared > 0 && gs_up_lds_bytes() > lds) lds = gs_up_lds_bytes();
   if (q3) launch_kernel(k_up_wide_q3, blocks, kWdWaves * 64, lds, s, p);
-  else if (w.h_planes == 2) launch_kernel(k_up_wide<2>, blocks, kWdWaves * 64, lds, s, p);
-  else launch_kernel(k_up_wide<3>, blocks, kWdWaves * 64, lds, s, p);
+  else if (w.h_planes == 2) launch_kernel(k_up_wide<2, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);
+  else if (ct == 1) launch_kernel(k_up_wide<3, 1>, blocks, kWdWaves * 64, lds, s, p);
+  else launch_kernel(k_up_wide<3, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);
   return hipGetLastError();
 }
 
@@ -1838,13 +1834,14 @@ hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const Exp
                             const WideCall& w, hipStream_t s) {
   const GroupedArgs p = wide_args(d, L, a, desc, nullptr, nullptr, w);
   const unsigned blocks = static_cast<unsigned>(p.dn_shared + p.slot_step * p.dn_groups);
-  const int rows = d.tokens < w.max_rows ? d.tokens : w.max_rows;
+  const int ct = d.tokens <= 16 ? 1 : kWdMaxCT;   // column tiles of a pass
   const bool q3 = d.quant == DSK_QUANT_Q3;
-  size_t lds = q3 ? wq_lds_bytes(2) : wide_lds(rows, w.h_planes, d.inter);
+  size_t lds = q3 ? wq_lds_bytes(2) : wd_lds_bytes(ct, w.h_planes, d.inter);
   if (p.dn_shared > 0 && gs_down_lds_bytes() > lds) lds = gs_down_lds_bytes();
   if (q3) launch_kernel(k_down_wide_q3, blocks, kWdWaves * 64, lds, s, p);
-  else if (w.h_planes == 2) launch_kernel(k_down_wide<2>, blocks, kWdWaves * 64, lds, s, p);
-  else launch_kernel(k_down_wide<3>, blocks, kWdWaves * 64, lds, s, p);
+  else if (w.h_planes == 2) launch_kernel(k_down_wide<2, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);
+  else if (ct == 1) launch_kernel(k_down_wide<3, 1>, blocks, kWdWaves * 64, lds, s, p);
+  else launch_kernel(k_down_wide<3, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);
   return hipGetLastError();
 }
 
@@ -1863,7 +1860,7 @@ bool wide_pair(const dsk_moe_desc& d) {
 hipError_t launch_experts_wide_pair(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                     const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                     int repeat, bool hs_ready) {
-  GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, WideCall{3, d.tokens, nullptr, 0, d.inter_shared > 0});
+  GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, WideCall{3, kAllRows, nullptr, 0, d.inter_shared > 0});
   if (hs_ready) p.up_shared = 0;
   p.x = reinterpret_cast<const uint16_t*>(a.ws + L.xb_hi);
   p.x_lo = reinterpret_cast<const uint16_t*>(a.ws + L.xb_lo);
@@ -1895,7 +1892,7 @@ hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, c
     hipError_t e = hipSuccess;
     if (wide) {
       if (d.quant == DSK_QUANT_FP4 && !x_planes_ready && (e = launch_pf_planes(d, L, a, s)) != hipSuccess) return e;
-      if ((e = launch_wide_up(d, L, a, desc, xrow, wrow, WideCall{3, d.tokens, nullptr, 0, false}, s)) != hipSuccess)
+      if ((e = launch_wide_up(d, L, a, desc, xrow, wrow, WideCall{3, kAllRows, nullptr, 0, false}, s)) != hipSuccess)
         return e;
       continue;
     }
@@ -1911,7 +1908,7 @@ hipError_t launch_grouped_down(const dsk_moe_desc& d, const Workspace& L, const 
                                const SlotDesc* desc, hipStream_t s, int repeat, bool h_planes) {
   if (h_planes) {
     for (int r = 0; r < repeat; ++r) {
-      const hipError_t e = launch_wide_down(d, L, a, desc, WideCall{3, d.tokens, nullptr, 0, d.inter_shared > 0}, s);
+      const hipError_t e = launch_wide_down(d, L, a, desc, WideCall{3, kAllRows, nullptr, 0, d.inter_shared > 0}, s);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -92,3 +92,25 @@ def test_wide_q3_prefill_slots(T, hot, E):
     the shared expert on the wide kernels beside GEMM tiles (64 and 256 experts), with
     fewer all on GEMM tiles (40 experts)."""
     _check(L.LayerSpec(H=512, E=E, k=4, I=2048, I_shared=256, quant=L.QUANT_Q3), T, hot, 470 + T, f"q3 E {E}")
+
+
+@pytest.mark.parametrize("quant,H,I,T,k", [("fp4", 1024, 512, 1, 8), ("fp4", 1024, 512, 3, 12), ("fp4", 1024, 768, 20, 4),
+                                           ("fp4", 3072, 512, 127, 2), ("q3", 1024, 640, 1, 8), ("q3", 1024, 640, 5, 12),
+                                           ("q3", 1024, 640, 24, 4)])
+def test_wide_repeated_experts(quant, H, I, T, k):
+    """A caller's routing that names an expert several times in a row: slots of more
+    rows than the call has tokens (1 to 16 tokens: the LDS of one column tile, with
+    more than 16 rows; more tokens: of two)."""
+    from dsk_moe.layer import experts_forward
+    print(f"wide repeated {quant} H={H} I={I} T={T} k={k}", flush=True)
+    spec = L.LayerSpec(H=H, E=16, k=k, I=I, I_shared=256, quant=L.QUANT_Q3 if quant == "q3" else L.QUANT_FP4)
+    d = synth.make_layer(spec, 450 + T, T)
+    rng = np.random.default_rng(T)
+    idx = np.where(np.arange(k) < k - k // 4, 3, rng.integers(0, spec.E, (T, k))).astype(np.int32)
+    w = (rng.random((T, k), dtype=np.float32) + 0.5) / k
+    r = L.moe_forward(d["x"], None, None, d["bank"], d["shared"], spec, routing=(idx, w, None, None))
+    assert int(r["counts"].max()) > T
+    out = experts_forward(d["x"].to(DEV), torch.from_numpy(idx).to(DEV), torch.from_numpy(w).to(DEV),
+                          to_bank(d["bank"]), to_shared(d["shared"]))
+    c, rel = assert_layer_close(out.cpu().float(), r["y_ref"])
+    print(f"cos={c:.9f} rel={rel:.2e} rows {int(r['counts'].max())}", flush=True)
