@@ -198,8 +198,8 @@ __device__ __forceinline__ void up_tile(const UpArgs& p, LoadA load_a, int K, in
         float h[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const float gg = fminf(g[q], p.limit);
-          const float uu = fminf(fmaxf(u[q], -p.limit), p.limit);
+          const float gg = clamp_gate(g[q], p.limit);
+          const float uu = clamp_up(u[q], p.limit);
           h[q] = gg / (1.0f + expf(-gg)) * uu * wr;
         }
         const int64_t off = dst + row0 + 4 * g4;

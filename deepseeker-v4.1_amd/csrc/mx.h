@@ -89,8 +89,8 @@ __device__ __forceinline__ float max_over_rows(float v) {
 // the exponential unit and the hardware reciprocal (a few ulp; the FP8 planes
 // the result goes into keep 2^-14 of their group's largest value).
 __device__ __forceinline__ float silu_clamped_fast(float g, float u, float limit) {
-  const float gg = fminf(g, limit);
-  const float uu = fminf(fmaxf(u, -limit), limit);
+  const float gg = clamp_gate(g, limit);
+  const float uu = clamp_up(u, limit);
   return gg * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gg)) * uu;
 }
 

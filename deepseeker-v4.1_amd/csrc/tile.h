@@ -348,9 +348,18 @@ __device__ __forceinline__ void split_bf16(float v, uint16_t& hi, uint16_t& lo) 
   lo = f32_to_bf16_bits(v - bf16_bits_to_f32(hi));
 }
 
+// The clamps of SwiGLU: min(g, limit) and u within +-limit.  A NaN stays one
+// (v_minimum3 / v_maximum3; fminf and fmaxf would turn it into the limit, and an
+// infinite activation, whose products are NaN where planes, pairs or factored sums
+// cancel, into finite outputs).
+__device__ __forceinline__ float clamp_gate(float g, float limit) { return __builtin_elementwise_minimum(g, limit); }
+__device__ __forceinline__ float clamp_up(float u, float limit) {
+  return __builtin_elementwise_minimum(__builtin_elementwise_maximum(u, -limit), limit);
+}
+
 __device__ __forceinline__ float silu_clamped(float g, float u, float limit) {
-  const float gg = fminf(g, limit);
-  const float uu = fminf(fmaxf(u, -limit), limit);
+  const float gg = clamp_gate(g, limit);
+  const float uu = clamp_up(u, limit);
   return gg / (1.0f + expf(-gg)) * uu;
 }
 

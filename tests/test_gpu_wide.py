@@ -114,3 +114,33 @@ def test_wide_repeated_experts(quant, H, I, T, k):
                           to_bank(d["bank"]), to_shared(d["shared"]))
     c, rel = assert_layer_close(out.cpu().float(), r["y_ref"])
     print(f"cos={c:.9f} rel={rel:.2e} rows {int(r['counts'].max())}", flush=True)
+
+
+@pytest.mark.parametrize("quant,H,I,T,E,k", [
+    ("fp4", 1024, 512, 20, 16, 4), ("fp4", 5120, 768, 4, 16, 4), ("fp4", 1024, 768, 200, 16, 4),
+    ("fp4", 2560, 768, 200, 64, 2), ("fp4", 384, 128, 9, 8, 2), ("q3", 1024, 640, 20, 16, 4), ("q3", 4096, 512, 10, 16, 4),
+    ("q3", 512, 2048, 130, 64, 4), ("q3", 1024, 640, 300, 16, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_not_finite_activations(quant, H, I, T, E, k, dtype):
+    """A row of x with an infinity or a NaN comes out as NaN throughout (as the oracle
+    gives it), on FP8 planes, bf16 pairs and factored sums alike; other rows are untouched."""
+    from dsk_moe.layer import experts_forward
+    print(f"not finite {quant} H={H} I={I} T={T} {dtype}", flush=True)
+    spec = L.LayerSpec(H=H, E=E, k=k, I=I, I_shared=128, quant=L.QUANT_Q3 if quant == "q3" else L.QUANT_FP4)
+    d = synth.make_layer(spec, 480, T)
+    rng = np.random.default_rng(T)
+    idx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    w = (rng.random((T, k), dtype=np.float32) + 0.5) / k
+    clean = d["x"].to(dtype)
+    x = clean.clone()
+    bad = [0, T // 2, T - 1]
+    for t, v in zip(bad, (float("inf"), float("-inf"), float("nan"))):
+        x[t, (77 * (t + 1)) % H] = v
+    r = L.moe_forward(x, None, None, d["bank"], None, spec, routing=(idx, w, None, None))
+    assert torch.isnan(r["y_ref"][bad]).all()
+    bank = to_bank(d["bank"])
+    run = lambda v: experts_forward(v.to(DEV), torch.from_numpy(idx).to(DEV), torch.from_numpy(w).to(DEV), bank).cpu()
+    out, ok = run(x), np.setdiff1d(np.arange(T), bad)
+    assert torch.isnan(out[bad]).all()
+    assert torch.equal(out[ok], run(clean)[ok])
+    assert_layer_close(out[ok].float(), r["y_ref"][ok])
