@@ -64,6 +64,7 @@ struct GroupedArgs {
   int y_bf16;                                    // routed rows rounded to bf16
   int slot_step;                                 // wide q3: a block takes every slot_step-th slot
   int sh_on;                                     // shared blocks under the switch too, ys rounded to bf16
+  int sh_tiles;                                  // shared expert in column tiles (up_block, down_block)
   int sh_tg;                                     // shared expert: groups of kGsCols tokens in blocks of their own
 };
 
@@ -533,6 +534,20 @@ __device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, int 
 
 static_assert(size_t{kGW / 2} * kGsCT * 64 * 16 <= gs_up_lds_bytes(), "the SwiGLU exchange fits the buffers");
 
+// Gate/up of the shared expert, block b: column tiles of a few row tiles (up to kGNC
+// tokens: the wide walk takes as long however few they are: experts' kernels of two
+// tokens at H 4096, I 2048, top-8 104 us with it, 82 with the tiles), or the wide walk over group
+// b % sh_tg of kGsCols tokens and every sh_tg-th after it.
+__device__ __forceinline__ void up_shared(const GroupedArgs& p, int b, uint16_t* lds) {
+  if (!p.sh_tiles) {
+    up_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds);
+    return;
+  }
+  const int rt = b * kGI + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kGKS;
+  auto load_w = [&](RawBF16& r, int role, uint32_t row, int kc) { load_raw_nc(r, role ? p.ws3 : p.ws1, row, p.H, kc); };
+  up_block<RawBF16>(p, load_w, [&](int) -> const void* { return p.ws1; }, rt, rt < p.Is / 16, p.T, 0, true, lds);
+}
+
 // Down of the shared expert over more than kGNC tokens, as up_shared_wide:
 // block b's eight waves each take one row tile of w2 (16 output rows) over
 // K = Is, the h planes (hi, lo) of up to kGsCols tokens staged per K block.
@@ -589,6 +604,114 @@ __device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, in
     }
     __syncthreads();   // the next group restages buffer 0
   }
+}
+
+// Down of one block: row tile rt (output rows 16 rt ..) of w2 for the n
+// dispatch rows base .. base + n - 1 (shared: tokens 0 .. n - 1), K = I (Is).
+template <typename Raw, typename LoadW, typename WPtr>
+__device__ __forceinline__ void down_block(const GroupedArgs& p, LoadW load_w, WPtr wptr, int rt, int n, int base,
+                                           bool shared, uint16_t* lds) {
+  constexpr int G = batch_blocks<Raw>();
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int item = wave / kDKS, ks = wave % kDKS;
+  const int K = shared ? p.Is : p.I, nblk = K / 128;
+  const int per = (nblk + kDKS - 1) / kDKS;
+  const int k0 = min(ks * per, nblk), k1 = min(k0 + per, nblk);
+  const int hs = K + 8;
+  const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
+  const uint16_t* src_hi = shared ? p.hs_hi : p.h_hi;
+  const uint16_t* src_lo = shared ? p.hs_lo : p.h_lo;
+  uint16_t* thi = lds;                      // [kGNC][K + 8] hi plane
+  uint16_t* tlo = lds + kGNC * hs;          // [kGNC][K + 8] lo plane
+  float (*red)[kDKS][64][4] = reinterpret_cast<float (*)[kDKS][64][4]>(lds);   // over the h tile
+  constexpr int NB = down_ring<Raw>();
+  for (int c0 = 0; c0 < n; c0 += kGNC) {
+    const int cols = min(kGNC, n - c0);
+    Raw a[NB][G];
+    // FP4: the scales of a batch's 2 blocks (all lane groups) as one 8-byte
+    // window instead of one byte per lane and block; the byte is picked at use
+    u32x2 wa[NB] = {};
+    // no condition on the loads (see load_raw_nc): blocks past the range
+    // re-read its last block (not computed)
+    auto ld = [&](Raw (&r)[G], u32x2& w, int kb) {
+      if constexpr (std::is_same_v<Raw, RawFP4> && G == 2) {
+        const int kbc = min(kb, k1 - 2);   // the range has an even number of blocks
+#pragma unroll
+        for (int i = 0; i < G; ++i) r[i].c = ldg16(static_cast<const uint8_t*>(wptr(0)) + row * static_cast<uint32_t>(K / 2) + (kbc + i) * 64 + g4 * 16);
+        w = ldg<u32x2>(static_cast<const uint8_t*>(wptr(1)) + row * static_cast<uint32_t>(K / 32) + kbc * 4);
+      } else {
+#pragma unroll
+        for (int i = 0; i < G; ++i) load_w(r[i], row, min(kb + i, k1 - 1) * 128 + g4 * 32);
+      }
+    };
+    // the h rows first (see up_block)
+    stage_rows(thi, src_hi, K, K, cols, [&](int r) { return base + c0 + r; });
+    stage_rows(tlo, src_lo, K, K, cols, [&](int r) { return base + c0 + r; });
+#pragma unroll
+    for (int i = 0; i < NB; ++i) ld(a[i], wa[i], k0 + i * G);
+    __syncthreads();
+    const bool tv = r16 < cols;
+    const uint16_t* bh = thi + (tv ? r16 : 0) * hs;
+    const uint16_t* bl = tlo + (tv ? r16 : 0) * hs;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto mm = [&](Raw (&r)[G], const u32x2& w, int kb) {
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        const int kc = (kb + i) * 128 + g4 * 32;
+        const bool ok = tv && kb + i < k1;
+        if constexpr (std::is_same_v<Raw, RawFP4> && G == 2) r[i].s = ((i == 0 ? w.x : w.y) >> (8 * g4)) & 0xffu;
+        mma_block(r[i], bh, kc, ok, acc);
+        mma_block(r[i], bl, kc, ok, acc);
+      }
+    };
+    // NB batches in a ring: each is multiplied, then reloaded NB batches ahead.
+    // Groups whose reloads all lie in the range run without conditions (a load
+    // under a condition makes the next use of an older batch wait for every
+    // load, as at a branch merge the wait counter cannot tell which were
+    // issued); the last groups reload only what remains.
+    const int nb = (k1 - k0 + G - 1) / G;
+    int j0 = 0;
+    for (; j0 + 2 * NB <= nb; j0 += NB) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        mm(a[i], wa[i], k0 + (j0 + i) * G);
+        ld(a[i], wa[i], k0 + (j0 + i + NB) * G);
+      }
+    }
+    for (; j0 < nb; j0 += NB) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        if (j0 + i < nb) {
+          mm(a[i], wa[i], k0 + (j0 + i) * G);
+          if (j0 + i + NB < nb) ld(a[i], wa[i], k0 + (j0 + i + NB) * G);
+        }
+      }
+    }
+    if constexpr (kDKS > 1) {
+      __syncthreads();   // every wave is done with the h tile
+      *reinterpret_cast<f32x4*>(&red[item][ks][lane][0]) = acc;
+      __syncthreads();
+    }
+    if (ks == 0 && tv) {
+#pragma unroll
+      for (int w = 1; w < kDKS; ++w) acc += *reinterpret_cast<const f32x4*>(&red[item][w][lane][0]);
+      float* out = shared ? p.ys : p.y;
+      *reinterpret_cast<f32x4*>(out + static_cast<int64_t>(base + c0 + r16) * p.H + rt * 16 + 4 * g4) = acc;
+    }
+    __syncthreads();   // the next column tile reuses the LDS
+  }
+}
+
+// Down of the shared expert, block b (up_shared).
+__device__ __forceinline__ void down_shared(const GroupedArgs& p, int b, uint16_t* lds) {
+  if (!p.sh_tiles) {
+    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds);
+    return;
+  }
+  const int rt = b * kDI + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kDKS;
+  auto load_w = [&](RawBF16& r, uint32_t row, int kc) { load_raw_nc(r, p.ws2, row, p.Is, kc); };
+  down_block<RawBF16>(p, load_w, [&](int) -> const void* { return p.ws2; }, rt, p.T, 0, true, lds);
 }
 
 // ---------------------------------------------------------------- wide FP4 slots
@@ -879,7 +1002,7 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.up_shared) {
-    up_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    up_shared(p, b, lds_g);
     return;
   }
   const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
@@ -902,7 +1025,7 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.dn_shared) {
-    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    down_shared(p, b, lds_g);
     return;
   }
   const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
@@ -1295,7 +1418,7 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.up_shared) {
     if (p.sh_on && !*p.on) return;
-    up_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    up_shared(p, b, lds_g);
     return;
   }
   const int rb = b - p.up_shared, first = rb / p.up_groups, grp = rb % p.up_groups;
@@ -1317,7 +1440,7 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.dn_shared) {
     if (p.sh_on && !*p.on) return;
-    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    down_shared(p, b, lds_g);
     return;
   }
   const int rb = b - p.dn_shared, first = rb / p.dn_groups, grp = rb % p.dn_groups;
@@ -1341,13 +1464,7 @@ __global__ __launch_bounds__(kGW * 64) __attribute__((amdgpu_waves_per_eu(4))) v
   const int b = static_cast<int>(blockIdx.x);
   const int item = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kGKS;
   if (b < p.up_shared) {
-    if (p.T > kGNC) {
-      up_shared_wide<false>(p, b, 0, kGsCols, lds_g);
-      return;
-    }
-    const int rt = b * kGI + item;
-    auto load_w = [&](RawBF16& r, int role, uint32_t row, int kc) { load_raw_nc(r, role ? p.ws3 : p.ws1, row, p.H, kc); };
-    up_block<RawBF16>(p, load_w, [&](int) -> const void* { return p.ws1; }, rt, rt < p.Is / 16, p.T, 0, true, lds_g);
+    up_shared(p, b, lds_g);
     return;
   }
   const int rb = b - p.up_shared;
@@ -1366,103 +1483,6 @@ __global__ __launch_bounds__(kGW * 64) __attribute__((amdgpu_waves_per_eu(4))) v
   }
   auto load_w = [&](Raw& r, int role, uint32_t row, int kc) { load_role_nc(r, wp, role, row, p.H, kc); };
   up_block<Raw>(p, load_w, [&](int i) { return wp[i]; }, rt, rt < p.I / 16, d->n_tok, d->tok_base, false, lds_g);
-}
-
-// Down of one block: row tile rt (output rows 16 rt ..) of w2 for the n
-// dispatch rows base .. base + n - 1 (shared: tokens 0 .. n - 1), K = I (Is).
-template <typename Raw, typename LoadW, typename WPtr>
-__device__ __forceinline__ void down_block(const GroupedArgs& p, LoadW load_w, WPtr wptr, int rt, int n, int base,
-                                           bool shared, uint16_t* lds) {
-  constexpr int G = batch_blocks<Raw>();
-  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r16 = lane & 15, g4 = lane >> 4;
-  const int item = wave / kDKS, ks = wave % kDKS;
-  const int K = shared ? p.Is : p.I, nblk = K / 128;
-  const int per = (nblk + kDKS - 1) / kDKS;
-  const int k0 = min(ks * per, nblk), k1 = min(k0 + per, nblk);
-  const int hs = K + 8;
-  const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
-  const uint16_t* src_hi = shared ? p.hs_hi : p.h_hi;
-  const uint16_t* src_lo = shared ? p.hs_lo : p.h_lo;
-  uint16_t* thi = lds;                      // [kGNC][K + 8] hi plane
-  uint16_t* tlo = lds + kGNC * hs;          // [kGNC][K + 8] lo plane
-  float (*red)[kDKS][64][4] = reinterpret_cast<float (*)[kDKS][64][4]>(lds);   // over the h tile
-  constexpr int NB = down_ring<Raw>();
-  for (int c0 = 0; c0 < n; c0 += kGNC) {
-    const int cols = min(kGNC, n - c0);
-    Raw a[NB][G];
-    // FP4: the scales of a batch's 2 blocks (all lane groups) as one 8-byte
-    // window instead of one byte per lane and block; the byte is picked at use
-    u32x2 wa[NB] = {};
-    // no condition on the loads (see load_raw_nc): blocks past the range
-    // re-read its last block (not computed)
-    auto ld = [&](Raw (&r)[G], u32x2& w, int kb) {
-      if constexpr (std::is_same_v<Raw, RawFP4> && G == 2) {
-        const int kbc = min(kb, k1 - 2);   // the range has an even number of blocks
-#pragma unroll
-        for (int i = 0; i < G; ++i) r[i].c = ldg16(static_cast<const uint8_t*>(wptr(0)) + row * static_cast<uint32_t>(K / 2) + (kbc + i) * 64 + g4 * 16);
-        w = ldg<u32x2>(static_cast<const uint8_t*>(wptr(1)) + row * static_cast<uint32_t>(K / 32) + kbc * 4);
-      } else {
-#pragma unroll
-        for (int i = 0; i < G; ++i) load_w(r[i], row, min(kb + i, k1 - 1) * 128 + g4 * 32);
-      }
-    };
-    // the h rows first (see up_block)
-    stage_rows(thi, src_hi, K, K, cols, [&](int r) { return base + c0 + r; });
-    stage_rows(tlo, src_lo, K, K, cols, [&](int r) { return base + c0 + r; });
-#pragma unroll
-    for (int i = 0; i < NB; ++i) ld(a[i], wa[i], k0 + i * G);
-    __syncthreads();
-    const bool tv = r16 < cols;
-    const uint16_t* bh = thi + (tv ? r16 : 0) * hs;
-    const uint16_t* bl = tlo + (tv ? r16 : 0) * hs;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    auto mm = [&](Raw (&r)[G], const u32x2& w, int kb) {
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int kc = (kb + i) * 128 + g4 * 32;
-        const bool ok = tv && kb + i < k1;
-        if constexpr (std::is_same_v<Raw, RawFP4> && G == 2) r[i].s = ((i == 0 ? w.x : w.y) >> (8 * g4)) & 0xffu;
-        mma_block(r[i], bh, kc, ok, acc);
-        mma_block(r[i], bl, kc, ok, acc);
-      }
-    };
-    // NB batches in a ring: each is multiplied, then reloaded NB batches ahead.
-    // Groups whose reloads all lie in the range run without conditions (a load
-    // under a condition makes the next use of an older batch wait for every
-    // load, as at a branch merge the wait counter cannot tell which were
-    // issued); the last groups reload only what remains.
-    const int nb = (k1 - k0 + G - 1) / G;
-    int j0 = 0;
-    for (; j0 + 2 * NB <= nb; j0 += NB) {
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        mm(a[i], wa[i], k0 + (j0 + i) * G);
-        ld(a[i], wa[i], k0 + (j0 + i + NB) * G);
-      }
-    }
-    for (; j0 < nb; j0 += NB) {
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        if (j0 + i < nb) {
-          mm(a[i], wa[i], k0 + (j0 + i) * G);
-          if (j0 + i + NB < nb) ld(a[i], wa[i], k0 + (j0 + i + NB) * G);
-        }
-      }
-    }
-    if constexpr (kDKS > 1) {
-      __syncthreads();   // every wave is done with the h tile
-      *reinterpret_cast<f32x4*>(&red[item][ks][lane][0]) = acc;
-      __syncthreads();
-    }
-    if (ks == 0 && tv) {
-#pragma unroll
-      for (int w = 1; w < kDKS; ++w) acc += *reinterpret_cast<const f32x4*>(&red[item][w][lane][0]);
-      float* out = shared ? p.ys : p.y;
-      *reinterpret_cast<f32x4*>(out + static_cast<int64_t>(base + c0 + r16) * p.H + rt * 16 + 4 * g4) = acc;
-    }
-    __syncthreads();   // the next column tile reuses the LDS
-  }
 }
 
 // Down of one q3 block in the factored form (as up_block_q3f): output row
@@ -1589,13 +1609,7 @@ k_down_grouped(GroupedArgs p) {
   const int b = static_cast<int>(blockIdx.x);
   const int item = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kDKS;
   if (b < p.dn_shared) {
-    if (p.T > kGNC) {
-      down_shared_wide(p, b, 0, kGsCols, lds_g);
-      return;
-    }
-    const int rt = b * kDI + item;
-    auto load_w = [&](RawBF16& r, uint32_t row, int kc) { load_raw_nc(r, p.ws2, row, p.Is, kc); };
-    down_block<RawBF16>(p, load_w, [&](int) -> const void* { return p.ws2; }, rt, p.T, 0, true, lds_g);
+    down_shared(p, b, lds_g);
     return;
   }
   const int rb = b - p.dn_shared;
@@ -1694,7 +1708,9 @@ GroupedArgs grouped_args(const dsk_moe_desc& d, const Workspace& L, const Expert
   p.hp = reinterpret_cast<uint8_t*>(a.ws + L.hp);
   p.up_groups = p.q3f ? d.inter / 16 : d.inter / 16 / kGI;   // factored q3: one row tile per block
   // shared gate/up: past kGNC tokens, four row tiles per block (up_shared_wide)
-  p.up_shared = d.tokens > kGNC ? (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2) : d.inter_shared / 16 / kGI;
+  p.sh_tiles = d.tokens <= kGNC ? 1 : 0;
+  p.sh_tg = 1;
+  p.up_shared = p.sh_tiles ? d.inter_shared / 16 / kGI : (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2);
   p.dn_groups = d.hidden / 16 / kDI;
   p.dn_shared = d.inter_shared > 0 ? p.dn_groups : 0;
   return p;
@@ -1786,6 +1802,17 @@ bool wide_shapes(const dsk_moe_desc& d) {
 
 namespace {
 
+int wide_col_tiles(const dsk_moe_desc& d) { return d.tokens <= 16 ? 1 : kWdMaxCT; }
+
+// The shared expert's column tiles (T rows of x, or of h's pair) in a wide launch: as
+// much LDS as two blocks a CU leave each.
+size_t shared_tile_lds(const dsk_moe_desc& d) {
+  const size_t x = static_cast<size_t>(d.tokens) * (d.hidden + 8) * 2, h = static_cast<size_t>(kGNC + d.tokens) * (d.inter_shared + 8) * 2;
+  const size_t red = static_cast<size_t>(kGI) * kGKS * 2 * 64 * 4 * sizeof(float);
+  return x > h ? (x > red ? x : red) : (h > red ? h : red);
+}
+bool wide_shared_tiles(const dsk_moe_desc& d) { return d.tokens <= kGNC && shared_tile_lds(d) <= kMaxLds / 2; }
+
 GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                       const int32_t* xrow, const float* wrow, const WideCall& w) {
   GroupedArgs p = grouped_args(d, L, a, desc, xrow, wrow);
@@ -1795,6 +1822,7 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
   p.on = w.on;
   p.sh_on = w.on && w.sh_on ? 1 : 0;
   p.y_bf16 = w.y_bf16;
+  p.sh_tiles = wide_shared_tiles(d) && d.x_dtype == DSK_DTYPE_BF16 ? 1 : 0;
   p.sh_tg = (d.tokens + kGsCols - 1) / kGsCols;
   p.up_groups = (d.inter / 16 + kWdWaves - 1) / kWdWaves;
   p.dn_groups = d.hidden / 256;
@@ -1808,9 +1836,19 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
   // without the wide kernels; even routing 200 tokens: 982 and 1029, without 1801)
   p.slot_step = max_slots(d);
   if (d.quant == DSK_QUANT_Q3 && w.on && p.slot_step > 64) p.slot_step = 64;
-  p.up_shared = w.shared ? (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2) * p.sh_tg : 0;
+  p.up_shared = !w.shared    ? 0
+                : p.sh_tiles ? d.inter_shared / 16 / kGI
+                             : (d.inter_shared / 16 + kGW / 2 - 1) / (kGW / 2) * p.sh_tg;
   p.dn_shared = w.shared && d.inter_shared > 0 ? d.hidden / 128 * p.sh_tg : 0;
   return p;
+}
+
+// LDS of a wide launch of the FP4 or q3 kernels: the slots' passes over K and the
+// shared expert's form (if any of its blocks are there).
+size_t wide_lds(const dsk_moe_desc& d, const GroupedArgs& p, int planes, int K, int shared_blocks, size_t shared_walk) {
+  size_t lds = d.quant == DSK_QUANT_Q3 ? wq_lds_bytes(planes) : wd_lds_bytes(wide_col_tiles(d), planes, K);
+  const size_t sh = shared_blocks == 0 ? 0 : p.sh_tiles ? shared_tile_lds(d) : shared_walk;
+  return sh > lds ? sh : lds;
 }
 
 }  // namespace
@@ -1818,11 +1856,10 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
 hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                           const int32_t* xrow, const float* wrow, const WideCall& w, hipStream_t s) {
   const GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, w);
-  const unsigned blocks = static_cast<unsigned>(p.up_shared + p.slot_step * p.up_groups);
-  const int ct = d.tokens <= 16 ? 1 : kWdMaxCT;   // column tiles of a pass
   const bool q3 = d.quant == DSK_QUANT_Q3;
-  size_t lds = q3 ? wq_lds_bytes(1) : wd_lds_bytes(ct, 2, d.hidden);
-  if (p.up_shared > 0 && gs_up_lds_bytes() > lds) lds = gs_up_lds_bytes();
+  const int ct = wide_col_tiles(d), planes = q3 ? 1 : 2;
+  const unsigned blocks = static_cast<unsigned>(p.up_shared + p.slot_step * p.up_groups);
+  const size_t lds = wide_lds(d, p, planes, d.hidden, p.up_shared, gs_up_lds_bytes());
   if (q3) launch_kernel(k_up_wide_q3, blocks, kWdWaves * 64, lds, s, p);
   else if (w.h_planes == 2) launch_kernel(k_up_wide<2, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);
   else if (ct == 1) launch_kernel(k_up_wide<3, 1>, blocks, kWdWaves * 64, lds, s, p);
@@ -1833,11 +1870,10 @@ hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const Exper
 hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                             const WideCall& w, hipStream_t s) {
   const GroupedArgs p = wide_args(d, L, a, desc, nullptr, nullptr, w);
-  const unsigned blocks = static_cast<unsigned>(p.dn_shared + p.slot_step * p.dn_groups);
-  const int ct = d.tokens <= 16 ? 1 : kWdMaxCT;   // column tiles of a pass
   const bool q3 = d.quant == DSK_QUANT_Q3;
-  size_t lds = q3 ? wq_lds_bytes(2) : wd_lds_bytes(ct, w.h_planes, d.inter);
-  if (p.dn_shared > 0 && gs_down_lds_bytes() > lds) lds = gs_down_lds_bytes();
+  const int ct = wide_col_tiles(d), planes = q3 ? 2 : w.h_planes;
+  const unsigned blocks = static_cast<unsigned>(p.dn_shared + p.slot_step * p.dn_groups);
+  const size_t lds = wide_lds(d, p, planes, d.inter, p.dn_shared, gs_down_lds_bytes());
   if (q3) launch_kernel(k_down_wide_q3, blocks, kWdWaves * 64, lds, s, p);
   else if (w.h_planes == 2) launch_kernel(k_down_wide<2, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);
   else if (ct == 1) launch_kernel(k_down_wide<3, 1>, blocks, kWdWaves * 64, lds, s, p);

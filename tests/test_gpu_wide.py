@@ -144,3 +144,31 @@ def test_not_finite_activations(quant, H, I, T, E, k, dtype):
     assert torch.isnan(out[bad]).all()
     assert torch.equal(out[ok], run(clean)[ok])
     assert_layer_close(out[ok].float(), r["y_ref"][ok])
+
+
+def _experts(quant, H, I, Is, T, E, k, seed, label):
+    """experts_forward of a random routing (no expert twice in a row) against the oracle."""
+    from dsk_moe.layer import experts_forward
+    print(f"wide {label} {quant} H={H} I={I} Is={Is} T={T} E={E} k={k}", flush=True)
+    spec = L.LayerSpec(H=H, E=E, k=k, I=I, I_shared=Is or 128, quant=L.QUANT_Q3 if quant == "q3" else L.QUANT_FP4)
+    d = synth.make_layer(spec, seed, T)
+    rng = np.random.default_rng(seed)
+    idx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    w = (rng.random((T, k), dtype=np.float32) + 0.5) / k
+    shared = d["shared"] if Is else None
+    r = L.moe_forward(d["x"], None, None, d["bank"], shared, spec, routing=(idx, w, None, None))
+    run = lambda: experts_forward(d["x"].to(DEV), torch.from_numpy(idx).to(DEV), torch.from_numpy(w).to(DEV),
+                                  to_bank(d["bank"]), to_shared(shared))
+    out = run()
+    assert torch.equal(out, run())
+    c, rel = assert_layer_close(out.cpu().float(), r["y_ref"])
+    print(f"cos={c:.9f} rel={rel:.2e} rows {sorted(set(int(v) for v in r['counts']))}", flush=True)
+
+
+@pytest.mark.parametrize("quant,H,I,Is,T", [("fp4", 1024, 2048, 384, 3), ("fp4", 5120, 768, 256, 7), ("fp4", 5120, 768, 256, 8),
+                                            ("fp4", 2048, 1024, 2304, 8), ("fp4", 1024, 2048, 384, 9), ("q3", 1024, 640, 256, 1),
+                                            ("q3", 1024, 640, 384, 8), ("q3", 1024, 640, 256, 9)])
+def test_wide_shared_expert_of_few_tokens(quant, H, I, Is, T):
+    """The shared expert beside wide slots: column tiles up to eight tokens (of as many
+    rows as the LDS of half a CU holds), the wide walk from there."""
+    _experts(quant, H, I, Is, T, 16, 4, 520 + T, "shared")
