@@ -1776,7 +1776,21 @@ int decode_grouped_up_min(const dsk_moe_desc& d) {
   return grouped_wide(d) ? 4 : kDecodeGroupedUpMin;
 }
 
-bool grouped_wide(const dsk_moe_desc& d) { return wide_shapes(d) && grouped_path(d) && !prefill_gemm(d); }
+// Little work: a wide block walks all of K however few blocks there are, so up to half
+// a block a CU (from H 4096 a quarter) stays with the column tiles: experts' kernels
+// with a shared expert, tiles and wide: H 3072, I 512, top-2: one token 27 and 33 us; H
+// 1024, I 768, top-4: one 23 and 26, 8 tokens (192 blocks) 29 and 28; layer of 4 tokens
+// at H 4096, I 1024, top-2 (64 blocks) 33 and 37.  So do two tokens with a shared
+// expert (H 4096, I 2048, top-8: one 58 and 48, two 69 and 83, three 94 and 89; H 5120,
+// I 2304, top-6: 63 and 54, 91 and 100, 121 and 110).
+static bool little_work(const dsk_moe_desc& d) {
+  if (d.tokens == 2 && d.inter_shared > 0) return true;
+  return int64_t{d.tokens} * d.top_k * d.inter <= int64_t{d.hidden < 4096 ? 128 : 64} * 128;
+}
+
+bool grouped_wide(const dsk_moe_desc& d) {
+  return wide_shapes(d) && grouped_path(d) && !prefill_gemm(d) && !little_work(d);
+}
 
 // Below 24 tokens the column tiles' factored products (H a multiple of 4096, I of
 // 512) keep their shapes: a layer of H 4096, I 2048, top-8 of 256 takes 8 / 12 / 16

@@ -172,3 +172,18 @@ def test_wide_shared_expert_of_few_tokens(quant, H, I, Is, T):
     """The shared expert beside wide slots: column tiles up to eight tokens (of as many
     rows as the LDS of half a CU holds), the wide walk from there."""
     _experts(quant, H, I, Is, T, 16, 4, 520 + T, "shared")
+
+
+@pytest.mark.parametrize("H,I,Is,T,k", [(1024, 512, 256, 1, 4), (1024, 512, 256, 8, 4), (1024, 512, 256, 9, 4), (4096, 256, 0, 16, 2),
+                                        (4096, 256, 0, 17, 2), (1024, 2048, 256, 1, 8), (1024, 2048, 256, 2, 8), (1024, 2048, 0, 2, 8),
+                                        (1024, 4096, 0, 4, 1), (1024, 4096, 0, 5, 1)])
+def test_wide_little_work(H, I, Is, T, k):
+    """Both sides of the work up to which FP4 slots stay with the column tiles (positions x
+    I of 16384, from H 4096 of 8192; two tokens with a shared expert)."""
+    _experts("fp4", H, I, Is, T, 16, k, 540 + T, "little work")
+
+
+@pytest.mark.parametrize("T,I,shared", [(4, 1280, True), (5, 1536, False), (8, 768, True)])
+def test_wide_decode_pipeline_sizes(T, I, shared):
+    """The decode pipeline's wide form (four tokens and more work than the column tiles keep)."""
+    _check(L.LayerSpec(H=1024, E=32, k=4, I=I, I_shared=256), T, 0, 560 + T, f"decode I {I}", shared=shared)
