@@ -61,6 +61,7 @@ struct GroupedArgs {
   const uint8_t* xe; uint8_t* he;                // their E8M0 bytes [T][H/32], [T*k][I/32]
   int max_rows;                                  // slots with more rows are another kernel's
   const int32_t* on;                             // device switch of the FP4 slots' blocks, or null (on)
+  int few;                                       // wide: slots of up to this many rows may run on wide_mul_few
   int y_bf16;                                    // routed rows rounded to bf16
   int slot_step;                                 // wide q3: a block takes every slot_step-th slot
   int sh_on;                                     // shared blocks under the switch too, ys rounded to bf16
@@ -892,57 +893,69 @@ __device__ __forceinline__ void wide_mul(const uint8_t* const (&W)[2], const uin
   });   // ends with a barrier: the buffers are free
 }
 
+// h of row tile rt, `tile` of its block, in NPH planes (two: of h rounded to bf16, as
+// the prefill GEMM rounds it) for dispatch rows base + [0, n), by the waves that
+// hold the tile's gate and up sums (`mine`); tiles 2j and 2j + 1 of a block share
+// their rows' exponents.
+template <int NCT, int NPH>
+__device__ __forceinline__ void wide_store_h(const GroupedArgs& p, const f32x4 (&gate)[NCT], const f32x4 (&up)[NCT],
+                                             bool mine, int tile, int rt, int n, int base, uint8_t* lds) {
+  const int lane = __lane_id(), r16 = lane & 15, g4 = lane >> 4;
+  float (*gmx)[NCT][16] = reinterpret_cast<float (*)[NCT][16]>(lds);   // [tile][row]: largest of its 16 features
+  float hv[NCT][4];
+  if (mine) {
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) {
+      const float wr = p.wrow[base + min(16 * c + r16, n - 1)];
+      float m = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v = silu_clamped(gate[c][q], up[c][q], p.limit) * wr;
+        if constexpr (NPH == 2) v = bf16_bits_to_f32(f32_to_bf16_bits(v));
+        hv[c][q] = v;
+        m = fmaxf(m, fabsf(v));
+      }
+      m = max_over_rows(m);
+      if (g4 == 0) gmx[tile][c][r16] = m;
+    }
+  }
+  __syncthreads();
+  if (mine) {
+    const int i0 = rt * 16 + 4 * g4;
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) {
+      const int ex = fp8_plane_exp(fmaxf(gmx[tile][c][r16], gmx[tile ^ 1][c][r16]));
+      uint32_t pl[NPH];
+      fp8_planes4<NPH>(hv[c], ex, pl);
+      if (16 * c + r16 < n) {
+        const int64_t r = base + 16 * c + r16;
+        uint8_t* dst = p.hp + r * (NPH * p.I) + (i0 >> 6) * (64 * NPH) + (i0 & 63);
+#pragma unroll
+        for (int i = 0; i < NPH; ++i) *reinterpret_cast<uint32_t*>(dst + 64 * i) = pl[i];
+        if ((tile & 1) == 0 && g4 == 0) p.he[r * (p.I / 32) + (i0 >> 5)] = static_cast<uint8_t>(e8m0_byte(ex));
+      }
+    }
+  }
+}
+
 // Gate/up of one FP4 slot: rows 128 grp + [0, 128) of w1 and w3 for dispatch
-// rows base + c0 + [0, min(n - c0, 16 NCT)); h in NPH planes (two: of h rounded
-// to bf16, as the prefill GEMM rounds it).
+// rows base + [0, n), n <= 16 NCT; h in NPH planes.
 template <int NCT, int NB, int NPH>
 __device__ __forceinline__ void up_wide_tile(const GroupedArgs& p, const void* const* wp, int grp, int n, int base,
                                              uint8_t* lds) {
   const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
   const int rt = grp * kWdWaves + wave;
-  const bool rok = rt < p.I / 16;
   const int K = p.H;
-  const uint32_t row = rok ? static_cast<uint32_t>(rt * 16 + r16) : 0u;
+  const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
   const uint8_t* const W[2] = {static_cast<const uint8_t*>(wp[0]), static_cast<const uint8_t*>(wp[2])};
   const uint8_t* const S[2] = {static_cast<const uint8_t*>(wp[1]), static_cast<const uint8_t*>(wp[3])};
   const uint32_t c0 = row * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
-  const uint32_t s0 = (rok ? static_cast<uint32_t>(rt * 16) : 0u) * static_cast<uint32_t>(K / 32);   // (the tile's first row)
+  const uint32_t s0 = static_cast<uint32_t>(rt * 16) * static_cast<uint32_t>(K / 32);   // (the tile's first row)
   const uint32_t co[2] = {c0, c0}, so[2] = {s0, s0};
   f32x4 acc[2][NCT];
   wide_mul<NCT, 2, NB>(W, S, co, so, p.xp, p.xe, K, n, [&](int r) { return p.xrow[base + r]; }, lds, acc);
-  float (*gmx)[NCT][16] = reinterpret_cast<float (*)[NCT][16]>(lds);   // [wave][tile][row]: largest of its 16 features
-  float hv[NCT][4];
-#pragma unroll
-  for (int c = 0; c < NCT; ++c) {
-    const float wr = p.wrow[base + min(16 * c + r16, n - 1)];
-    float m = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float v = silu_clamped(acc[0][c][q], acc[1][c][q], p.limit) * wr;
-      if constexpr (NPH == 2) v = bf16_bits_to_f32(f32_to_bf16_bits(v));
-      hv[c][q] = rok ? v : 0.0f;
-      m = fmaxf(m, fabsf(hv[c][q]));
-    }
-    m = max_over_rows(m);
-    if (g4 == 0) gmx[wave][c][r16] = m;
-  }
-  __syncthreads();
-  // one exponent per dispatch row and 32 features (waves 2j, 2j + 1)
-  const int i0 = rt * 16 + 4 * g4;
-#pragma unroll
-  for (int c = 0; c < NCT; ++c) {
-    const int ex = fp8_plane_exp(fmaxf(gmx[wave][c][r16], gmx[wave ^ 1][c][r16]));
-    uint32_t pl[NPH];
-    fp8_planes4<NPH>(hv[c], ex, pl);
-    if (rok && 16 * c + r16 < n) {
-      const int64_t r = base + 16 * c + r16;
-      uint8_t* dst = p.hp + r * (NPH * p.I) + (i0 >> 6) * (64 * NPH) + (i0 & 63);
-#pragma unroll
-      for (int i = 0; i < NPH; ++i) *reinterpret_cast<uint32_t*>(dst + 64 * i) = pl[i];
-      if ((wave & 1) == 0 && g4 == 0) p.he[r * (p.I / 32) + (i0 >> 5)] = static_cast<uint8_t>(e8m0_byte(ex));
-    }
-  }
+  wide_store_h<NCT, NPH>(p, acc[0], acc[1], true, wave, rt, n, base, lds);
   __syncthreads();   // the next rows reuse the LDS
 }
 
@@ -984,6 +997,186 @@ __device__ __forceinline__ void down_wide_tile(const GroupedArgs& p, int slot, i
   }
 }
 
+// ---------------------------------------------------------------- FP4 slots of few rows
+// Slots of up to kWfRows rows where the slots are many for the batch's rows
+// (wide_few_mode): their planes fit the LDS for all of K, so the waves walk without
+// barriers, and a block's rows are half as many with the K range split between two
+// waves of a row tile pair, so that blocks are half as long and the launch's last
+// ones leave less of the chip idle.  H 4096, top-8 of 256, even routing, gate/up and
+// down against the passes above: 8 tokens 93 -> 88 and 57 -> 49 us (layer 157 -> 148;
+// 10 tokens 198 -> 183, 16 243 -> 240), at H 5120, top-6 of 384, 8 tokens' experts
+// 186 -> 165.  Split in four: 8 tokens 165 (planes staged by twice the blocks).
+// Weights ahead of the planes in a block's first loads: 3-8 us slower (the planes'
+// waits then cover them).
+constexpr int kWfRows = 3;
+constexpr int kWfKS = 2;                       // K ranges of a row tile pair, one wave each
+constexpr int kWfTiles = kWdWaves / kWfKS;     // row tile pairs of a block
+constexpr int kWfNB = 4;                       // steps in flight (two: the same; five spill)
+__host__ __device__ constexpr int wf_row(int NP, int K) { return NP * K + 64; }   // rows on distinct banks
+__host__ __device__ constexpr int wf_steps(int K) { return (K / kWdStep + kWfKS - 1) / kWfKS; }   // of a K range
+constexpr size_t wf_lds_bytes(int rows, int NP, int K) {
+  return size_t(rows) * (wf_row(NP, K) + wd_scale_row(K)) + size_t(32 * kWdWaves) * wd_scale_row(wf_steps(K) * kWdStep);
+}
+
+// Blocks of a slot are kWfKS times as many with this on.  Where the passes' blocks and
+// the shared expert's would fill between half the CUs and all of them once, the passes
+// keep their longer walk (one block a CU; 8 tokens' experts 31 us and 36 at H 2048, I
+// 1024, one token with a shared expert 48 and 64 at H 4096), and where a slot has more
+// than one and a half rows on average, few of them are small (skewed routing, 8 tokens:
+// layer 64 us and 85).
+__device__ __forceinline__ bool wide_few_mode(int slots, int blocks, int positions) {
+  return 2 * positions <= 3 * slots && (blocks <= 128 || blocks > 256);
+}
+
+// acc[a], in the waves of K range 0: row tile a of this wave by the slot's n rows (row
+// r from source row src(r) of the planes q / exponents e; columns past them repeat the
+// last).  The caller may reuse the LDS past the first wf_red_bytes of it.
+constexpr int wf_red_bytes = (kWfKS - 1) * kWfTiles * 2 * 64 * 16;
+template <int NP, typename Src>
+__device__ __forceinline__ void wide_mul_few(const uint8_t* const (&W)[2], const uint8_t* const (&S)[2],
+                                             const uint32_t (&co)[2], const uint32_t (&so)[2], const uint8_t* q,
+                                             const uint8_t* e, int K, int n, Src src, uint8_t* lds, f32x4 (&acc)[2]) {
+  constexpr int kThreads = kWdWaves * 64, Q = 4, NB = kWfNB;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4, ks = wave % kWfKS, tile = wave / kWfKS;
+  const int es = wd_scale_row(K), row = wf_row(NP, K), per = NP * K / 16;   // per: 16-byte pieces of a row
+  // this wave's steps (none where the ranges before it cover K: st0 is then the last)
+  const int ns = max(min(wf_steps(K), K / kWdStep - ks * wf_steps(K)), 0);
+  const int st0 = min(ks * wf_steps(K), K / kWdStep - 1);
+  const int kw = max(ns, 1) * kWdStep, ew = wd_scale_row(kw);
+  uint8_t* xe = lds + n * row;
+  uint8_t* ws = xe + n * es + wave * (32 * wd_scale_row(wf_steps(K) * kWdStep));
+  const int inv = (65536 + K / 256 - 1) / (K / 256), invw = (65536 + kw / 256 - 1) / (kw / 256);
+  auto esrc = [&](int r) { return e + static_cast<uint32_t>(src(r)) * static_cast<uint32_t>(K / 32); };
+  auto wsrc = [&](int r) { return (r < 16 ? S[0] + so[0] : S[1] + so[1]) + (r & 15) * (K / 32) + 8 * st0; };
+  auto at = [&](int c) { return static_cast<uint32_t>(src(c / per)) * static_cast<uint32_t>(NP * K) + 16u * (c % per); };
+  WideScales<1> esc;
+  WideScales<kWdScales / kWfKS> wsc;
+  u32x4 xv[Q], w[NB][2][2];
+  const int total = n * per;
+#pragma unroll
+  for (int j = 0; j < Q; ++j) xv[j] = ldg16(q + at(min(tid + j * kThreads, total - 1)));   // no condition on the load
+  wsc.load(32, kw, invw, lane, 64, wsrc);
+  esc.load(n, K, inv, tid, kThreads, esrc);
+  asm volatile("" ::: "memory");
+  auto ldw = [&](int i, int kb) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      w[i][a][0] = ldg16(W[a] + kb * (kWdStep / 2) + co[a]);
+      w[i][a][1] = ldg16(W[a] + kb * (kWdStep / 2) + co[a] + 64);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < NB; ++i) ldw(i, st0 + max(min(i, ns - 1), 0));
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < Q; ++j) {
+    const int c = tid + j * kThreads;
+    if (c < total) *reinterpret_cast<u32x4*>(lds + (c / per) * row + 16 * (c % per)) = xv[j];
+  }
+  for (int c = tid + Q * kThreads; c < total; c += kThreads)
+    *reinterpret_cast<u32x4*>(lds + (c / per) * row + 16 * (c % per)) = ldg16(q + at(c));
+  wsc.store(ws, 32, kw, invw, lane, 64, wsrc);
+  esc.store(xe, n, K, inv, tid, kThreads, esrc);
+  acc[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+  acc[1] = acc[0];
+  const int br = min(r16, n - 1);
+  const uint8_t* wsl = ws + r16 * ew + g4;                    // + 8 per step
+  const uint8_t* xel = xe + br * es + g4 + 8 * st0;
+  const uint8_t* xb = lds + br * row + 16 * g4 + NP * kWdStep * st0;
+  __syncthreads();
+  auto mm = [&](int i) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint32_t s0 = wsl[4 * b], s1 = wsl[16 * ew + 4 * b], bs = xel[4 * b];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const uint8_t* x = xb + b * 128 * NP + 64 * p;
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(x), hi = *reinterpret_cast<const u32x4*>(x + 64 * NP);
+        acc[0] = mx_mfma(w[i][0][b], s0, lo, hi, bs - 4u * p, acc[0]);
+        acc[1] = mx_mfma(w[i][1][b], s1, lo, hi, bs - 4u * p, acc[1]);
+      }
+    }
+    asm volatile("" : "+v"(acc[0]), "+v"(acc[1])::"memory");   // (see wide_mul)
+    wsl += 8;
+    xel += 8;
+    xb += NP * kWdStep;
+  };
+  int st = 0;
+  for (; st + 2 * NB <= ns; st += NB) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      mm(i);
+      ldw(i, st0 + st + i + NB);
+    }
+  }
+  for (; st < ns; st += NB) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      if (st + i < ns) {
+        mm(i);
+        if (st + i + NB < ns) ldw(i, st0 + st + i + NB);
+      }
+    }
+  }
+  __syncthreads();   // every wave is done with the planes
+  f32x4 (*red)[kWfTiles][2][64] = reinterpret_cast<f32x4 (*)[kWfTiles][2][64]>(lds);   // [range - 1][tile][a][lane]
+  if (ks) {
+    red[ks - 1][tile][0][lane] = acc[0];
+    red[ks - 1][tile][1][lane] = acc[1];
+  }
+  __syncthreads();
+  if (!ks) {
+#pragma unroll
+    for (int r = 0; r < kWfKS - 1; ++r) {
+      acc[0] += red[r][tile][0][lane];
+      acc[1] += red[r][tile][1][lane];
+    }
+  }
+}
+
+// Gate/up of one slot of few rows: rows 16 kWfTiles grp + [0, 16 kWfTiles) of w1 and w3.
+template <int NPH>
+__device__ __forceinline__ void up_wide_few(const GroupedArgs& p, const void* const* wp, int grp, int n, int base,
+                                            uint8_t* lds) {
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4, tile = wave / kWfKS;
+  const int rt = grp * kWfTiles + tile, K = p.H;
+  const uint8_t* const W[2] = {static_cast<const uint8_t*>(wp[0]), static_cast<const uint8_t*>(wp[2])};
+  const uint8_t* const S[2] = {static_cast<const uint8_t*>(wp[1]), static_cast<const uint8_t*>(wp[3])};
+  const uint32_t c0 = static_cast<uint32_t>(rt * 16 + r16) * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
+  const uint32_t s0 = static_cast<uint32_t>(rt * 16) * static_cast<uint32_t>(K / 32);
+  const uint32_t co[2] = {c0, c0}, so[2] = {s0, s0};
+  f32x4 acc[2];
+  wide_mul_few<2>(W, S, co, so, p.xp, p.xe, K, n, [&](int r) { return p.xrow[base + r]; }, lds, acc);
+  const f32x4 g[1] = {acc[0]}, u[1] = {acc[1]};
+  wide_store_h<1, NPH>(p, g, u, wave % kWfKS == 0, tile, rt, n, base, lds + wf_red_bytes);
+}
+
+// Down of one slot of few rows: output rows 32 kWfTiles grp + [0, 32 kWfTiles) of w2.
+template <int NPH>
+__device__ __forceinline__ void down_wide_few(const GroupedArgs& p, int slot, int grp, int n, int base, uint8_t* lds) {
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int rt = (grp * kWfTiles + wave / kWfKS) * 2, K = p.I;
+  const uint8_t* W2 = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 6));
+  const uint8_t* S2 = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 7));
+  const uint8_t* const W[2] = {W2, W2};
+  const uint8_t* const S[2] = {S2, S2};
+  const uint32_t c0 = static_cast<uint32_t>(rt * 16 + r16) * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
+  const uint32_t s0 = static_cast<uint32_t>(rt * 16) * static_cast<uint32_t>(K / 32);
+  const uint32_t co[2] = {c0, c0 + static_cast<uint32_t>(8 * K)}, so[2] = {s0, s0 + static_cast<uint32_t>(K / 2)};
+  f32x4 acc[2];
+  wide_mul_few<NPH>(W, S, co, so, p.hp, p.he, K, n, [&](int r) { return base + r; }, lds, acc);
+  if (wave % kWfKS == 0 && r16 < n) {
+    const int64_t o = static_cast<int64_t>(base + r16) * p.H + rt * 16 + 4 * g4;
+    *reinterpret_cast<f32x4*>(p.y + o) = acc[0];
+    *reinterpret_cast<f32x4*>(p.y + o + 16) = acc[1];
+  }
+}
+
+// ---------------------------------------------------------------- the wide FP4 kernels
 // Column tiles of a pass and steps in flight.  Of one column tile three steps:
 // two took 289 us of gate/up at 64 tokens (H 4096, top-8 of 256) against 259,
 // four 307 (12 KB in flight per wave then overrun the XCD's L2: a 128-byte row
@@ -992,10 +1185,10 @@ __device__ __forceinline__ void down_wide_tile(const GroupedArgs& p, int slot, i
 constexpr int kWdMaxCT = 2;
 constexpr int kWdNB1 = 3, kWdNB2 = 2;
 
-// Blocks [0, up_shared): the shared expert, sh_tg groups of kGsCols tokens
-// each; the others: up_groups blocks per slot, which walk its rows in passes of
-// up to CT column tiles.  (A slot has more rows than the call has tokens where a
-// caller's routing names an expert twice in a row.)
+// Blocks [0, up_shared): the shared expert; the others: up_groups blocks per slot
+// (or kWfKS times as many), which walk its rows in passes of up to CT column tiles.
+// (A slot has more rows than the call has tokens where a caller's routing names an
+// expert twice in a row.)
 template <int NPH, int CT>
 __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_up_wide(GroupedArgs p) {
   extern __shared__ __align__(16) uint16_t lds_g[];
@@ -1005,13 +1198,23 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     up_shared(p, b, lds_g);
     return;
   }
-  const int rb = b - p.up_shared, slot = rb / p.up_groups, grp = rb % p.up_groups;
-  if (slot >= p.active[0] || (p.on && !*p.on)) return;
+  const int rb = b - p.up_shared, n_act = p.active[0];
+  const bool few = CT == 1 && p.few > 0 && wide_few_mode(n_act, n_act * p.up_groups + p.up_shared, p.T * p.k);
+  const int groups = few ? kWfKS * p.up_groups : p.up_groups;
+  const int slot = rb / groups, grp = rb % groups;
+  if (slot >= n_act || (p.on && !*p.on)) return;
   const SlotDesc* d = p.desc + slot;
   const int n = d->n_tok, base = d->tok_base;
   if (n > p.max_rows) return;
   const void* const wp[4] = {desc_ptr(p.desc, slot, 0), desc_ptr(p.desc, slot, 1), desc_ptr(p.desc, slot, 3),
                              desc_ptr(p.desc, slot, 4)};
+  if constexpr (CT == 1) {
+    if (few && n <= p.few) {
+      up_wide_few<NPH>(p, wp, grp, n, base, lds);
+      return;
+    }
+    if (grp >= p.up_groups) return;
+  }
   int r = 0;
   if (CT == 2 || n > 16)
     for (; n - r > 16 * (CT - 1); r += 16 * CT)
@@ -1028,11 +1231,21 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     down_shared(p, b, lds_g);
     return;
   }
-  const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
-  if (slot >= p.active[0] || (p.on && !*p.on)) return;
+  const int rb = b - p.dn_shared, n_act = p.active[0];
+  const bool few = CT == 1 && p.few > 0 && wide_few_mode(n_act, n_act * p.dn_groups + p.dn_shared, p.T * p.k);
+  const int groups = few ? kWfKS * p.dn_groups : p.dn_groups;
+  const int slot = rb / groups, grp = rb % groups;
+  if (slot >= n_act || (p.on && !*p.on)) return;
   const SlotDesc* d = p.desc + slot;
   const int n = d->n_tok, base = d->tok_base;
   if (n > p.max_rows) return;
+  if constexpr (CT == 1) {
+    if (few && n <= p.few) {
+      down_wide_few<NPH>(p, slot, grp, n, base, lds);
+      return;
+    }
+    if (grp >= p.dn_groups) return;
+  }
   int r = 0;
   if (CT == 2 || n > 16)
     for (; n - r > 16 * (CT - 1); r += 16 * CT)
@@ -1857,10 +2070,19 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
   return p;
 }
 
-// LDS of a wide launch of the FP4 or q3 kernels: the slots' passes over K and the
-// shared expert's form (if any of its blocks are there).
+// Rows up to which a slot may run on wide_mul_few, with LDS for two blocks a CU.
+int wide_few_rows(const dsk_moe_desc& d, int planes, int K) {
+  if (wide_col_tiles(d) != 1 || d.quant != DSK_QUANT_FP4) return 0;
+  int rows = kWfRows;
+  while (rows > 0 && wf_lds_bytes(rows, planes, K) > kMaxLds / 2) --rows;
+  return rows;
+}
+
+// LDS of a wide launch of the FP4 or q3 kernels: the slots' passes or few rows over K,
+// and the shared expert's form (if any of its blocks are there).
 size_t wide_lds(const dsk_moe_desc& d, const GroupedArgs& p, int planes, int K, int shared_blocks, size_t shared_walk) {
   size_t lds = d.quant == DSK_QUANT_Q3 ? wq_lds_bytes(planes) : wd_lds_bytes(wide_col_tiles(d), planes, K);
+  if (p.few > 0 && wf_lds_bytes(p.few, planes, K) > lds) lds = wf_lds_bytes(p.few, planes, K);
   const size_t sh = shared_blocks == 0 ? 0 : p.sh_tiles ? shared_tile_lds(d) : shared_walk;
   return sh > lds ? sh : lds;
 }
@@ -1869,10 +2091,11 @@ size_t wide_lds(const dsk_moe_desc& d, const GroupedArgs& p, int planes, int K, 
 
 hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                           const int32_t* xrow, const float* wrow, const WideCall& w, hipStream_t s) {
-  const GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, w);
+  GroupedArgs p = wide_args(d, L, a, desc, xrow, wrow, w);
   const bool q3 = d.quant == DSK_QUANT_Q3;
   const int ct = wide_col_tiles(d), planes = q3 ? 1 : 2;
-  const unsigned blocks = static_cast<unsigned>(p.up_shared + p.slot_step * p.up_groups);
+  p.few = wide_few_rows(d, planes, d.hidden);
+  const unsigned blocks = static_cast<unsigned>(p.up_shared + p.slot_step * p.up_groups * (p.few > 0 ? kWfKS : 1));
   const size_t lds = wide_lds(d, p, planes, d.hidden, p.up_shared, gs_up_lds_bytes());
   if (q3) launch_kernel(k_up_wide_q3, blocks, kWdWaves * 64, lds, s, p);
   else if (w.h_planes == 2) launch_kernel(k_up_wide<2, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);
@@ -1883,10 +2106,11 @@ hipError_t launch_wide_up(const dsk_moe_desc& d, const Workspace& L, const Exper
 
 hipError_t launch_wide_down(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, const SlotDesc* desc,
                             const WideCall& w, hipStream_t s) {
-  const GroupedArgs p = wide_args(d, L, a, desc, nullptr, nullptr, w);
+  GroupedArgs p = wide_args(d, L, a, desc, nullptr, nullptr, w);
   const bool q3 = d.quant == DSK_QUANT_Q3;
   const int ct = wide_col_tiles(d), planes = q3 ? 2 : w.h_planes;
-  const unsigned blocks = static_cast<unsigned>(p.dn_shared + p.slot_step * p.dn_groups);
+  p.few = wide_few_rows(d, planes, d.inter);
+  const unsigned blocks = static_cast<unsigned>(p.dn_shared + p.slot_step * p.dn_groups * (p.few > 0 ? kWfKS : 1));
   const size_t lds = wide_lds(d, p, planes, d.inter, p.dn_shared, gs_down_lds_bytes());
   if (q3) launch_kernel(k_down_wide_q3, blocks, kWdWaves * 64, lds, s, p);
   else if (w.h_planes == 2) launch_kernel(k_down_wide<2, kWdMaxCT>, blocks, kWdWaves * 64, lds, s, p);

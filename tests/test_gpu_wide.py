@@ -146,14 +146,15 @@ def test_not_finite_activations(quant, H, I, T, E, k, dtype):
     assert_layer_close(out[ok].float(), r["y_ref"][ok])
 
 
-def _experts(quant, H, I, Is, T, E, k, seed, label):
+def _experts(quant, H, I, Is, T, E, k, seed, label, idx=None):
     """experts_forward of a random routing (no expert twice in a row) against the oracle."""
     from dsk_moe.layer import experts_forward
     print(f"wide {label} {quant} H={H} I={I} Is={Is} T={T} E={E} k={k}", flush=True)
     spec = L.LayerSpec(H=H, E=E, k=k, I=I, I_shared=Is or 128, quant=L.QUANT_Q3 if quant == "q3" else L.QUANT_FP4)
     d = synth.make_layer(spec, seed, T)
     rng = np.random.default_rng(seed)
-    idx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    if idx is None:
+        idx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
     w = (rng.random((T, k), dtype=np.float32) + 0.5) / k
     shared = d["shared"] if Is else None
     r = L.moe_forward(d["x"], None, None, d["bank"], shared, spec, routing=(idx, w, None, None))
@@ -187,3 +188,16 @@ def test_wide_little_work(H, I, Is, T, k):
 def test_wide_decode_pipeline_sizes(T, I, shared):
     """The decode pipeline's wide form (four tokens and more work than the column tiles keep)."""
     _check(L.LayerSpec(H=1024, E=32, k=4, I=I, I_shared=256), T, 0, 560 + T, f"decode I {I}", shared=shared)
+
+
+@pytest.mark.parametrize("H,I,Is,T,k", [(5120, 256, 0, 16, 4), (1024, 768, 256, 16, 4), (5120, 2304, 0, 1, 2), (1024, 1280, 0, 9, 4),
+                                        (7168, 256, 128, 12, 6), (2048, 2304, 0, 7, 4)])
+def test_wide_few_rows(H, I, Is, T, k):
+    """Slots of one, two, three and four rows beside each other where the slots are many
+    for the rows (K ranges of one step and none, of an odd number of steps; blocks that
+    fill less than half the CUs, more than all of them, and between)."""
+    idx = np.arange(T * k).reshape(T, k)
+    for first, rows in ((0, 4), (4, 3), (7, 2)):          # rows that share their first expert
+        if first + rows <= T:
+            idx[first:first + rows, 0] = idx[first, 0]
+    _experts("fp4", H, I, Is, T, 72, k, 580 + T, "few rows", idx=idx.astype(np.int32))
