@@ -621,6 +621,15 @@ hipError_t launch_split_x(const dsk_moe_desc& d, const Workspace& L, const Exper
   return hipGetLastError();
 }
 
+// float32 calls of little work stay with the general kernels, whose blocks are short: a
+// wide block walks all of K however few there are (general and wide, without a shared
+// expert: H 2048, I 1024, top-4: one token 20 and 32 us, two 27 and 32, three 37 and 33;
+// with one: one token 27 and 43, three 44 and 44, at H 4096, I 2048, top-8: one 71 and
+// 73, two 116 and 113).
+static bool pair_little_work(const dsk_moe_desc& d) {
+  return int64_t{d.tokens} * d.top_k * d.inter <= int64_t{d.inter_shared > 0 ? 128 : 64} * 128;
+}
+
 hipError_t launch_experts(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                           hipStream_t s, int repeat) {
   const int T = d.tokens, H = d.hidden, I = d.inter, Is = d.inter_shared, k = d.top_k;
@@ -658,7 +667,7 @@ hipError_t launch_experts(const dsk_moe_desc& d, const Workspace& L, const Exper
     if ((e = launch_split_x(d, L, a, s)) != hipSuccess) return e;
     xb_hi = reinterpret_cast<const uint16_t*>(a.ws + L.xb_hi);
     xb_lo = reinterpret_cast<const uint16_t*>(a.ws + L.xb_lo);
-    if (wide_pair(d)) {
+    if (wide_pair(d) && !pair_little_work(d)) {
       if ((e = launch_experts_wide_pair(d, L, a, desc, xrow, wrow, s, repeat, false)) != hipSuccess) return e;
       return a.rows_out ? hipSuccess : launch_combine(d, L, a, s, repeat);
     }

@@ -146,7 +146,7 @@ def test_not_finite_activations(quant, H, I, T, E, k, dtype):
     assert_layer_close(out[ok].float(), r["y_ref"][ok])
 
 
-def _experts(quant, H, I, Is, T, E, k, seed, label, idx=None):
+def _experts(quant, H, I, Is, T, E, k, seed, label, idx=None, f32=False):
     """experts_forward of a random routing (no expert twice in a row) against the oracle."""
     from dsk_moe.layer import experts_forward
     print(f"wide {label} {quant} H={H} I={I} Is={Is} T={T} E={E} k={k}", flush=True)
@@ -157,12 +157,16 @@ def _experts(quant, H, I, Is, T, E, k, seed, label, idx=None):
         idx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
     w = (rng.random((T, k), dtype=np.float32) + 0.5) / k
     shared = d["shared"] if Is else None
+    if f32:
+        d["x"] = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(seed))
     r = L.moe_forward(d["x"], None, None, d["bank"], shared, spec, routing=(idx, w, None, None))
     run = lambda: experts_forward(d["x"].to(DEV), torch.from_numpy(idx).to(DEV), torch.from_numpy(w).to(DEV),
                                   to_bank(d["bank"]), to_shared(shared))
     out = run()
     assert torch.equal(out, run())
     c, rel = assert_layer_close(out.cpu().float(), r["y_ref"])
+    if f32:
+        assert rel < 1e-4       # (see _check)
     print(f"cos={c:.9f} rel={rel:.2e} rows {sorted(set(int(v) for v in r['counts']))}", flush=True)
 
 
@@ -201,3 +205,10 @@ def test_wide_few_rows(H, I, Is, T, k):
         if first + rows <= T:
             idx[first:first + rows, 0] = idx[first, 0]
     _experts("fp4", H, I, Is, T, 72, k, 580 + T, "few rows", idx=idx.astype(np.int32))
+
+
+@pytest.mark.parametrize("H,I,Is,T,k", [(1024, 512, 256, 8, 4), (1024, 512, 256, 9, 4), (1024, 512, 0, 4, 4), (1024, 512, 0, 5, 4),
+                                        (512, 2048, 128, 1, 8), (512, 2048, 0, 1, 8)])
+def test_wide_float32_little_work(H, I, Is, T, k):
+    """Both sides of the work up to which float32 calls stay with the general kernels."""
+    _experts("fp4", H, I, Is, T, 16, k, 600 + T, "float32 little work", f32=True)
