@@ -105,11 +105,8 @@ Workspace workspace_layout(const dsk_moe_desc& d) {
     L.xp = take(bf16x && d.quant == DSK_QUANT_FP4 ? T * 2 * (H + H / 32)
                 : bf16x && grouped_x_q3(d)     ? T * (2 * H + H / 8)
                                                : 0);
-    // the wide kernels' h planes: up to 512 rows of the sizes below in space of their own,
-    // else where the bf16 h pair would be (so that workspaces keep their sizes)
-    const bool own = bf16x && d.quant == DSK_QUANT_FP4 && H % 1024 == 0 && H <= 4096 &&
-                     (I == 512 || I == 1024 || I == 2048) && N <= 512;
-    L.hp = own ? take(N * 3 * (I + I / 32)) : L.h_hi;
+    // the wide kernels' h planes
+    L.hp = bf16x && wide_own_space(d) ? take(N * 3 * (I + I / 32)) : L.h_hi;
   }
   const size_t tile_bytes = prefill_gemm(d) ? (3 + 2 * static_cast<size_t>(prefill_max_tiles(d))) * 4 : 0;
   if (prefill_mx(d) && !prefill_mx_own_space(d)) {

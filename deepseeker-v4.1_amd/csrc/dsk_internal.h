@@ -402,6 +402,13 @@ hipError_t launch_pf_planes(const dsk_moe_desc& d, const Workspace& L, const Exp
 // q3 experts' wide kernels take these shapes (launch_wide_up / _down dispatch on
 // the format; h as the bf16 hi / lo pair, rows float32).
 bool wide_q3(const dsk_moe_desc& d);
+// h's three planes have workspace of their own: up to 512 dispatch rows of the sizes
+// below (at others they lie where the bf16 h pair would be, so that workspaces keep
+// their sizes).
+inline bool wide_own_space(const dsk_moe_desc& d) {
+  return d.quant == DSK_QUANT_FP4 && d.x_dtype == DSK_DTYPE_BF16 && d.hidden % 1024 == 0 && d.hidden <= 4096 &&
+         (d.inter == 512 || d.inter == 1024 || d.inter == 2048) && int64_t{d.tokens} * d.top_k <= 512;
+}
 // The grouped path runs its FP4 / q3 slots on the wide kernels.
 bool grouped_wide(const dsk_moe_desc& d);
 bool grouped_wide_q3(const dsk_moe_desc& d);

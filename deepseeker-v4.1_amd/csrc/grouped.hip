@@ -1945,11 +1945,21 @@ hipError_t grouped_down(const dsk_moe_desc& d, const GroupedArgs& p, hipStream_t
 
 }  // namespace
 
+// Rows handed to the caller stay float32, so they keep what the column tiles hold: bf16
+// products with float32 sums and h as a pair (FP4: 2.5e-6 of the rows, against 2.6e-5 on
+// the scaled MFMAs, whose sums and planes hold 2^-14), the factored q3 products (8.4e-6
+// against 1.1e-5).  Where h's planes have space of their own, the rows are the planes'.
+// H 5120, I 2304, top-6, tiles and wide: 20 tokens 424 and 331 us; H 4096, I 2048,
+// top-8, 127 tokens 761 and 593.
+static bool rows_on_tiles(const dsk_moe_desc& d) {
+  return d.quant == DSK_QUANT_FP4 ? !wide_own_space(d) : d.hidden % 4096 == 0 && d.inter % 512 == 0;
+}
+
 hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                   const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                   int repeat) {
   hipError_t e;
-  if (grouped_wide(d) || grouped_wide_q3(d)) {
+  if ((grouped_wide(d) || grouped_wide_q3(d)) && !(a.rows_out && rows_on_tiles(d))) {
     const bool planes = d.quant == DSK_QUANT_FP4;
     const WideCall w{3, kAllRows, nullptr, 0, d.inter_shared > 0};
     if ((e = stage_open(kStageUp)) != hipSuccess) return e;

@@ -122,3 +122,39 @@ def test_pinned_rows_take_their_ascending_place():
                     pinned_gather_fn=lambda *_: {e: (rows, c.to(DEV)) for e, (rows, c) in rev.items()})
     rp = L.moe_forward(d["x"], d["gate_w"], d["gate_b"], d["bank"], None, spec, pinned=rev)
     np.testing.assert_array_equal(out.float().numpy(), rp["out"].float().numpy())
+
+
+@pytest.mark.parametrize("quant,H,I,T", [("fp4", 5120, 512, 6), ("fp4", 1024, 768, 24), ("q3", 4096, 512, 26)])
+def test_expert_rows_of_bf16_activations_keep_float32(quant, H, I, T):
+    """``dsk_expert_rows`` with bf16 x, whose rows leave in float32: h as a bf16 hi / lo
+    pair (2^-17 of each value, here at most 2^-16 of the rows in the 2-norm) and float32
+    sums, where a layer's rows may come from FP8 planes (2^-14 of a group's largest)."""
+    import ctypes
+    from dsk_moe import _lib
+    from dsk_moe.ops import dispatch, make_desc, ptr, stream_of, workspace
+    print(f"rows {quant} H={H} I={I} T={T}", flush=True)
+    E, k = 16, 4
+    spec = L.LayerSpec(H=H, E=E, k=k, I=I, I_shared=128, quant=L.QUANT_Q3 if quant == "q3" else L.QUANT_FP4)
+    d = synth.make_layer(spec, 620, T)
+    rng = np.random.default_rng(T)
+    idx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    w = (rng.random((T, k), dtype=np.float32) + 0.5) / k
+    want = torch.zeros((T * k, H), dtype=torch.float64)
+    for e in np.unique(idx):
+        w1, w3, w2 = (torch.from_numpy(d["bank"].dequant(int(e), n)).double() for n in ("w1", "w3", "w2"))
+        t, j = np.nonzero(idx == e)
+        x = d["x"][t].double()
+        g, u = torch.clamp(x @ w1.T, max=10.0), torch.clamp(x @ w3.T, -10.0, 10.0)
+        h = g / (1.0 + torch.exp(-g)) * u * torch.from_numpy(w[t, j]).double()[:, None]
+        want[torch.from_numpy(t * k + j)] = h @ w2.T
+    bank, dev = to_bank(d["bank"]), torch.device("cuda:0")
+    x, wt = d["x"].to(dev), torch.from_numpy(w).to(dev)
+    desc = make_desc(tokens=T, hidden=H, n_experts=E, top_k=k, inter=I, quant=quant, x_dtype=torch.bfloat16, limit=10.0)
+    s = dispatch(torch.from_numpy(idx).to(dev), E)
+    rows, ws = torch.empty((T * k, H), device=dev), workspace(desc, dev)
+    _lib.call("dsk_expert_rows", ctypes.byref(desc), ptr(bank.table), ptr(x), ptr(wt), ptr(s["counts"]), ptr(s["offsets"]),
+              ptr(s["perm"]), ptr(s["rank"]), ptr(s["active"]), ptr(rows), ptr(ws), ws.numel(), stream_of(dev))
+    want = want[s["perm"][:T * k].cpu().long()]
+    err = float((rows.cpu().double() - want).norm() / want.norm())
+    print(f"err={err:.2e}", flush=True)
+    assert err < 2.0 ** -16
