@@ -373,10 +373,13 @@ hipError_t launch_grouped_up_routed(const dsk_moe_desc& d, const Workspace& L, c
 // Wide FP4 kernels (grouped.hip): a slot's dispatch rows in passes of up to 32
 // over the whole of K, x and h as FP8 planes in stage rows.
 constexpr int kAllRows = 0x7fffffff;   // WideCall::max_rows: every slot, whatever its rows
+// The prefill tile list's switch word: routed tiles on the MX kernels; slots of few
+// rows on the wide kernels.
+constexpr int kTilesMx = 1, kTilesWide = 2;
 struct WideCall {
   int h_planes;              // 3, or 2 of h rounded to bf16 (the prefill GEMM's form, in Workspace::hp)
   int max_rows;              // slots with more dispatch rows are another kernel's
-  const int32_t* on;         // device switch of the slots' blocks, or null
+  const int32_t* on;         // device switch of the slots' blocks (kTilesWide), or null
   int y_bf16;                // routed rows as bf16
   bool shared;               // also the shared expert (hs hi / lo planes, float32 ys)
   bool sh_on = false;        // ... under the same switch, ys rounded to bf16 (q3)

@@ -705,7 +705,7 @@ struct PfArgs {
   uint16_t* ys;                             // [T][H] the shared output, rounded to bf16
   int y_bf16;                               // routed rows rounded to bf16 (FP4 layer, combined here)
   int row_tiles;                            // weight-row tiles per token tile
-  const int32_t* mx_on;                     // [0]: routed tiles on the MX kernels (k_pf_tiles)
+  const int32_t* mx_on;                     // [0]: the switch word, kTilesMx (k_pf_tiles)
   const uint8_t* xq; const uint8_t* xe;     // x as FP8 planes in stage rows [T][2H], E8M0 [T][H/32]
   uint8_t* hq; uint8_t* he;                 // h of the MX slots, the same form [T*k][2I], [T*k][I/32]
 };
@@ -748,7 +748,7 @@ __device__ __forceinline__ bool pf_unit_2d(const PfArgs& p, int t0, int n, int& 
 // The shared expert's units when the MX kernels take every routed tile
 // (2-D per XCD where the shapes allow), else every unit (1-D per XCD).
 __device__ __forceinline__ bool pf_unit(const PfArgs& p, int& tile, int& rt) {
-  if (*p.mx_on == 1) {
+  if (*p.mx_on & kTilesMx) {
     const int n = p.tiles[0] - p.tiles[1];
     return n % 4 == 0 && p.row_tiles % 2 == 0 ? pf_unit_2d(p, p.tiles[1], n, tile, rt)
                                                : pf_unit_in(p, p.tiles[1], n, tile, rt);
@@ -1054,7 +1054,7 @@ __device__ __forceinline__ void mx_up_tile(const PfArgs& p, const SlotDesc* d, i
 __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_up(PfArgs p) {
   extern __shared__ __align__(16) char mx_lds[];
   int tile, rt;
-  if (!*p.mx_on || !pf_unit_in(p, 0, p.tiles[1], tile, rt)) return;
+  if (!(*p.mx_on & kTilesMx) || !pf_unit_in(p, 0, p.tiles[1], tile, rt)) return;
   const int slot = p.tiles[2 + tile], first = p.tiles[2 + p.max_tiles + tile];
   const SlotDesc* d = p.desc + slot;
   const int cnt = min(kPfToksMx, d->n_tok - first);
@@ -1118,7 +1118,7 @@ __device__ __forceinline__ void mx_down_tile(const PfArgs& p, const SlotDesc* d,
 __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_down(PfArgs p) {
   extern __shared__ __align__(16) char mx_lds[];
   int tile, rt;
-  if (!*p.mx_on || !pf_unit_in(p, 0, p.tiles[1], tile, rt)) return;
+  if (!(*p.mx_on & kTilesMx) || !pf_unit_in(p, 0, p.tiles[1], tile, rt)) return;
   const int slot = p.tiles[2 + tile], first = p.tiles[2 + p.max_tiles + tile];
   const SlotDesc* d = p.desc + slot;
   const int cnt = min(kPfToksMx, d->n_tok - first);
@@ -1142,10 +1142,10 @@ __global__ __launch_bounds__(256) void k_pf_planes(const uint16_t* __restrict__ 
 // (kPfToksMx rows each) when the layer allows it (mx) and every active
 // slot's six FP4 arrays are 16-byte aligned (the LDS DMA's pieces), else on
 // the 8-wave kernels (kPfToks rows each).  Slots of at most `narrow` rows are
-// the wide kernels' with the MX kernels, and of q3 layers when at least
-// min_narrow slots are that small.  with_shared: the shared expert's tiles
-// (2: only if the narrow q3 slots stay here; it is the wide kernels' else).
-// tiles[2 + 2 max_tiles]: 1 on the MX kernels, 2 narrow q3 slots on the wide ones, 0.
+// the wide kernels' (of FP4 layers: with the MX kernels) when at least min_narrow
+// slots are that small.  with_shared: the shared expert's tiles (2: only if the
+// narrow slots stay here; it is the wide kernels' else).
+// tiles[2 + 2 max_tiles]: the switch word.
 __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ desc,
                                                    const int32_t* __restrict__ active, int E, int T,
                                                    int with_shared, int max_tiles, int mx, int narrow, int min_narrow,
@@ -1162,8 +1162,8 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   const int rtoks = on ? kPfToksMx : kPfToks;
   const int rows = t < n_act ? desc[t].n_tok : 0;
   const bool few = __syncthreads_count(rows > 0 && rows <= narrow) < min_narrow;
-  const bool wide_q3 = !mx && narrow > 0 && !few;
-  const int cnt = (on || wide_q3) && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;
+  const bool wide = narrow > 0 && !few && (on || !mx);
+  const int cnt = wide && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;
   int incl = cnt;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
@@ -1182,7 +1182,7 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
     tiles[2 + off + j] = t;
     tiles[2 + max_tiles + off + j] = j * rtoks;
   }
-  const int sh = with_shared == 1 || (with_shared && !wide_q3) ? (T + kPfToks - 1) / kPfToks : 0;
+  const int sh = with_shared == 1 || (with_shared && !wide) ? (T + kPfToks - 1) / kPfToks : 0;
   for (int j = t; j < sh; j += 1024) {
     tiles[2 + total + j] = -1;
     tiles[2 + max_tiles + total + j] = j * kPfToks;
@@ -1190,7 +1190,7 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   if (t == 0) {
     tiles[0] = total + sh;
     tiles[1] = total;
-    tiles[2 + 2 * max_tiles] = on ? 1 : wide_q3 ? 2 : 0;
+    tiles[2 + 2 * max_tiles] = (on ? kTilesMx : 0) | (wide ? kTilesWide : 0);
   }
 }
 
@@ -1213,9 +1213,11 @@ int prefill_max_tiles(const dsk_moe_desc& d) {
 // 16 rows (one pass): 300 tokens at H 4096, top-8 of 256, gate/up + down 1868 us
 // on GEMM tiles alone, 1213 with, 1327 with slots of up to 32 rows.
 // Few such slots (skewed routing) are better left to the tiles (they fill the
-// same launch; the wide kernels' walk over K takes its 40 us and more however few
-// blocks it has: 128 tokens on 15 experts, 220 us a layer without, 288 with), so
-// k_pf_tiles counts them: from two tiles a CU on (prefill_min_narrow).
+// same launch; the wide kernels' walk over K takes its 20 to 40 us and more however few
+// blocks it has: q3, 128 tokens on 15 experts, 220 us a layer without, 288 with; FP4,
+// 600 tokens on 15, 476 and 514), so k_pf_tiles counts them: from two blocks a CU on
+// (prefill_min_narrow).  FP4 prompts whose shared expert runs there have the launch
+// anyway, and keep them.
 int prefill_narrow_rows(const dsk_moe_desc& d) {
   if (int64_t{d.tokens} * d.top_k > int64_t{96} * d.n_experts) return 0;
   if (d.quant == DSK_QUANT_Q3)   // (with more than 16 rows a slot on average few are that small)
@@ -1229,7 +1231,7 @@ int prefill_narrow_rows(const dsk_moe_desc& d) {
 // tokens and 64 features each), under the routed slots' stream (q3: where the
 // narrow slots do, its output rounded to bf16 as the GEMM tiles write it).
 static int prefill_min_narrow(const dsk_moe_desc& d) {
-  return d.quant == DSK_QUANT_Q3 ? (2 * 256 * 128 + d.inter - 1) / d.inter : 0;
+  return d.quant == DSK_QUANT_Q3 || !prefill_shared_wide(d) ? (2 * 256 * 128 + d.inter - 1) / d.inter : 0;
 }
 
 bool prefill_shared_wide(const dsk_moe_desc& d) {

@@ -212,3 +212,14 @@ def test_wide_few_rows(H, I, Is, T, k):
 def test_wide_float32_little_work(H, I, Is, T, k):
     """Both sides of the work up to which float32 calls stay with the general kernels."""
     _experts("fp4", H, I, Is, T, 16, k, 600 + T, "float32 little work", f32=True)
+
+
+@pytest.mark.parametrize("T,E,k,hot,I", [(820, 64, 3, 2, 768), (820, 128, 3, 2, 768), (810, 24, 2, 1, 1024), (600, 64, 3, 2, 768)])
+def test_skewed_fp4_prompt(T, E, k, hot, I):
+    """Skewed prompts: too few narrow slots for the wide kernels (left to the GEMM tiles),
+    enough of them, and, up to 800 tokens, whatever their number beside the shared expert."""
+    r = _check(L.LayerSpec(H=512, E=E, k=k, I=I, I_shared=128), T, hot, 640 + E, "skewed prompt")
+    narrow = int(((r["counts"] > 0) & (r["counts"] <= 32)).sum())
+    need = -(-2 * 256 * 128 // I)
+    assert (r["counts"][:hot] == T).all()
+    assert narrow >= need if E == 128 else narrow < need
