@@ -376,6 +376,7 @@ constexpr int kAllRows = 0x7fffffff;   // WideCall::max_rows: every slot, whatev
 // The prefill tile list's switch word: routed tiles on the MX kernels; slots of few
 // rows on the wide kernels.
 constexpr int kTilesMx = 1, kTilesWide = 2;
+constexpr int kTilesFull = 4;          // most MX tiles have more than 64 rows
 struct WideCall {
   int h_planes;              // 3, or 2 of h rounded to bf16 (the prefill GEMM's form, in Workspace::hp)
   int max_rows;              // slots with more dispatch rows are another kernel's

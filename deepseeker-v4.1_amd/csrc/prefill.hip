@@ -552,8 +552,13 @@ __device__ __forceinline__ void mx_mma(const MxOps<AF>& o, int pl, int n_ct, f32
 // few) runs as 64 columns: the four waves split the weight rows (64 each)
 // instead of leaving the two waves of columns 64..127 idle, and half the
 // token rows are loaded.  At H 5120 and 2000 tokens (31 rows a
-// slot): gate/up 1419 -> 1328 us, down 679 -> 632.
+// slot): gate/up 1419 -> 1328 us, down 679 -> 632.  A launch of more than
+// one and less than two rounds of units (two workgroups a CU), most of them of more
+// than 64 rows, keeps the 128-column form: 600 tokens on 15 experts (592 units) gate/up
+// 158 us, 173 with 64 columns; even routing, most of few rows, 512 tokens' layer 860
+// and 824.
 constexpr int kMxThreads = 256;
+constexpr int kMxRound = 2 * 256;   // units of a round
 constexpr int kPfToksMx = 128;   // dispatch rows of an MX tile
 
 template <int TOK>
@@ -1051,6 +1056,11 @@ __device__ __forceinline__ void mx_up_tile(const PfArgs& p, const SlotDesc* d, i
   }
 }
 
+__device__ __forceinline__ bool mx_narrow(const PfArgs& p, int cnt) {
+  const int units = p.tiles[1] * p.row_tiles;
+  return cnt <= 64 && (units <= kMxRound || units >= 2 * kMxRound || !(*p.mx_on & kTilesFull));
+}
+
 __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_up(PfArgs p) {
   extern __shared__ __align__(16) char mx_lds[];
   int tile, rt;
@@ -1058,7 +1068,7 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_up(PfArgs p) {
   const int slot = p.tiles[2 + tile], first = p.tiles[2 + p.max_tiles + tile];
   const SlotDesc* d = p.desc + slot;
   const int cnt = min(kPfToksMx, d->n_tok - first);
-  if (cnt <= 64) mx_up_tile<64>(p, d, first, cnt, rt, mx_lds);
+  if (mx_narrow(p, cnt)) mx_up_tile<64>(p, d, first, cnt, rt, mx_lds);
   else mx_up_tile<kPfToksMx>(p, d, first, cnt, rt, mx_lds);
 }
 
@@ -1122,7 +1132,7 @@ __global__ __launch_bounds__(kMxThreads, 2) void k_pf_mx_down(PfArgs p) {
   const int slot = p.tiles[2 + tile], first = p.tiles[2 + p.max_tiles + tile];
   const SlotDesc* d = p.desc + slot;
   const int cnt = min(kPfToksMx, d->n_tok - first);
-  if (cnt <= 64) mx_down_tile<64>(p, d, first, cnt, rt, mx_lds);
+  if (mx_narrow(p, cnt)) mx_down_tile<64>(p, d, first, cnt, rt, mx_lds);
   else mx_down_tile<kPfToksMx>(p, d, first, cnt, rt, mx_lds);
 }
 
@@ -1164,6 +1174,7 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   const bool few = __syncthreads_count(rows > 0 && rows <= narrow) < min_narrow;
   const bool wide = narrow > 0 && !few && (on || !mx);
   const int cnt = wide && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;
+  const int small = __syncthreads_count(cnt > 0 && rows - (cnt - 1) * rtoks <= 64);   // tiles of at most 64 rows
   int incl = cnt;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
@@ -1190,7 +1201,7 @@ __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ 
   if (t == 0) {
     tiles[0] = total + sh;
     tiles[1] = total;
-    tiles[2 + 2 * max_tiles] = (on ? kTilesMx : 0) | (wide ? kTilesWide : 0);
+    tiles[2 + 2 * max_tiles] = (on ? kTilesMx : 0) | (wide ? kTilesWide : 0) | (2 * small < total ? kTilesFull : 0);
   }
 }
 
