@@ -1238,15 +1238,18 @@ int prefill_narrow_rows(const dsk_moe_desc& d) {
 
 // The shared expert's GEMM tiles are one block per 128 features and 256 tokens:
 // 16 blocks at 200 tokens, 107 us beside idle CUs for its gate/up (59 for its
-// down).  Up to 512 tokens it runs as blocks of the wide kernels instead (64
+// down).  Up to 800 tokens (q3: 512) it runs as blocks of the wide kernels instead (64
 // tokens and 64 features each), under the routed slots' stream (q3: where the
-// narrow slots do, its output rounded to bf16 as the GEMM tiles write it).
+// narrow slots do, its output rounded to bf16 as the GEMM tiles write it).  Layer at
+// H 4096, I 2048, top-8 of 256, with the GEMM tiles and so, even and skewed routing: 600
+// tokens 978 and 906, 487 and 469 us; 800 tokens 1034 and 986, 555 and 540; 1000 tokens
+// 1097 and 1067, 650 and 649; 1200 tokens 1155 and 1156, 733 and 780.
 static int prefill_min_narrow(const dsk_moe_desc& d) {
   return d.quant == DSK_QUANT_Q3 || !prefill_shared_wide(d) ? (2 * 256 * 128 + d.inter - 1) / d.inter : 0;
 }
 
 bool prefill_shared_wide(const dsk_moe_desc& d) {
-  return prefill_narrow_rows(d) > 0 && d.inter_shared > 0 && d.tokens <= 512;
+  return prefill_narrow_rows(d) > 0 && d.inter_shared > 0 && d.tokens <= (d.quant == DSK_QUANT_Q3 ? 512 : 800);
 }
 
 hipError_t launch_pf_planes(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s) {
