@@ -384,6 +384,10 @@ int dsk::forward_layer(const dsk_moe_desc* d, const void* x, const void* gate_w,
   a.scores = scores; a.bias = gate_b;
   a.route = DecodeRoute{idx_buf, w_buf, ra.out.desc, active, ra.rowmap, ra.out.xrow, ra.out.wrow, rank};
   const bool decode = decode_pipeline(*d);
+  if (!decode && d->tokens > kFusedMaxTokens && prefill_gemm(*d) && dispatch_writes_tiles(d->n_experts)) {
+    ra.out.pf = prefill_tiles(*d, reinterpret_cast<int32_t*>(ws + L.pf_tiles));
+    a.tiles_ready = 1;
+  }
   // the unfused top-k kernel writes x in the form the gate/up that follows reads (FP8
   // planes for FP4 experts, the factored q3 form for q3 experts; prefill: its MX planes)
   if (!decode && d->tokens > kFusedMaxTokens && !rn && d->x_dtype == DSK_DTYPE_BF16) {

@@ -11,7 +11,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const int32_t* __restrict__ i
                                                    const dsk_expert_ptrs* __restrict__ table,
                                                    DispatchOut o) {
   extern __shared__ int32_t lds[];
-  dispatch_block(idx, N, E, k, nbits, wflat, table, o, lds);
+  dispatch_block<true>(idx, N, E, k, nbits, wflat, table, o, lds);
 }
 
 // Multi-block form.  Block b takes positions [b C, (b + 1) C) (C =
@@ -92,6 +92,7 @@ __global__ __launch_bounds__(1024) void k_disp_scan(int n_seg, int E, const dsk_
     tot_a += wflag[w];
   }
   const int xc = off_c + ic - cnt, xa = off_a + ia - act;
+  bool ok = true;
   if (e < E) {
     o.offsets[e] = xc;
     if (act) {
@@ -105,6 +106,7 @@ __global__ __launch_bounds__(1024) void k_disp_scan(int n_seg, int E, const dsk_
         d.p[6] = t.w2; d.p[7] = t.s2; d.p[8] = t.b2;
         d.pad2 = nullptr;
         o.desc[xa] = d;
+        ok = slot_aligned16(d);
       }
     }
   }
@@ -112,6 +114,7 @@ __global__ __launch_bounds__(1024) void k_disp_scan(int n_seg, int E, const dsk_
     o.offsets[E] = tot_c;
     o.active[0] = tot_a;
   }
+  if (o.pf.tiles) prefill_tiles_block(o.pf, xa, cnt, ok);
 }
 
 // 3. the block counts its waves again, and each wave walks its 128 positions

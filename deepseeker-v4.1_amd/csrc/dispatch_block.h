@@ -16,7 +16,7 @@
 // active expert and the token and route weight of every dispatch row.
 #pragma once
 
-#include "dsk_internal.h"
+#include "prefill_tiles.h"
 
 namespace dsk {
 
@@ -65,7 +65,9 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 // Chunks of 64 positions whose loads a wave issues together.
 constexpr int kDispBatch = 8;
 
-// LDS needed: (S * E + E + 32) int32.
+// LDS needed: (S * E + E + 32) int32.  kTiles: with the prefill tile list (o.pf) if it
+// is asked for, by blocks of 1024 threads (dispatch_writes_tiles).
+template <bool kTiles = false>
 __device__ __forceinline__ void dispatch_block(const int32_t* __restrict__ idx, int N, int E, int k,
                                                int nbits, const float* __restrict__ wflat,
                                                const dsk_expert_ptrs* __restrict__ table,
@@ -119,6 +121,8 @@ __device__ __forceinline__ void dispatch_block(const int32_t* __restrict__ idx, 
   int off_c = 0, off_a = 0;
   for (int w = 0; w < wave; ++w) { off_c += wsum[w]; off_a += wflag[w]; }
   int xc = off_c + ic - run_cnt, xa = off_a + ia - run_act;
+  int slot = 0, rows = 0;   // kTiles: this thread's slot
+  bool ok = true;
   for (int e = e_beg; e < e_end; ++e) {
     const int c = base[e];
     o.offsets[e] = xc;
@@ -134,6 +138,11 @@ __device__ __forceinline__ void dispatch_block(const int32_t* __restrict__ idx, 
         d.p[6] = t.w2; d.p[7] = t.s2; d.p[8] = t.b2;
         d.pad2 = nullptr;
         o.desc[xa] = d;
+        if constexpr (kTiles) {
+          slot = xa;
+          rows = c;
+          ok = slot_aligned16(d);
+        }
       }
       ++xa;
     }
@@ -142,6 +151,9 @@ __device__ __forceinline__ void dispatch_block(const int32_t* __restrict__ idx, 
   if (tid == nthr - 1) {
     o.offsets[E] = xc;
     o.active[0] = xa;
+  }
+  if constexpr (kTiles) {
+    if (o.pf.tiles) prefill_tiles_block(o.pf, slot, rows, ok);
   }
   __syncthreads();
 

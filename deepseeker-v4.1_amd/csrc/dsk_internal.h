@@ -113,14 +113,24 @@ struct SlotDesc {
 };
 static_assert(sizeof(SlotDesc) == 96, "SlotDesc layout");
 
+// The prefill GEMM's tile list (prefill_tiles_block; null: none).
+struct PrefillTiles {
+  int32_t* tiles;            // [3 + 2 max_tiles]
+  int T, with_shared, max_tiles, mx, narrow, min_narrow;
+};
+
 struct DispatchOut {
   int32_t* counts; int32_t* offsets; int32_t* perm; int32_t* rank; int32_t* active;
   SlotDesc* desc;            // [E] or null
   int32_t* xrow;             // [T*k] token of each dispatch row, or null
   float* wrow;               // [T*k] route weight of each dispatch row
   int32_t* hist = nullptr;   // [blocks][E] per-block counts of the multi-block form, or null
+  PrefillTiles pf = {};      // the tile list, written by the block that writes desc (dispatch_writes_tiles)
 };
 
+// The block that writes the descriptors has a thread per slot (it then also writes
+// the prefill tile list, a launch of 5 us less).
+inline bool dispatch_writes_tiles(int E) { return E <= 512; }
 // From this many (token, slot) positions, and with a histogram area, the
 // dispatch runs as three kernels over blocks of kDispBlockPositions.
 constexpr int kDispMultiMin = 8192;
@@ -303,6 +313,7 @@ struct ExpertsArgs {
   float* scores; const float* bias;
   DecodeRoute route;
   int x_planes_ready;        // the routing kernels already wrote x's FP8 planes / q3 form (RouteArgs::xp)
+  int tiles_ready;           // the dispatch wrote the prefill tile list (DispatchOut::pf)
 };
 
 // Opens the gate/up, down and combine stages as it launches them.
@@ -349,6 +360,7 @@ struct PrefillArgs {
   char* ws;
   float* rows_out;           // per-row outputs instead of the workspace's (or null)
   int x_planes_ready;        // the routing kernels already wrote x's FP8 planes
+  int tiles_ready;           // the dispatch wrote the tile list
   const ExpertsArgs* call;   // the call's arguments (the wide kernels')
 };
 hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, const PrefillArgs& a,
@@ -419,6 +431,8 @@ bool grouped_wide_q3(const dsk_moe_desc& d);
 // Prefill layers: slots of up to this many dispatch rows run on the wide
 // kernels instead of the GEMM tiles (0: none), and whether the shared expert does.
 int prefill_narrow_rows(const dsk_moe_desc& d);
+// The tile list of a prefill layer at `tiles`.
+PrefillTiles prefill_tiles(const dsk_moe_desc& d, int32_t* tiles);
 bool prefill_shared_wide(const dsk_moe_desc& d);
 // The grouped q3 gate/up takes x scaled for the factored product, with its
 // 64-group sums (Workspace::xp).

@@ -654,7 +654,7 @@ hipError_t launch_experts(const dsk_moe_desc& d, const Workspace& L, const Exper
   const uint16_t* xb_lo = nullptr;
   if (prefill_gemm(d)) {
     PrefillArgs pa{desc, a.active, xrow, wrow, a.x, a.ws1, a.ws3, a.ws2, a.ws, a.rows_out, a.x_planes_ready,
-                   &a};
+                   a.tiles_ready, &a};
     if ((e = launch_experts_prefill(d, L, pa, s, repeat)) != hipSuccess) return e;
     return a.rows_out ? hipSuccess : launch_combine(d, L, a, s, repeat);
   }

@@ -1198,11 +1198,12 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     up_shared(p, b, lds_g);
     return;
   }
+  if (p.on && !(*p.on & kTilesWide)) return;   // (first: an empty launch is as long as its loads)
   const int rb = b - p.up_shared, n_act = p.active[0];
   const bool few = CT == 1 && p.few > 0 && wide_few_mode(n_act, n_act * p.up_groups + p.up_shared, p.T * p.k);
   const int groups = few ? kWfKS * p.up_groups : p.up_groups;
   const int slot = rb / groups, grp = rb % groups;
-  if (slot >= n_act || (p.on && !(*p.on & kTilesWide))) return;
+  if (slot >= n_act) return;
   const SlotDesc* d = p.desc + slot;
   const int n = d->n_tok, base = d->tok_base;
   if (n > p.max_rows) return;
@@ -1231,11 +1232,12 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     down_shared(p, b, lds_g);
     return;
   }
+  if (p.on && !(*p.on & kTilesWide)) return;   // (first: an empty launch is as long as its loads)
   const int rb = b - p.dn_shared, n_act = p.active[0];
   const bool few = CT == 1 && p.few > 0 && wide_few_mode(n_act, n_act * p.dn_groups + p.dn_shared, p.T * p.k);
   const int groups = few ? kWfKS * p.dn_groups : p.dn_groups;
   const int slot = rb / groups, grp = rb % groups;
-  if (slot >= n_act || (p.on && !(*p.on & kTilesWide))) return;
+  if (slot >= n_act) return;
   const SlotDesc* d = p.desc + slot;
   const int n = d->n_tok, base = d->tok_base;
   if (n > p.max_rows) return;
@@ -1634,9 +1636,9 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     up_shared(p, b, lds_g);
     return;
   }
+  if (p.on && !(*p.on & kTilesWide)) return;
   const int rb = b - p.up_shared, first = rb / p.up_groups, grp = rb % p.up_groups;
   const int n_act = p.active[0];
-  if (p.on && !(*p.on & kTilesWide)) return;
   for (int slot = first; slot < n_act; slot += p.slot_step) {
     const SlotDesc* d = p.desc + slot;
     const int n = d->n_tok, base = d->tok_base;
@@ -1656,9 +1658,9 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     down_shared(p, b, lds_g);
     return;
   }
+  if (p.on && !(*p.on & kTilesWide)) return;
   const int rb = b - p.dn_shared, first = rb / p.dn_groups, grp = rb % p.dn_groups;
   const int n_act = p.active[0];
-  if (p.on && !(*p.on & kTilesWide)) return;
   for (int slot = first; slot < n_act; slot += p.slot_step) {
     const SlotDesc* d = p.desc + slot;
     const int n = d->n_tok, base = d->tok_base;

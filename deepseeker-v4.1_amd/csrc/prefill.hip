@@ -44,6 +44,7 @@
 // with the row tiles of one token tile adjacent, which keeps that tile's
 // activations in the XCD's L2 while they are reused.
 #include "mx.h"
+#include "prefill_tiles.h"
 
 namespace dsk {
 namespace {
@@ -284,11 +285,6 @@ __device__ __forceinline__ void wait_barrier() {
 }
 
 __device__ __forceinline__ int swz(int r, int c) { return c ^ ((r >> 1) & 7); }
-
-// The DMA loads read 16-byte pieces at 16-byte steps from the given bases.
-__device__ __forceinline__ bool aligned16(const void* a, const void* b) {
-  return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
-}
 
 // Stage chunk (row, chunk) loaded by lane i of load j of wave w, for 128-byte
 // rows spread over 4 loads per lane: LDS position p = (4 w + j) 64 + i.
@@ -559,7 +555,6 @@ __device__ __forceinline__ void mx_mma(const MxOps<AF>& o, int pl, int n_ct, f32
 // and 824.
 constexpr int kMxThreads = 256;
 constexpr int kMxRound = 2 * 256;   // units of a round
-constexpr int kPfToksMx = 128;   // dispatch rows of an MX tile
 
 template <int TOK>
 struct DmaMx {
@@ -1146,63 +1141,11 @@ __global__ __launch_bounds__(256) void k_pf_planes(const uint16_t* __restrict__ 
   pf_planes_chunk(x, H, c, true, q, ex);
 }
 
-// Tile list from the dispatch descriptors (one block of 1024 threads; one
-// thread per active expert slot, E <= 1024): routed tiles, then the shared
-// expert's tiles of kPfToks tokens.  The routed tiles run on the MX kernels
-// (kPfToksMx rows each) when the layer allows it (mx) and every active
-// slot's six FP4 arrays are 16-byte aligned (the LDS DMA's pieces), else on
-// the 8-wave kernels (kPfToks rows each).  Slots of at most `narrow` rows are
-// the wide kernels' (of FP4 layers: with the MX kernels) when at least min_narrow
-// slots are that small.  with_shared: the shared expert's tiles (2: only if the
-// narrow slots stay here; it is the wide kernels' else).
-// tiles[2 + 2 max_tiles]: the switch word.
 __global__ __launch_bounds__(1024) void k_pf_tiles(const SlotDesc* __restrict__ desc,
-                                                   const int32_t* __restrict__ active, int E, int T,
-                                                   int with_shared, int max_tiles, int mx, int narrow, int min_narrow,
-                                                   int32_t* __restrict__ tiles) {
-  __shared__ int32_t wsum[16];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int n_act = min(active[0], E);
-  bool ok = true;
-  if (mx && t < n_act) {
-    const SlotDesc& d = desc[t];
-    ok = aligned16(d.p[0], d.p[1]) && aligned16(d.p[3], d.p[4]) && aligned16(d.p[6], d.p[7]);
-  }
-  const bool on = mx && __syncthreads_and(ok ? 1 : 0);
-  const int rtoks = on ? kPfToksMx : kPfToks;
-  const int rows = t < n_act ? desc[t].n_tok : 0;
-  const bool few = __syncthreads_count(rows > 0 && rows <= narrow) < min_narrow;
-  const bool wide = narrow > 0 && !few && (on || !mx);
-  const int cnt = wide && rows <= narrow ? 0 : (rows + rtoks - 1) / rtoks;
-  const int small = __syncthreads_count(cnt > 0 && rows - (cnt - 1) * rtoks <= 64);   // tiles of at most 64 rows
-  int incl = cnt;
-#pragma unroll
-  for (int s = 1; s < 64; s <<= 1) {
-    const int v = __shfl_up(incl, s, 64);
-    if (lane >= s) incl += v;
-  }
-  if (lane == 63) wsum[wave] = incl;
-  __syncthreads();
-  int base = 0, total = 0;
-  for (int w = 0; w < 16; ++w) {
-    base += w < wave ? wsum[w] : 0;
-    total += wsum[w];
-  }
-  const int off = base + incl - cnt;
-  for (int j = 0; j < cnt; ++j) {
-    tiles[2 + off + j] = t;
-    tiles[2 + max_tiles + off + j] = j * rtoks;
-  }
-  const int sh = with_shared == 1 || (with_shared && !wide) ? (T + kPfToks - 1) / kPfToks : 0;
-  for (int j = t; j < sh; j += 1024) {
-    tiles[2 + total + j] = -1;
-    tiles[2 + max_tiles + total + j] = j * kPfToks;
-  }
-  if (t == 0) {
-    tiles[0] = total + sh;
-    tiles[1] = total;
-    tiles[2 + 2 * max_tiles] = (on ? kTilesMx : 0) | (wide ? kTilesWide : 0) | (2 * small < total ? kTilesFull : 0);
-  }
+                                                   const int32_t* __restrict__ active, int E, PrefillTiles o) {
+  const int t = threadIdx.x;
+  const bool have = t < min(active[0], E);
+  prefill_tiles_block(o, t, have ? desc[t].n_tok : 0, !have || !o.mx || slot_aligned16(desc[t]));
 }
 
 }  // namespace
@@ -1252,6 +1195,12 @@ bool prefill_shared_wide(const dsk_moe_desc& d) {
   return prefill_narrow_rows(d) > 0 && d.inter_shared > 0 && d.tokens <= (d.quant == DSK_QUANT_Q3 ? 512 : 800);
 }
 
+PrefillTiles prefill_tiles(const dsk_moe_desc& d, int32_t* tiles) {
+  const bool sh_wide = prefill_shared_wide(d);
+  return {tiles, d.tokens, d.inter_shared == 0 ? 0 : !sh_wide ? 1 : d.quant == DSK_QUANT_Q3 ? 2 : 0, prefill_max_tiles(d),
+          prefill_mx(d) ? 1 : 0, prefill_narrow_rows(d), prefill_min_narrow(d)};
+}
+
 hipError_t launch_pf_planes(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a, hipStream_t s) {
   const int64_t chunks = static_cast<int64_t>(d.tokens) * (d.hidden / 8);
   uint8_t* xp = reinterpret_cast<uint8_t*>(a.ws + L.xp);
@@ -1272,8 +1221,7 @@ hipError_t launch_experts_prefill(const dsk_moe_desc& d, const Workspace& L, con
   const bool sh_wide = prefill_shared_wide(d);
   const WideCall wide{2, narrow, tiles + 2 + 2 * max_tiles, prefill_rows_bf16(d, a.rows_out) ? 1 : 0, sh_wide,
                       q3};
-  launch_kernel(k_pf_tiles, 1, 1024, 0, s, a.desc, a.active, d.n_experts, T, Is == 0 ? 0 : !sh_wide ? 1 : q3 ? 2 : 0,
-                max_tiles, mx ? 1 : 0, narrow, prefill_min_narrow(d), tiles);
+  if (!a.tiles_ready) launch_kernel(k_pf_tiles, 1, 1024, 0, s, a.desc, a.active, d.n_experts, prefill_tiles(d, tiles));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
 

@@ -223,3 +223,42 @@ def test_skewed_fp4_prompt(T, E, k, hot, I):
     need = -(-2 * 256 * 128 // I)
     assert (r["counts"][:hot] == T).all()
     assert narrow >= need if E == 128 else narrow < need
+
+
+def test_tile_list_of_the_dispatch():
+    """The tile list written by the multi-block dispatch (8192 positions and more) is the
+    one that the entry point with a routing of its own makes: the same rows."""
+    from dsk_moe.layer import experts_forward
+    print("tile list", flush=True)
+    spec = L.LayerSpec(H=512, E=40, k=4, I=512, I_shared=128)
+    for T in (2080, 700):
+        d = synth.make_layer(spec, 660, T, zipf_s=0.5)
+        bank, shared, x = to_bank(d["bank"]), to_shared(d["shared"]), d["x"].to(DEV)
+        idx, w = torch.empty((T, spec.k), dtype=torch.int32, device=DEV), torch.empty((T, spec.k), device=DEV)
+        layer = dsk_moe.MoELayer(d["gate_w"].to(DEV), d["gate_b"].to(DEV), bank, shared, spec.k)
+        out = layer(x, idx=idx, w=w)
+        assert torch.equal(out, experts_forward(x, idx, w, bank, shared))
+        r = L.moe_forward(d["x"], None, None, d["bank"], d["shared"], spec, routing=(idx.cpu().numpy(), w.cpu().numpy(), None, None))
+        assert_layer_close(out.cpu().float(), r["y_ref"])
+
+
+@pytest.mark.parametrize("role,T", [("w1", 150), ("w2", 150), ("w3", 600)])
+def test_prompt_with_arrays_at_eight_bytes(role, T):
+    """FP4 codes of one role off 16-byte alignment: the register-staged GEMM loop takes
+    every slot, narrow ones too, beside the shared expert's wide blocks."""
+    print(f"arrays at eight bytes {role} T={T}", flush=True)
+    spec = L.LayerSpec(H=1024, E=48, k=2, I=768, I_shared=256)
+    d = synth.make_layer(spec, 680, T)
+    r = L.moe_forward(d["x"], d["gate_w"], d["gate_b"], d["bank"], d["shared"], spec)
+    bank = to_bank(d["bank"])
+    codes, scales = bank.roles[role]
+    raw = torch.empty(codes.numel() + 8, dtype=torch.uint8, device=DEV)
+    off = raw[8:].view(codes.shape)
+    off.copy_(codes)
+    assert off.data_ptr() % 16 == 8
+    roles = dict(bank.roles)
+    roles[role] = (off, scales)
+    layer = dsk_moe.MoELayer(d["gate_w"].to(DEV), d["gate_b"].to(DEV), dsk_moe.ResidentBank("fp4", roles),
+                             to_shared(d["shared"]), spec.k)
+    out = layer(d["x"].to(DEV)).cpu()
+    assert_layer_close(out.float(), r["y_ref"])
