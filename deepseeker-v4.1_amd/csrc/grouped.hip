@@ -1957,6 +1957,15 @@ static bool rows_on_tiles(const dsk_moe_desc& d) {
   return d.quant == DSK_QUANT_FP4 ? !wide_own_space(d) : d.hidden % 4096 == 0 && d.inter % 512 == 0;
 }
 
+// The factored q3 down keeps its column tiles to 27 tokens, the gate/up beside it only
+// below 24 (q3_tiles): at H 4096, I 2048, top-8 of 256 and 24 tokens the gate/up takes
+// 281 and 277 us (skewed routing 90 and 66) in tiles and wide, the down 142 and 170 (52
+// and 44).  Layers with tiles, wide and so: 24 tokens 415, 418 and 402 us (skewed 152,
+// 133 and 134), 26 tokens 432, 435 and 419; 28 tokens, 459 and 455, are faster wide.
+static bool q3_down_tiles(const dsk_moe_desc& d) {
+  return d.quant == DSK_QUANT_Q3 && d.hidden % 4096 == 0 && down_q3f(d) && d.tokens < 28;
+}
+
 hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, const ExpertsArgs& a,
                                   const SlotDesc* desc, const int32_t* xrow, const float* wrow, hipStream_t s,
                                   int repeat) {
@@ -1970,6 +1979,7 @@ hipError_t launch_experts_grouped(const dsk_moe_desc& d, const Workspace& L, con
       if ((e = launch_wide_up(d, L, a, desc, xrow, wrow, w, s)) != hipSuccess) return e;
     }
     if ((e = stage_open(kStageDown)) != hipSuccess) return e;
+    if (q3_down_tiles(d)) return grouped_down(d, grouped_args(d, L, a, desc, xrow, wrow), s, repeat);
     for (int r = 0; r < repeat; ++r)
       if ((e = launch_wide_down(d, L, a, desc, w, s)) != hipSuccess) return e;
     return e;

@@ -61,8 +61,8 @@ def test_wide_float32_pairs(T, hot, H, I):
                                        (40, 4, 5120, 512), (150, 0, 1024, 768), (300, 4, 512, 1024)])
 def test_wide_q3(T, hot, H, I):
     """q3: sets of eight rows and a part of one, passes of sixteen, one to three blocks
-    after the last superblock, the decode pipeline's form (1, 2, 4 tokens), and, from 128
-    tokens, slots beside the GEMM tiles (300: none of them narrow)."""
+    after the last superblock, the decode pipeline's form (1, 2, 4 tokens), and from 128
+    tokens GEMM tiles alone (more than 16 rows a slot on average)."""
     _check(L.LayerSpec(H=H, E=16, k=4, I=I, I_shared=256, quant=L.QUANT_Q3), T, hot, 410 + T, f"q3 H {H} I {I}")
 
 
@@ -262,3 +262,23 @@ def test_prompt_with_arrays_at_eight_bytes(role, T):
                              to_shared(d["shared"]), spec.k)
     out = layer(d["x"].to(DEV)).cpu()
     assert_layer_close(out.float(), r["y_ref"])
+
+
+@pytest.mark.parametrize("T", [23, 24, 27, 28])
+def test_wide_q3_down_beside_column_tiles(T):
+    """H 4096: column tiles to 23 tokens, the wide gate/up with the tiles' down to 27, then
+    both wide."""
+    _check(L.LayerSpec(H=4096, E=12, k=3, I=512, I_shared=128, quant=L.QUANT_Q3), T, 1, 700 + T, "q3 down")
+
+
+@pytest.mark.parametrize("T,hot,wide", [(130, 0, True), (130, 1, True), (200, 4, False)])
+def test_wide_q3_prompt_after_the_last_superblock(T, hot, wide):
+    """q3 from 128 tokens with two blocks of H and three of I after their last superblock:
+    enough slots of at most 16 rows (the wide kernels, beside GEMM tiles for the hot
+    expert), and too few."""
+    spec = L.LayerSpec(H=768, E=64, k=4, I=1408, I_shared=128, quant=L.QUANT_Q3)
+    r = _check(spec, T, hot, 720 + T, f"q3 prompt hot={hot}")
+    narrow = int(((r["counts"] > 0) & (r["counts"] <= 16)).sum())
+    assert T * spec.k <= 16 * spec.E
+    assert (narrow >= -(-2 * 256 * 128 // spec.I)) == wide
+    assert not hot or int(r["counts"].max()) > 16
