@@ -467,7 +467,10 @@ __device__ __forceinline__ void gs_walk(int nb, MM mm, LW ldw, LX ldx, SX stx, M
 // 2i + 1 take row tile 4b + i of w1 (gate) and of w3 (up), so that a wave
 // holds one role's accumulators and a ring of four weight batches; the up
 // wave hands its sums to the gate wave through LDS for SwiGLU.
-// kPair: x as a bf16 hi / lo pair (two planes staged and multiplied, as in the down).
+// kPair: x as a bf16 hi / lo pair (two planes staged and multiplied, as in the down),
+// a step's products in a sum of their own (see wide_mul_pair: one chain over K cost
+// float32 layers 0.3 to 0.8 % of their error: 20 tokens at H 4096 4.309e-6, 4.284e-6
+// so, 4.289e-6 in the general kernels).
 template <bool kPair>
 __device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, int first, int step, uint16_t* lds) {
   constexpr int NB = kPair ? 2 : 3, NX = kPair ? 2 : 1;
@@ -493,8 +496,14 @@ __device__ __forceinline__ void up_shared_wide(const GroupedArgs& p, int b, int 
       for (int c = 0; c < kGsCT; ++c)
         if (c < nct) {
           const uint16_t* x = lds + buf * NX * kGsPlane + (c * 16 + r16) * kGsStride;
-          mma_block(w[i], x, g4 * 32, true, acc[c]);
-          if constexpr (kPair) mma_block(w[i], x + kGsPlane, g4 * 32, true, acc[c]);
+          if constexpr (kPair) {
+            f32x4 st = {0.f, 0.f, 0.f, 0.f};
+            mma_block(w[i], x, g4 * 32, true, st);
+            mma_block(w[i], x + kGsPlane, g4 * 32, true, st);
+            acc[c] += st;
+          } else {
+            mma_block(w[i], x, g4 * 32, true, acc[c]);
+          }
         }
     };
     auto ldw = [&](int i, int kb) { load_raw_nc(w[i], W, row, K, kb * 128 + g4 * 32); };
@@ -552,6 +561,8 @@ __device__ __forceinline__ void up_shared(const GroupedArgs& p, int b, uint16_t*
 // Down of the shared expert over more than kGNC tokens, as up_shared_wide:
 // block b's eight waves each take one row tile of w2 (16 output rows) over
 // K = Is, the h planes (hi, lo) of up to kGsCols tokens staged per K block.
+// kPair: as there.
+template <bool kPair>
 __device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, int first, int step, uint16_t* lds) {
   constexpr int NB = 2;
   const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -573,8 +584,10 @@ __device__ __forceinline__ void down_shared_wide(const GroupedArgs& p, int b, in
       for (int c = 0; c < kGsCT; ++c) {
         if (c < nct) {
           const int o = (c * 16 + r16) * kGsStride;
-          mma_block(w[i], hi + o, g4 * 32, true, acc[c]);
-          mma_block(w[i], hi + kGsPlane + o, g4 * 32, true, acc[c]);
+          f32x4 st = kPair ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[c];
+          mma_block(w[i], hi + o, g4 * 32, true, st);
+          mma_block(w[i], hi + kGsPlane + o, g4 * 32, true, st);
+          acc[c] = kPair ? acc[c] + st : st;
         }
       }
     };
@@ -707,7 +720,7 @@ __device__ __forceinline__ void down_block(const GroupedArgs& p, LoadW load_w, W
 // Down of the shared expert, block b (up_shared).
 __device__ __forceinline__ void down_shared(const GroupedArgs& p, int b, uint16_t* lds) {
   if (!p.sh_tiles) {
-    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds);
+    down_shared_wide<false>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds);
     return;
   }
   const int rt = b * kDI + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kDKS;
@@ -1388,7 +1401,7 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   uint8_t* lds = reinterpret_cast<uint8_t*>(lds_g);
   const int b = static_cast<int>(blockIdx.x);
   if (b < p.dn_shared) {
-    down_shared_wide(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
+    down_shared_wide<true>(p, b / p.sh_tg, (b % p.sh_tg) * kGsCols, p.sh_tg * kGsCols, lds_g);
     return;
   }
   const int rb = b - p.dn_shared, slot = rb / p.dn_groups, grp = rb % p.dn_groups;
