@@ -9,12 +9,13 @@
 // The wide kernels (k_up_wide, k_down_wide and their float32 and q3 forms)
 // take most shapes: a block's waves walk all of K of one slot together with the
 // weights straight in registers and all of the slot's rows of a pass staged.
-// The others (k_up_grouped, k_down_grouped: FP4 with H or I out of the wide
-// kernels' range, q3 below one superblock or 24 tokens, the decode pipeline's
-// down at three tokens) are column tiles: a block takes one slot (an active expert, or the
-// shared expert as a pseudo-slot over all T tokens) and a group of row tiles;
-// it walks the slot's dispatch rows in column tiles of kGNC.  For each column tile the block gathers only that
-// tile's activation rows into LDS (x for gate/up, the h planes for down), the
+// The others (k_up_grouped, k_down_grouped: FP4 with H out of the wide kernels'
+// range, of little work, or whose rows leave in float32; q3 below one superblock or
+// 24 tokens; the decode pipeline's down at three tokens; the shared expert of up to
+// eight tokens) are column tiles: a block takes one slot (an active expert, or the
+// shared expert as a pseudo-slot over all T tokens) and a group of row tiles; it
+// walks the slot's dispatch rows in column tiles of kGNC.  For each column tile the
+// block gathers only that tile's activation rows into LDS (x for gate/up, the h planes for down), the
 // waves issue their first weight batches behind those loads (not in front of
 // them, where the LDS stores would wait for the weights too), and each wave
 // then multiplies its K range; K ranges are added in a fixed
@@ -1192,7 +1193,7 @@ __device__ __forceinline__ void down_wide_few(const GroupedArgs& p, int slot, in
 // ---------------------------------------------------------------- the wide FP4 kernels
 // Column tiles of a pass and steps in flight.  Of one column tile three steps:
 // two took 289 us of gate/up at 64 tokens (H 4096, top-8 of 256) against 259,
-// four 307 (12 KB in flight per wave then overrun the XCD's L2: a 128-byte row
+// four 307 (16 KB in flight per wave then overrun the XCD's L2: a 128-byte row
 // piece is two loads).  Two column tiles leave registers for two steps; four
 // spill.
 constexpr int kWdMaxCT = 2;
@@ -1370,12 +1371,11 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
   const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
   const int rt = grp * kWdWaves + wave, K = p.H;
-  const bool rok = rt < p.I / 16;
   const uint8_t* const W[2] = {static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 0)),
                                static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3))};
   const uint8_t* const S[2] = {static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 1)),
                                static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 4))};
-  const uint32_t row0 = rok ? static_cast<uint32_t>(rt * 16) : 0u;
+  const uint32_t row0 = static_cast<uint32_t>(rt * 16);
   const uint32_t c0 = (row0 + r16) * static_cast<uint32_t>(K / 2) + static_cast<uint32_t>(g4 * 16);
   const uint32_t s0 = row0 * static_cast<uint32_t>(K / 32);
   const uint32_t co[2] = {c0, c0}, so[2] = {s0, s0};
@@ -1383,7 +1383,7 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
     const int m = min(n - r, 16);
     f32x4 acc[2];
     wide_mul_pair(W, S, co, so, p.x, p.x_lo, K, m, [&](int i) { return p.xrow[base + r + i]; }, lds, acc);
-    if (rok && r16 < m) {
+    if (r16 < m) {
       const int64_t row = base + r + r16;
       const float wr = p.wrow[row];
       uint16_t hh[4], hl[4];
@@ -1441,9 +1441,9 @@ __global__ __launch_bounds__(kWdWaves * 64) __attribute__((amdgpu_waves_per_eu(4
 // a block more than the 128 + 8q form.  Up to 16 dispatch rows a pass.
 //
 // Bound by the weight stream and, near it, by the masking.  Gate/up and down at H 4096, top-8 of 256
-// (against blocks of eight K ranges and eight rows a pass): 16 tokens 226 -> 220 and
-// 121 -> 124 us, 64 tokens 416 -> 371 and 212 -> 210, 100 tokens 507 -> 426 and 262
-// -> 256. At H 5120, I 2304, top-6 of 384, where the other kernels dequantise every
+// (against blocks of eight K ranges and eight rows a pass): 64 tokens 416 -> 371 and
+// 212 -> 210 us, 100 tokens 507 -> 426 and 262 -> 256 (at 16 tokens, 226 -> 220 and 121 ->
+// 124 with even routing, skewed routing lost 3 %: q3_tiles).  At H 5120, I 2304, top-6 of 384, where the other kernels dequantise every
 // weight: 24 tokens 696 -> 361 and 369 -> 199, 6 tokens 367 -> 108 and 121 -> 72.
 constexpr int kWqStep = 512;                                // K of a step: a superblock
 constexpr int kWqNB = 2;                                    // steps in flight
@@ -1585,8 +1585,7 @@ __device__ __forceinline__ void up_wide_q3(const GroupedArgs& p, int slot, int g
   const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
   const int role = wave & 1, pair = wave >> 1, rt = grp * kWqUpTiles + pair, K = p.H;
-  const bool rok = rt < p.I / 16;
-  const uint32_t row = rok ? static_cast<uint32_t>(rt * 16 + r16) : 0u;
+  const uint32_t row = static_cast<uint32_t>(rt * 16 + r16);
   const uint8_t* W = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3 * role));
   const uint8_t* S = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3 * role + 1));
   const uint8_t* B = static_cast<const uint8_t*>(desc_ptr(p.desc, slot, 3 * role + 2));
@@ -1601,7 +1600,7 @@ __device__ __forceinline__ void up_wide_q3(const GroupedArgs& p, int slot, int g
       for (int i = 0; i < 2; ++i) xch[pair][s2][i][lane] = acc[s2][i];
   }
   __syncthreads();
-  if (!role && rok) {
+  if (!role) {
 #pragma unroll
     for (int s2 = 0; s2 < NS; ++s2)
 #pragma unroll
@@ -2086,10 +2085,10 @@ GroupedArgs wide_args(const dsk_moe_desc& d, const Workspace& L, const ExpertsAr
   p.y_bf16 = w.y_bf16;
   p.sh_tiles = wide_shared_tiles(d) && d.x_dtype == DSK_DTYPE_BF16 ? 1 : 0;
   p.sh_tg = (d.tokens + kGsCols - 1) / kGsCols;
-  p.up_groups = (d.inter / 16 + kWdWaves - 1) / kWdWaves;
+  p.up_groups = d.inter / 16 / kWdWaves;
   p.dn_groups = d.hidden / 256;
   if (d.quant == DSK_QUANT_Q3) {
-    p.up_groups = (d.inter / 16 + kWqUpTiles - 1) / kWqUpTiles;
+    p.up_groups = d.inter / 16 / kWqUpTiles;
     p.dn_groups = d.hidden / 128;
   }
   // q3 under the device switch: blocks for 64 slots, each walking every 64th.  Skewed

@@ -1169,7 +1169,7 @@ int prefill_max_tiles(const dsk_moe_desc& d) {
 // Few such slots (skewed routing) are better left to the tiles (they fill the
 // same launch; the wide kernels' walk over K takes its 20 to 40 us and more however few
 // blocks it has: q3, 128 tokens on 15 experts, 220 us a layer without, 288 with; FP4,
-// 600 tokens on 15, 476 and 514), so k_pf_tiles counts them: from two blocks a CU on
+// 600 tokens on 15, 476 and 514), so the tile list counts them: from two blocks a CU on
 // (prefill_min_narrow).  FP4 prompts whose shared expert runs there have the launch
 // anyway, and keep them.
 int prefill_narrow_rows(const dsk_moe_desc& d) {

@@ -180,11 +180,12 @@ def test_wide_shared_expert_of_few_tokens(quant, H, I, Is, T):
 
 
 @pytest.mark.parametrize("H,I,Is,T,k", [(1024, 512, 256, 1, 4), (1024, 512, 256, 8, 4), (1024, 512, 256, 9, 4), (4096, 256, 0, 16, 2),
-                                        (4096, 256, 0, 17, 2), (1024, 2048, 256, 1, 8), (1024, 2048, 256, 2, 8), (1024, 2048, 0, 2, 8),
+                                        (4096, 256, 0, 17, 2), (1024, 2048, 256, 1, 8), (1024, 2048, 256, 2, 8), (1024, 2048, 0, 2, 8), (8192, 256, 0, 20, 2),
                                         (1024, 4096, 0, 4, 1), (1024, 4096, 0, 5, 1)])
 def test_wide_little_work(H, I, Is, T, k):
     """Both sides of the work up to which FP4 slots stay with the column tiles (positions x
-    I of 16384, from H 4096 of 8192; two tokens with a shared expert)."""
+    I of 16384, from H 4096 of 8192; two tokens with a shared expert), and a hidden size
+    past the wide kernels'."""
     _experts("fp4", H, I, Is, T, 16, k, 540 + T, "little work")
 
 
