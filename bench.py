@@ -609,7 +609,7 @@ def main() -> int:
         mx = mx_decode(T, args.quant)
         if args.quant == "q3":
             up_k = "k_up_wide_q3" if T >= 24 else "k_up_grouped" if T >= 8 else "k_up_q3"
-            dn_k = ("k_down_wide_q3 + k_combine" if T >= 24 else
+            dn_k = ("k_down_wide_q3 + k_combine" if T >= 28 else
                     "k_down_grouped + k_combine" if T >= 3 else "k_down_q3")
         else:
             up_k = "k_up_wide" if T >= 4 else "k_up_mx" if mx else "k_up_stream"
