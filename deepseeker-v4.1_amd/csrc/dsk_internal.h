@@ -230,7 +230,8 @@ inline bool decode_pipeline(const dsk_moe_desc& d) {
 // down kernels run the routed products as scaled FP4 x FP8 MFMAs, with the
 // activations split into FP8 planes (two for x, three for h) on the B side.
 // The down kernel's waves take two K blocks each of the intermediate, so I is a
-// multiple of 256 up to kMxMaxWaves of them; kMxInter, the eight-wave form, has
+// multiple of 256 up to kMxMaxWaves waves of them (2304; nothing wider has been
+// measured, and takes the streaming kernels); kMxInter, the eight-wave form, has
 // kernels of its own.  (The shared expert runs in the decode pipeline's first
 // two kernels.)  At H 5120, I 2304, top-6 of 384 one
 // token took 99.5 us without these kernels, 67.7 with; two 164 and 107 of kernels.
